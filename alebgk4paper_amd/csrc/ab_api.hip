@@ -174,21 +174,23 @@ struct Timer
     void toc(int st) { prof_end(c, st); }
 };
 
-int fp64_transport(ab_ctx *c, double dt)
+// diag: the degeneracy and overshoot flags are wanted (ab_step with stats).
+int fp64_transport(ab_ctx *c, double dt, bool diag)
 {
     if (table2d(c)) return table2d_transport(c, dt);
     const double tol = c->cfg.mls_tol > 0 ? c->cfg.mls_tol : 1e-12;
     DevCloud v = c->view();
+    diag = diag || c->cfg.mls_clamp;
     launch_transport_fp64(v, c->g, c->gt, dt, c->cfg.radius, c->cfg.mls_order, tol,
                           c->cfg.mls_clamp, c->mlsflag, c->mlsovr, c->ilist, c->n_int, false,
-                          c->stream);
+                          diag, c->stream);
     launch_transport_fp64(v, c->g, c->gt, dt, c->cfg.radius, c->cfg.mls_order, tol,
                           c->cfg.mls_clamp, c->mlsflag, c->mlsovr, c->blist, c->n_bnd, true,
-                          c->stream);
+                          diag, c->stream);
     return hipGetLastError() == hipSuccess ? AB_OK : AB_ERR_HIP;
 }
 
-int fp64_step(ab_ctx *c, double dt)
+int fp64_step(ab_ctx *c, double dt, bool diag)
 {
     DevCloud v = c->view();
     hipStream_t s = c->stream;
@@ -200,7 +202,7 @@ int fp64_step(ab_ctx *c, double dt)
     if ((rc = zero_step_flags(c))) return rc;
     tm.toc(ST_REDUCE);
     tm.tic();
-    if ((rc = fp64_transport(c, dt))) return rc;
+    if ((rc = fp64_transport(c, dt, diag))) return rc;
     tm.toc(ST_TRANSPORT);
     const bool fused = table2d(c);
     if (fused)
@@ -249,7 +251,7 @@ int fp64_step(ab_ctx *c, double dt)
 // interior particle fails it, a second collision of every interior particle
 // and the moments again. No host synchronisation: the re-transport and the
 // second collision are launched always and act only where flagged.
-int fp64_step_mood(ab_ctx *c, double dt)
+int fp64_step_mood(ab_ctx *c, double dt, bool diag)
 {
     DevCloud v = c->view();
     hipStream_t s = c->stream;
@@ -261,13 +263,14 @@ int fp64_step_mood(ab_ctx *c, double dt)
     if ((rc = zero_step_flags(c))) return rc;
     tm.toc(ST_REDUCE);
     tm.tic();
-    if ((rc = fp64_transport(c, dt))) return rc;
+    if ((rc = fp64_transport(c, dt, diag))) return rc;
     tm.toc(ST_TRANSPORT);
     tm.tic();
     launch_mood_check(v, c->gt, c->rho, c->mood, c->limflag, s);
     const double tol = c->cfg.mls_tol > 0 ? c->cfg.mls_tol : 1e-12;
     launch_transport_fp64(v, c->g, c->gt, dt, c->cfg.radius, 1, tol, c->cfg.mls_clamp,
-                          c->mlsflag, c->mlsovr, c->ilist, c->n_int, false, s, c->mood);
+                          c->mlsflag, c->mlsovr, c->ilist, c->n_int, false,
+                          diag || c->cfg.mls_clamp, s, c->mood);
     launch_mood_commit(v, c->g, c->gt, c->mood, c->limflag, c->pmass, s);
     tm.toc(ST_LIMIT_COMMIT);
     tm.tic();
@@ -292,7 +295,7 @@ int fp64_step_mood(ab_ctx *c, double dt)
     return hipGetLastError() == hipSuccess ? AB_OK : AB_ERR_HIP;
 }
 
-int do_step(ab_ctx *c, double dt)
+int do_step(ab_ctx *c, double dt, bool diag = false)
 {
     if (!c->uploaded) { c->err = "ab_step before ab_upload"; return AB_ERR_STATE; }
     if (!(dt > 0.0) || !std::isfinite(dt)) { c->err = "dt must be positive and finite"; return AB_ERR_ARG; }
@@ -302,8 +305,8 @@ int do_step(ab_ctx *c, double dt)
         if (rc && c->err.empty()) c->err = "table step failed";
         return rc;
     }
-    if (c->cfg.limiter == AB_LIMITER_MOOD) return fp64_step_mood(c, dt);
-    return fp64_step(c, dt);
+    if (c->cfg.limiter == AB_LIMITER_MOOD) return fp64_step_mood(c, dt, diag);
+    return fp64_step(c, dt, diag);
 }
 
 }  // namespace
@@ -792,7 +795,7 @@ int ab_download_voxels(ab_ctx *c, int *voxel)
 int ab_step(ab_ctx *c, double dt, ab_step_stats *st)
 {
     if (!c) return AB_ERR_ARG;
-    int rc = do_step(c, dt);
+    int rc = do_step(c, dt, st != nullptr);
     if (rc || !st) return rc;
     double sc[S_COUNT];
     HIPCHK(c, hipMemcpyAsync(sc, c->scal, sizeof sc, hipMemcpyDeviceToHost, c->stream));
@@ -959,7 +962,7 @@ int ab_transport_only(ab_ctx *c, double dt)
     if (table_mode(c)) { c->err = "ab_transport_only runs the AB_PREC_FP64 formulation"; return AB_ERR_UNSUPPORTED; }
     int rc;
     if ((rc = zero_step_flags(c))) return rc;
-    if ((rc = fp64_transport(c, dt))) { c->err = "transport launch failed"; return rc; }
+    if ((rc = fp64_transport(c, dt, false))) { c->err = "transport launch failed"; return rc; }
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return AB_OK;
 }

@@ -242,11 +242,14 @@ void prof_begin(ab_ctx *c);
 void prof_end(ab_ctx *c, int stage);
 void prof_flush(ab_ctx *c);
 
-// ---- k_fp64.hip ------------------------------------------------------------
+// ---- k_mls.hip -------------------------------------------------------------
+// diag: the flags and overshoots of the step statistics (and the clamp).
 void launch_transport_fp64(const DevCloud &c, const double *g, double *gt, double dt,
                            double h, int order, double tol, int clamp, int *mlsflag,
-                           double *mlsovr, const int *list, int nlist, bool boundary,
+                           double *mlsovr, const int *list, int nlist, bool boundary, bool diag,
                            hipStream_t s, const int *only = nullptr);
+
+// ---- k_fp64.hip ------------------------------------------------------------
 // The reference's CPU-step limiter (MOOD): positivity to zero and the
 // transport check (flags), the commit after the flagged particles'
 // re-transport, and the post-collision admissibility check.

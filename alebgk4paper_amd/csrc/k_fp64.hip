@@ -1,11 +1,5 @@
-// k_fp64.hip -- the reference formulation of the ALE-BGK step in FP64 on gfx950.
-//
-// Transport: one thread per (particle, velocity node), coalesced over the
-// node index; a workgroup covers 256 nodes of one particle and stages that
-// particle's neighbour positions in LDS (every lane reads the same entry: an
-// LDS broadcast). Interior and boundary particles are launched from compact
-// lists, each with its compile-time basis size, instead of sweeping the whole
-// grid twice with early exits as the reference does (CudaBackend.cu:1667-1677).
+// k_fp64.hip -- the reference formulation of the ALE-BGK step in FP64 on gfx950
+// after its transport (k_mls.hip).
 //
 // Per-particle stages: one 256-thread workgroup per particle, coalesced over
 // the node index, with fixed-order workgroup reductions. They fuse reference
@@ -21,312 +15,6 @@
 namespace ab {
 
 namespace {
-
-__device__ __forceinline__ void node_velocity(const DevCloud &c, int lin, double &vx,
-                                              double &vy, double &vz)
-{
-    int Nv = c.Nv;
-    int iv = lin % Nv, jv = (lin / Nv) % Nv, kv = lin / (Nv * Nv);
-    vx = vnode(c.vlo, c.dv, iv);
-    vy = vnode(c.vlo, c.dv, jv);
-    vz = (c.dim == 3) ? vnode(c.vlo, c.dv, kv) : 0.0;
-}
-
-// kCopyGt + kTransportNode3DT<P, BND> (Solver/CudaBackend.cu:191-197, 699-869).
-template <int P, bool BND>
-__global__ __launch_bounds__(kBlock) void k_transport3d(DevCloud c, const double *__restrict__ g,
-                                                        double *__restrict__ gt, double dt,
-                                                        double h, double tol, int clamp,
-                                                        int *mlsflag, double *mlsovr,
-                                                        const int *__restrict__ list,
-                                                        int nchunk, const int *__restrict__ only)
-{
-    __shared__ double sx[AB_MAX_NEIGH], sy[AB_MAX_NEIGH], sz[AB_MAX_NEIGH];
-    __shared__ int sj[AB_MAX_NEIGH];
-    __shared__ double sred[2 * (kBlock / kWave)];
-    const int b = xcd_remap(blockIdx.x, gridDim.x);
-    const int i = list[b / nchunk];
-    if (only && !only[i]) return;            // whole block: one particle
-    const int lin = (b % nchunk) * kBlock + threadIdx.x;
-    const int nn = c.nneigh[i];
-    for (int t = threadIdx.x; t < nn; t += kBlock)
-    {
-        int j = c.neigh[(size_t)i * AB_MAX_NEIGH + t];
-        sj[t] = j; sx[t] = c.x[j]; sy[t] = c.y[j]; sz[t] = c.z[j];
-    }
-    __syncthreads();
-
-    const size_t gs = (size_t)c.gstride;
-    double excess = 0.0;
-    int flag = 0;
-    if (lin < c.nodes)
-    {
-        double vx, vy, vz;
-        node_velocity(c, lin, vx, vy, vz);
-        const double g_self = g[(size_t)i * gs + lin];
-        double out = g_self;
-        bool gated = false;
-        if (BND)
-        {
-            double cn = wall_cn3(vx, vy, vz, c.wux[i], c.wuy[i], c.wuz[i], c.wnx[i], c.wny[i],
-                                 c.wnz[i]);
-            gated = (cn >= 0.0);
-        }
-        if (!gated)
-        {
-            const double xf = c.x[i] - (vx - c.mvx[i]) * dt;
-            const double yf = c.y[i] - (vy - c.mvy[i]) * dt;
-            const double zf = c.z[i] - (vz - c.mvz[i]) * dt;
-            const double hh = h * h;
-            double A[P * P], b1[P];
-#pragma unroll
-            for (int q = 0; q < P * P; ++q) A[q] = 0.0;
-#pragma unroll
-            for (int q = 0; q < P; ++q) b1[q] = 0.0;
-            bool has = false;
-            double sumW = 0.0, sumWG = 0.0, gmin = 1e300, gmax = -1e300;
-            for (int m = 0; m < nn; ++m)
-            {
-                const double dxn = sx[m] - xf, dyn = sy[m] - yf, dzn = sz[m] - zf;
-                const double r2 = dxn * dxn + dyn * dyn + dzn * dzn;
-                const double q2 = r2 / hh;                  // mlsWeightSq
-                double w = 0.0;
-                if (q2 < 1.0) { double t1 = 1.0 - q2; w = t1 * t1; }
-                if (w < 1e-30) continue;
-                double basis[P];
-                const double ssx = dxn / h, ssy = dyn / h, ssz = dzn / h;
-                basis[0] = 1.0; basis[1] = ssx; basis[2] = ssy; basis[3] = ssz;
-                if constexpr (P >= 10)
-                {
-                    basis[4] = ssx * ssx; basis[5] = ssy * ssy; basis[6] = ssz * ssz;
-                    basis[7] = ssx * ssy; basis[8] = ssx * ssz; basis[9] = ssy * ssz;
-                }
-                const double gj = g[(size_t)sj[m] * gs + lin];
-#pragma unroll
-                for (int p1 = 0; p1 < P; ++p1)
-                {
-                    const double wb = w * basis[p1];
-#pragma unroll
-                    for (int p2 = p1; p2 < P; ++p2) A[p1 * P + p2] += wb * basis[p2];
-                    b1[p1] += wb * gj;
-                }
-                sumW += w;
-                sumWG += w * gj;
-                gmin = fmin(gmin, gj);
-                gmax = fmax(gmax, gj);
-                has = true;
-            }
-            if (has)
-            {
-                double dmax = 0.0;
-#pragma unroll
-                for (int k = 0; k < P; ++k) dmax = fmax(dmax, A[k * P + k]);
-                bool degenerate = (dmax <= 0.0);
-#pragma unroll
-                for (int k = 0; k < P; ++k)
-                {
-                    double d = A[k * P + k];
-#pragma unroll
-                    for (int j = 0; j < k; ++j) { double l = A[j * P + k]; d -= l * l; }
-                    if (!(d > tol * dmax)) degenerate = true;
-                    d = degenerate ? 1.0 : sqrt(d);
-                    A[k * P + k] = d;
-#pragma unroll
-                    for (int m2 = k + 1; m2 < P; ++m2)
-                    {
-                        double v = A[k * P + m2];
-#pragma unroll
-                        for (int j = 0; j < k; ++j) v -= A[j * P + k] * A[j * P + m2];
-                        A[k * P + m2] = v / d;
-                    }
-                }
-#pragma unroll
-                for (int k = 0; k < P; ++k)
-                {
-                    double v = b1[k];
-#pragma unroll
-                    for (int j = 0; j < k; ++j) v -= A[j * P + k] * b1[j];
-                    b1[k] = v / A[k * P + k];
-                }
-#pragma unroll
-                for (int k = P - 1; k >= 0; --k)
-                {
-                    double v = b1[k];
-#pragma unroll
-                    for (int j = k + 1; j < P; ++j) v -= A[k * P + j] * b1[j];
-                    b1[k] = v / A[k * P + k];
-                }
-                out = b1[0];
-                if (degenerate || !isfinite(out)) out = (sumW > 0.0) ? (sumWG / sumW) : g_self;
-                if (degenerate || !isfinite(b1[0])) flag |= 1;
-                excess = fmax(fmax(out - gmax, gmin - out), 0.0);
-                bool overshoot = (out < gmin) || (out > gmax);
-                if (overshoot) flag |= 2;
-                if (overshoot && clamp) out = fmin(fmax(out, gmin), gmax);
-            }
-        }
-        gt[(size_t)i * gs + lin] = out;
-    }
-    // One flag word and one overshoot sum per workgroup.
-    double red[1] = {excess};
-    block_sum<1>(red, sred);
-    int f = flag;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) f |= __shfl_xor(f, o, kWave);
-    __shared__ int sflag[kBlock / kWave];
-    if ((threadIdx.x & (kWave - 1)) == 0) sflag[threadIdx.x / kWave] = f;
-    __syncthreads();
-    if (threadIdx.x == 0)
-    {
-        int fa = 0;
-        for (int q = 0; q < kBlock / kWave; ++q) fa |= sflag[q];
-        if (fa && mlsflag) atomicOr(&mlsflag[i], fa);
-        if (red[0] > 0.0 && mlsovr)
-        {
-            double dv3 = c.dv * c.dv * c.dv;
-            atomicAdd(&mlsovr[i], red[0] * dv3);
-        }
-    }
-}
-
-// kCopyGt + kTransportNode, 2-D Chu layers (Solver/CudaBackend.cu:199-300):
-// weight through sqrt + mlsWeight, Gauss with partial pivoting on both layers.
-// Row swaps compare unrolled row indices against the pivot so A stays in
-// registers. A is summed in its upper triangle and mirrored: the reference
-// sums every entry, so the lower triangle differs from its by the rounding
-// of w phi_a phi_b against w phi_b phi_a.
-template <int P, bool BND>
-__global__ __launch_bounds__(kBlock) void k_transport2d(DevCloud c, const double *__restrict__ g,
-                                                        double *__restrict__ gt, double dt,
-                                                        double h, const int *__restrict__ list,
-                                                        int nchunk, const int *__restrict__ only)
-{
-    __shared__ double sx[AB_MAX_NEIGH], sy[AB_MAX_NEIGH];
-    __shared__ int sj[AB_MAX_NEIGH];
-    const int b = xcd_remap(blockIdx.x, gridDim.x);
-    const int i = list[b / nchunk];
-    if (only && !only[i]) return;            // whole block: one particle
-    const int lin = (b % nchunk) * kBlock + threadIdx.x;
-    const int nn = c.nneigh[i];
-    if (c.inst) h = c.ih[c.inst[i]];
-    for (int t = threadIdx.x; t < nn; t += kBlock)
-    {
-        int j = c.neigh[(size_t)i * AB_MAX_NEIGH + t];
-        sj[t] = j; sx[t] = c.x[j]; sy[t] = c.y[j];
-    }
-    __syncthreads();
-    if (lin >= c.nodes) return;
-    const size_t gs = (size_t)c.gstride;
-    const int Nv2 = c.nodes;
-    const double vx = vnode(c.vlo, c.dv, lin % c.Nv);
-    const double vy = vnode(c.vlo, c.dv, lin / c.Nv);
-    double o1 = g[(size_t)i * gs + lin], o2 = g[(size_t)i * gs + lin + Nv2];
-    bool gated = false;
-    if (BND)
-    {
-        double cn = wall_cn2(vx, vy, c.wux[i], c.wuy[i], c.wnx[i], c.wny[i]);
-        gated = (cn >= 0.0);
-    }
-    if (!gated)
-    {
-        const double xf = c.x[i] - (vx - c.mvx[i]) * dt;
-        const double yf = c.y[i] - (vy - c.mvy[i]) * dt;
-        double A[P * P], bb1[P], bb2[P];
-#pragma unroll
-        for (int q = 0; q < P * P; ++q) A[q] = 0.0;
-#pragma unroll
-        for (int q = 0; q < P; ++q) { bb1[q] = 0.0; bb2[q] = 0.0; }
-        bool has = false;
-        for (int m = 0; m < nn; ++m)
-        {
-            const double dxn = sx[m] - xf, dyn = sy[m] - yf;
-            const double r = sqrt(dxn * dxn + dyn * dyn);
-            double w = 0.0;                                   // mlsWeight
-            if (r < h) { double qq = r / h; double t1 = 1.0 - qq * qq; w = t1 * t1; }
-            if (w < 1e-30) continue;
-            double basis[P];
-            const double ssx = dxn / h, ssy = dyn / h;
-            basis[0] = 1.0; basis[1] = ssx; basis[2] = ssy;
-            if constexpr (P >= 6) { basis[3] = ssx * ssx; basis[4] = ssx * ssy; basis[5] = ssy * ssy; }
-            // A is symmetric: the upper triangle here, mirrored after the sum
-#pragma unroll
-            for (int p1 = 0; p1 < P; ++p1)
-#pragma unroll
-                for (int p2 = p1; p2 < P; ++p2) A[p1 * P + p2] += w * basis[p1] * basis[p2];
-            const double *gj = g + (size_t)sj[m] * gs;
-            const double gn1 = gj[lin], gn2 = gj[lin + Nv2];
-#pragma unroll
-            for (int q = 0; q < P; ++q)
-            {
-                bb1[q] += w * basis[q] * gn1;
-                bb2[q] += w * basis[q] * gn2;
-            }
-            has = true;
-        }
-        if (has)
-        {
-#pragma unroll
-            for (int p1 = 1; p1 < P; ++p1)
-#pragma unroll
-                for (int p2 = 0; p2 < p1; ++p2) A[p1 * P + p2] = A[p2 * P + p1];
-#pragma unroll
-            for (int col = 0; col < P; ++col)
-            {
-                int piv = col;
-                double mx = fabs(A[col * P + col]);
-#pragma unroll
-                for (int row = col + 1; row < P; ++row)
-                    if (fabs(A[row * P + col]) > mx) { mx = fabs(A[row * P + col]); piv = row; }
-#pragma unroll
-                for (int row = col + 1; row < P; ++row)
-                {
-                    if (row == piv)
-                    {
-#pragma unroll
-                        for (int q = 0; q < P; ++q)
-                        {
-                            double t1 = A[col * P + q];
-                            A[col * P + q] = A[row * P + q];
-                            A[row * P + q] = t1;
-                        }
-                        double tb = bb1[col]; bb1[col] = bb1[row]; bb1[row] = tb;
-                        tb = bb2[col]; bb2[col] = bb2[row]; bb2[row] = tb;
-                    }
-                }
-                const double d = A[col * P + col];
-                if (fabs(d) < 1e-30) continue;
-#pragma unroll
-                for (int row = col + 1; row < P; ++row)
-                {
-                    const double f = A[row * P + col] / d;
-#pragma unroll
-                    for (int q = col; q < P; ++q) A[row * P + q] -= f * A[col * P + q];
-                    bb1[row] -= f * bb1[col];
-                    bb2[row] -= f * bb2[col];
-                }
-            }
-            double s1[P], s2[P];
-#pragma unroll
-            for (int row = P - 1; row >= 0; --row)
-            {
-                double v1 = bb1[row], v2 = bb2[row];
-#pragma unroll
-                for (int q = row + 1; q < P; ++q)
-                {
-                    v1 -= A[row * P + q] * s1[q];
-                    v2 -= A[row * P + q] * s2[q];
-                }
-                const double d = A[row * P + row];
-                s1[row] = fabs(d) > 1e-30 ? v1 / d : 0.0;
-                s2[row] = fabs(d) > 1e-30 ? v2 / d : 0.0;
-            }
-            o1 = s1[0];
-            o2 = s2[0];
-        }
-    }
-    gt[(size_t)i * gs + lin] = o1;
-    gt[(size_t)i * gs + lin + Nv2] = o2;
-}
 
 // Per-particle mass partial: sum of g*dv^d over the mass-carrying layer
 // (kSumMass3D / kSumMass per-thread part, CudaBackend.cu:391-436).
@@ -1151,37 +839,6 @@ __global__ __launch_bounds__(kBlock) void k_pad_check(DevCloud c, const double *
 }
 
 }  // namespace
-
-void launch_transport_fp64(const DevCloud &c, const double *g, double *gt, double dt, double h,
-                           int order, double tol, int clamp, int *mlsflag, double *mlsovr,
-                           const int *list, int nlist, bool boundary, hipStream_t s,
-                           const int *only)
-{
-    if (nlist <= 0) return;
-    const int nchunk = (c.nodes + kBlock - 1) / kBlock;
-    const int nb = nlist * nchunk;
-    if (c.dim == 3)
-    {
-        if (boundary)
-            k_transport3d<4, true><<<nb, kBlock, 0, s>>>(c, g, gt, dt, h, tol, clamp, mlsflag,
-                                                         mlsovr, list, nchunk, only);
-        else if (order >= 2)
-            k_transport3d<10, false><<<nb, kBlock, 0, s>>>(c, g, gt, dt, h, tol, clamp, mlsflag,
-                                                           mlsovr, list, nchunk, only);
-        else
-            k_transport3d<4, false><<<nb, kBlock, 0, s>>>(c, g, gt, dt, h, tol, clamp, mlsflag,
-                                                          mlsovr, list, nchunk, only);
-    }
-    else
-    {
-        if (boundary)
-            k_transport2d<3, true><<<nb, kBlock, 0, s>>>(c, g, gt, dt, h, list, nchunk, only);
-        else if (order >= 2)
-            k_transport2d<6, false><<<nb, kBlock, 0, s>>>(c, g, gt, dt, h, list, nchunk, only);
-        else
-            k_transport2d<3, false><<<nb, kBlock, 0, s>>>(c, g, gt, dt, h, list, nchunk, only);
-    }
-}
 
 void launch_mass_partials(const DevCloud &c, const double *g, double *pmass, hipStream_t s)
 {

@@ -1,0 +1,118 @@
+"""The FP64 formulation's MLS transport where its stencils are not the
+lattice's (jittered, degenerate, values that are not finite) and with and
+without the step statistics.
+
+Tolerances: transport 1e-12 of each particle's largest |g| (a 10 x 10 solve in
+FP64 in another order of sums, on stencils as well conditioned as a lattice's);
+everything else exact or stated at the assertion.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import alebgk4paper_amd as A
+import oracle_ctypes as O
+from helpers import geom_of, setup
+
+pytestmark = pytest.mark.gpu
+
+
+def _oracle_cloud(cl, neigh, nn):
+    return O.Cloud(cl.cfg.dim, cl.cfg.nv, cl.cfg.vmin,
+                   (cl.cfg.vmax - cl.cfg.vmin) / (cl.cfg.nv - 1), cl.x, cl.y, cl.z, cl.boundary,
+                   cl.wall, neigh, nn)
+
+
+def _jittered(name, nx, nv, order, amp=0.15):
+    case, cl, *_ = setup(name, nx, nv, order=order)
+    rng = np.random.default_rng(5)
+    dx = 1e-6 / (nx - 1)
+    inner = cl.boundary == 0
+    for k in ("x", "y", "z")[:cl.cfg.dim]:
+        getattr(cl, k)[inner] += amp * dx * rng.uniform(-1, 1, int(inner.sum()))
+    neigh, nn, _ = O.neighbours(geom_of(cl.cfg, case), cl.x, cl.y, cl.z)
+    return case, cl, _oracle_cloud(cl, neigh, nn), 0.5 * dx / 1303.0
+
+
+@pytest.mark.parametrize("name,nx,nv,order", [("cavity3d", 9, 4, 2), ("cavity3d", 8, 7, 1),
+                                              ("cavity2d", 12, 7, 2), ("cavity2d", 12, 17, 1)])
+def test_transport_on_a_jittered_cloud(name, nx, nv, order):
+    print(f"[mls] jittered {name} {nx} Nv {nv} order {order}", flush=True)
+    case, cl, ocl, dt = _jittered(name, nx, nv, order)
+    sol = A.Solver(cl, precision=A.PREC_FP64)
+    sol.transport_only(dt)
+    want = O.transport(ocl, cl.g, dt, cl.cfg.radius, order)
+    scale = np.abs(cl.g).max(axis=1, keepdims=True)
+    assert (np.abs(sol.gt() - want) / scale).max() < 1e-12
+
+
+@pytest.mark.parametrize("amp", [0.0, 0.15])
+def test_step_statistics_match_oracle_and_change_nothing(amp):
+    """Flags and overshoots of the transport with stats; the same state, bit
+    for bit, without them."""
+    case, cl, ocl, dt = _jittered("cavity3d", 9, 5, 2, amp)
+    _, fl, ov = O.transport(ocl, cl.g, dt, cl.cfg.radius, 2, flags=True)
+    a, b = A.Solver(cl, precision=A.PREC_FP64), A.Solver(cl, precision=A.PREC_FP64)
+    st = a.step(dt, stats=True)
+    b.step(dt)
+    assert np.array_equal(a.g(), b.g())
+    assert st["n_mls_degenerate"] == int((fl & 1).astype(bool).sum())
+    assert st["n_mls_extrapolate"] == int((fl & 2).astype(bool).sum())
+    # an excess is a difference of values: rounding of the larger one, 1e-12 of it
+    assert abs(st["mls_ovr_sum"] - ov.sum()) <= 1e-12 * np.abs(cl.g).sum() + 1e-9 * ov.sum()
+
+
+@pytest.mark.parametrize("name", ["cavity3d", "cavity2d"])
+def test_values_outside_the_support_do_not_enter(name):
+    """A neighbour that is not finite reaches exactly the nodes whose foot
+    point has it in its support, as in the oracle."""
+    case, cl, ocl, dt = _jittered(name, 9, 5, 2, 0.0)
+    p = cl.N // 2
+    cl.g[p] = np.nan
+    cl.g[p + 1] = np.inf
+    want = O.transport(ocl, cl.g, dt, cl.cfg.radius, 2)
+    sol = A.Solver(cl, precision=A.PREC_FP64)
+    sol.transport_only(dt)
+    got = sol.gt()
+    assert np.array_equal(np.isfinite(got), np.isfinite(want))
+    ok = np.isfinite(want)
+    assert np.abs(got[ok] - want[ok]).max() < 1e-12 * np.abs(cl.g[np.isfinite(cl.g)]).max()
+
+
+@pytest.mark.parametrize("order", [1, 2])
+def test_collinear_stencils_2d(order):
+    """Rows of particles out of each other's reach: every stencil is a line
+    and A is singular. The nodes that do not leave the line (v_y = 0) have exact
+    zeros in A, which the pivoted elimination skips; there the result is the
+    oracle's where the line determines its own terms. The others divide rounding by rounding in the reference too."""
+    case, cl, *_ = setup("cavity2d", 9, 5, order=order)
+    cl.y = np.ascontiguousarray(cl.y * 4.0)
+    neigh, nn, _ = O.neighbours(geom_of(cl.cfg, case), cl.x, cl.y, cl.z)
+    # neighbours of the same row only, whatever the voxels did with the rows
+    N = cl.N
+    neigh = np.full((N, A.MAX_NEIGH), 0, np.int32)
+    nn = np.zeros(N, np.int32)
+    for i in range(N):
+        j = [q for q in range(i - i % 9, i - i % 9 + 9)
+             if q != i and abs(cl.x[q] - cl.x[i]) < cl.cfg.radius]
+        neigh[i, :len(j)], nn[i] = j, len(j)
+    cl.neigh, cl.nneigh = neigh, nn
+    dt = 0.5 * (1e-6 / 8) / 1303.0
+    want = O.transport(_oracle_cloud(cl, neigh, nn), cl.g, dt, cl.cfg.radius, order)
+    sol = A.Solver(cl, precision=A.PREC_FP64)
+    sol.transport_only(dt)
+    got = sol.gt()
+    v = A.velocities(cl.cfg)
+    # ... and the line itself must determine 1, x, x^2: three neighbours in the
+    # support, with room to its edge
+    on = np.zeros((N, 25), bool)
+    for i in range(N):
+        for k in np.nonzero(v[:, 1] == 0.0)[0]:
+            d = np.abs(cl.x[neigh[i, :nn[i]]] - (cl.x[i] - v[k, 0] * dt))
+            on[i, k] = (d < 0.9 * cl.cfg.radius).sum() >= 3
+    on = np.tile(on, 2)
+    assert on.sum() > 100
+    # elimination of a matrix whose other rows are zero: 1e-11 of the largest value
+    scale = np.abs(cl.g).max(axis=1, keepdims=True)
+    assert (np.abs(got - want) / scale)[on].max() < 1e-11
