@@ -76,6 +76,7 @@ void free_cloud(ab_ctx *c)
     c->bid = nullptr;
     table_free(c);
     table2d_free(c);
+    stencil_free(c);
     c->coef_dt = -1.0;
 }
 
@@ -181,6 +182,7 @@ int fp64_transport(ab_ctx *c, double dt, bool diag)
     const double tol = c->cfg.mls_tol > 0 ? c->cfg.mls_tol : 1e-12;
     DevCloud v = c->view();
     diag = diag || c->cfg.mls_clamp;
+    if (c->dim == 3) return stencil_transport(c, dt, tol, diag);
     launch_transport_fp64(v, c->g, c->gt, dt, c->cfg.radius, c->cfg.mls_order, tol,
                           c->cfg.mls_clamp, c->mlsflag, c->mlsovr, c->ilist, c->n_int, false,
                           diag, c->stream);
@@ -353,6 +355,12 @@ int graph_coefficients(ab_ctx *c, double dt)
         int rc = table2d_prepare(c, dt);
         if (rc) return rc;
     }
+    // likewise the stencil classes, which a captured step does not look for
+    if (c->dim == 3 && !table_mode(c) && !c->st_valid)
+    {
+        int rc = stencil_prepare(c);
+        if (rc) return rc;
+    }
     return AB_OK;
 }
 
@@ -403,6 +411,7 @@ int relayout_cloud(ab_ctx *c, const int *src, int n)
     const int oldN = c->N;
     c->N = n;
     c->cfg.n_particles = n;
+    stencil_free(c);               // sized by N
     int rc = alloc_cloud(c);
     auto gather = [&](auto *from, auto *to, int stride) {
         const size_t tot = (size_t)n * stride;
@@ -702,6 +711,7 @@ int ab_upload(ab_ctx *c, const ab_cloud_view *v)
     }
     c->uploaded = true;
     c->mass_valid = false;
+    c->st_valid = false;
     c->gen++;
     if (table_mode(c))
     {
@@ -741,6 +751,7 @@ int ab_rebuild_neighbours(ab_ctx *c)
         if ((rc = dalloc(c, &c->vox, (size_t)c->N)) || (rc = dalloc(c, &c->vlist, 2 * (size_t)c->N)))
             return rc;
     }
+    c->st_valid = false;
     Timer tm(c);
     tm.tic();
     if (int e = launch_neighbours(c->view(), f, c->vox, c->vcount, c->vstart, c->vlist, nvox,
@@ -1074,6 +1085,7 @@ int ab_set_wall_state(ab_ctx *c, int n, const int *idx, const double *x, const d
             if (mv) s[9 + a] = mv[3 * k + a];
         }
     }
+    c->st_valid = false;
     int *di = nullptr;
     double *ds = nullptr;
     int rc;

@@ -127,6 +127,18 @@ struct ab_ctx
     int *vox = nullptr, *vcount = nullptr, *vstart = nullptr, *vlist = nullptr;
     int nvox = 0;
 
+    // classes of congruent stencils (3-D FP64 transport, k_stencil.hip): the
+    // class key and the row ids of each particle, the first particle, member
+    // count and coefficient slot of each key, the key of each slot; counters;
+    // the runs (sorted by bin) and the particles of no class; coefficients of every slot
+    int *st_key = nullptr, *st_rb = nullptr, *st_rep = nullptr, *st_cnt = nullptr;
+    int *st_slot = nullptr, *st_skey = nullptr, *st_n = nullptr;
+    int *st_run = nullptr, *st_int = nullptr, *st_bnd = nullptr, *st_bin = nullptr;
+    unsigned char *st_follow = nullptr;
+    double *st_coef = nullptr;
+    int st_maxslot = 0;
+    bool st_valid = false;         // false once positions, lists or wall state change
+
     // table pipelines (AB_PREC_MIXED / AB_PREC_FP64_TABLE)
     int S = 0;                     // padded per-particle stride of the tables
     void *gs = nullptr;            // stored g, [N][S], FP32 or FP64
@@ -247,7 +259,16 @@ void prof_flush(ab_ctx *c);
 void launch_transport_fp64(const DevCloud &c, const double *g, double *gt, double dt,
                            double h, int order, double tol, int clamp, int *mlsflag,
                            double *mlsovr, const int *list, int nlist, bool boundary, bool diag,
-                           hipStream_t s, const int *only = nullptr);
+                           hipStream_t s, const int *only = nullptr,
+                           const int *nlist_dev = nullptr);
+
+// ---- k_stencil.hip ---------------------------------------------------------
+// The 3-D transport with the normal equations shared by congruent stencils.
+// stencil_prepare: the classes of the current cloud (after every change of
+// positions, lists, flags, wall or mesh velocities: st_valid).
+int stencil_transport(ab_ctx *ctx, double dt, double tol, bool diag);
+int stencil_prepare(ab_ctx *ctx);
+void stencil_free(ab_ctx *ctx);
 
 // ---- k_fp64.hip ------------------------------------------------------------
 // The reference's CPU-step limiter (MOOD): positivity to zero and the

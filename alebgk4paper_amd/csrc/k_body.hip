@@ -701,6 +701,7 @@ extern "C" int ab_body_step(ab_ctx *c, double dt, int nb, ab_rigid_body *bodies,
         if (bodies[b].shape < AB_BODY_SQUARE || bodies[b].shape > AB_BODY_CUBE ||
             bodies[b].npts <= 0 || !(bodies[b].mass > 0.0) || !(bodies[b].size > 0.0))
         { c->err = "ab_body_step: invalid body"; return AB_ERR_ARG; }
+    c->st_valid = false;           // the surface moves
     hipStream_t s = c->stream;
     const bool d3 = c->dim == 3;
     int rc;

@@ -564,6 +564,7 @@ extern "C" int ab_cloud_manage(ab_ctx *c, int nbodies, const ab_body *bodies, co
         d.ox = b.o[0]; d.oy = b.o[1];
         for (int m = 0; m < 9; ++m) d.rm[m] = b.rm[m];
     }
+    c->st_valid = false;
     const int N0 = c->N;
     c->cm_src.resize(N0);
     for (int i = 0; i < N0; ++i) c->cm_src[i] = i;

@@ -36,9 +36,11 @@ extern "C" {
 #define AB_ERR_NOMEM 5            /* device allocation failed */
 
 /* Arithmetic of the step. */
-#define AB_PREC_FP64 0        /* the reference formulation in FP64: per
-                                 (particle, node) normal equations and
-                                 Cholesky every step (kTransportNode3DT) */
+#define AB_PREC_FP64 0        /* the reference formulation in FP64: normal
+                                 equations assembled and solved every step
+                                 (kTransportNode3DT), per (particle, node);
+                                 in 3-D once per node for particles with
+                                 congruent stencils. Any cloud */
 #define AB_PREC_MIXED 1       /* MLS coefficients factorised once in FP64,
                                  transport contraction, collision and storage
                                  in FP32; conservation sums, wall scaling and

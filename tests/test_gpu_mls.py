@@ -116,3 +116,92 @@ def test_collinear_stencils_2d(order):
     # elimination of a matrix whose other rows are zero: 1e-11 of the largest value
     scale = np.abs(cl.g).max(axis=1, keepdims=True)
     assert (np.abs(got - want) / scale)[on].max() < 1e-11
+
+
+# ---- stencils shared by congruent particles --------------------------------------
+
+def _variant(kind, nx, nv, order):
+    """A lattice cloud altered so that some, all or no particles share stencils."""
+    case, cl, *_ = setup("cavity3d", nx, nv, order=order)
+    rng = np.random.default_rng(11)
+    dx = 1e-6 / (nx - 1)
+    inner = np.nonzero(cl.boundary == 0)[0]
+    if kind == "few":                       # a few particles off the lattice
+        for p in rng.choice(inner, 5, replace=False):
+            cl.x[p] += 0.2 * dx * rng.uniform(-1, 1)
+            cl.z[p] += 0.2 * dx * rng.uniform(-1, 1)
+    elif kind == "tiny":                    # displaced by less than a lattice check would see
+        cl.y[inner[::3]] += 1e-9 * dx
+    elif kind == "permuted":                # no two neighbours in row order
+        q = rng.permutation(cl.N)
+        for k in ("x", "y", "z", "boundary", "wall", "mom", "g"):
+            setattr(cl, k, np.ascontiguousarray(getattr(cl, k)[q]))
+    elif kind == "holes":                   # particles missing, as inside a body
+        keep = np.ones(cl.N, bool)
+        keep[rng.choice(inner, 12, replace=False)] = False
+        for k in ("x", "y", "z", "boundary", "wall", "mom", "g"):
+            setattr(cl, k, np.ascontiguousarray(getattr(cl, k)[keep]))
+    elif kind == "twice":                   # two particles at one site
+        q = np.concatenate([np.arange(cl.N), inner[40:42]])
+        for k in ("x", "y", "z", "boundary", "wall", "mom", "g"):
+            setattr(cl, k, np.ascontiguousarray(getattr(cl, k)[q]))
+    elif kind == "mesh":                    # particles with a mesh velocity, zero mostly
+        cl.mesh = np.zeros((cl.N, 3))
+        cl.mesh[inner[10:30]] = (30.0, -20.0, 10.0)
+    elif kind == "lid":                     # a wall velocity that varies along the lid
+        lid = np.nonzero(np.abs(cl.z - case.dom[4]) < 1e-13)[0]
+        cl.wall[lid, 3] = 1e6 * cl.x[lid]
+    neigh, nn, _ = O.neighbours(geom_of(cl.cfg, case), cl.x, cl.y, cl.z)
+    ocl = _oracle_cloud(cl, neigh, nn) if cl.mesh is None else \
+        O.Cloud(3, nv, cl.cfg.vmin, (cl.cfg.vmax - cl.cfg.vmin) / (nv - 1), cl.x, cl.y, cl.z,
+                cl.boundary, cl.wall, neigh, nn, cl.mesh)
+    return case, cl, ocl, 0.5 * dx / 1303.0
+
+
+@pytest.mark.parametrize("kind,nx,nv,order", [
+    ("lattice", 13, 5, 2), ("lattice", 18, 4, 1), ("lattice", 5, 5, 2), ("lattice", 7, 9, 2),
+    ("few", 13, 5, 2), ("tiny", 12, 5, 2), ("permuted", 11, 5, 2), ("holes", 14, 4, 2),
+    ("twice", 11, 4, 2), ("mesh", 12, 5, 2), ("lid", 12, 5, 2)])
+def test_shared_stencils_match_oracle(kind, nx, nv, order):
+    print(f"[mls] shared stencils {kind} {nx} Nv {nv} order {order}", flush=True)
+    case, cl, ocl, dt = _variant(kind, nx, nv, order)
+    sol = A.Solver(cl, precision=A.PREC_FP64)
+    sol.transport_only(dt)
+    want = O.transport(ocl, cl.g, dt, cl.cfg.radius, order)
+    scale = np.abs(cl.g).max(axis=1, keepdims=True)
+    assert (np.abs(sol.gt() - want) / scale).max() < 1e-12
+
+
+def test_stencils_follow_the_cloud():
+    """After a transport, particles move and gain a mesh velocity
+    (ab_set_wall_state); the next transport, eager and as a replay of a graph
+    captured before, sees them."""
+    case, cl, ocl, dt = _variant("lattice", 11, 4, 2)
+    sols = [A.Solver(cl, precision=A.PREC_FP64) for _ in range(3)]
+    graph = A.Graph([sols[1]], dt, 1)
+    for s in sols[:2]:
+        s.transport_only(dt)
+    inner = np.nonzero(cl.boundary == 0)[0]
+    p = inner[100:110]
+    rng = np.random.default_rng(2)
+    xyz = np.stack([cl.x, cl.y, cl.z], 1)[p] + 0.1 * 1e-7 * rng.uniform(-1, 1, (len(p), 3))
+    mv = np.tile([5.0, -7.0, 3.0], (len(p), 1))
+    for s in sols:
+        s.set_wall_state(p, xyz=xyz, mv=mv)
+    sols[0].step(dt)
+    graph.launch()
+    graph.synchronize()
+    sols[2].step(dt)
+    assert np.array_equal(sols[0].g(), sols[2].g())
+    assert np.array_equal(sols[1].g(), sols[2].g())
+    graph.close()
+    for k, a in enumerate((cl.x, cl.y, cl.z)):
+        a[p] = xyz[:, k]
+    cl.mesh = np.zeros((cl.N, 3))
+    cl.mesh[p] = mv
+    nb, nn = sols[0].neighbours()
+    ocl = O.Cloud(3, 4, cl.cfg.vmin, (cl.cfg.vmax - cl.cfg.vmin) / 3, cl.x, cl.y, cl.z, cl.boundary,
+                  cl.wall, nb, nn, cl.mesh)
+    st = O.State(ocl, cl.g, cl.mom)
+    O.step(ocl, st, dt, case.tau, case.R, cl.cfg.radius, 2)
+    assert np.abs(sols[0].g() - st.g).max() < 1e-10 * np.abs(st.g).max()
