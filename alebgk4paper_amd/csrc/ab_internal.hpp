@@ -111,6 +111,8 @@ struct ab_ctx
     int *moodfail = nullptr;       // 1: some particle failed the post-collision check
     double *mlsovr = nullptr;
     double *pmass = nullptr;       // per-particle partial sums
+    double *pnew = nullptr;        // committed mass per particle of the fused commit and collision
+    double *prho = nullptr;        // its wall densities (3-D)
     double *scal = nullptr;        // ab::ScalarSlot
     bool mass_valid = false;       // pmass holds the current g's masses
     // Bumped whenever the device arrays are freed, re-allocated or refilled
@@ -171,7 +173,6 @@ struct ab_ctx
     int t2_nv = 0, t2_nh = 0, t2_nit = 0;   // column runs, row runs, all items
     int t2_run = -1;               // run length index of the apply (-1: the default, 8 outputs)
     double t2_dt = -1.0;           // dt the coefficients were built for
-    double *t2_pnew = nullptr;     // committed mass per particle of the fused commit and collision
 
     // discrete-Maxwellian collision (cfg.collision) and its MLP warm start
     double *dm_alpha = nullptr;    // N x 5 solution of the last step
@@ -295,11 +296,11 @@ void launch_wall_collide(const DevCloud &c, const DmArgs &dm, double *g, const d
                          double tau, double R, double *rho, double *ux, double *uy,
                          double *uz, double *T, double *pmass, hipStream_t s,
                          const int *guard = nullptr);
-// fold_scale1: after launch_commit_collide2, whose wall densities still
-// lack the first rescale, the boundary particles' rho is multiplied by it.
+// rho_wall: after launch_commit_collide2/3, whose wall densities still lack
+// the first rescale, the boundary particles' rho is rho_wall times it.
 void launch_final(const DevCloud &c, double *g, const double *scal, double R, double *rho,
                   double *ux, double *uy, double *uz, double *T, double *pmass,
-                  hipStream_t s, const int *guard = nullptr, bool fold_scale1 = false);
+                  hipStream_t s, const int *guard = nullptr, const double *rho_wall = nullptr);
 // The 2-D step's positivity, commit, wall and collision in one pass (the
 // first rescale folded into the end-of-step one): g from gt, the committed
 // masses into pnew, the collided masses into pmass.
@@ -307,6 +308,12 @@ void launch_commit_collide2(const DevCloud &c, double *g, const double *gt, doub
                             double tau, double R, double *rho, double *ux, double *uy,
                             double *T, double *limflag, double *pnew, double *pmass,
                             hipStream_t s);
+// The same of the 3-D step (continuous collision); the wall densities into
+// rho_wall, rho itself only read (NAD).
+void launch_commit_collide3(const DevCloud &c, double *g, const double *gt, double dt,
+                            double tau, double R, const double *rho, double *rho_wall, double *ux,
+                            double *uy, double *uz, double *T, double *limflag, double *pnew,
+                            double *pmass, hipStream_t s);
 
 // ---- k_neigh.hip -------------------------------------------------------------
 int launch_neighbours(const DevCloud &c, const ab_config &cfg, int *vox, int *vcount,

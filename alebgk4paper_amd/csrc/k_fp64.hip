@@ -1,12 +1,14 @@
 // k_fp64.hip -- the reference formulation of the ALE-BGK step in FP64 on gfx950
 // after its transport (k_mls.hip).
 //
-// Per-particle stages: one 256-thread workgroup per particle, coalesced over
-// the node index, with fixed-order workgroup reductions. They fuse reference
-// kernels that touch only their own particle:
-//   limit_commit  kPositivity3D + kNAD3D + kCommit  (+ mass partial)
-//   wall_collide  kScaleG + kWallBC3D + kMoments3D + kCollisionNode3D
-//   final         kScaleG + kMoments3D
+// Per-particle stages, fixed-order reductions, fusing reference kernels that
+// touch only their own particle:
+//   commit_collide3 / 2  kPositivity + kNAD3D + kCommit + kScaleG + kWallBC /
+//                 kMoments + kCollisionNode (the continuous collision)
+//   limit_commit  kPositivity3D + kNAD3D + kCommit  (+ mass partial) and
+//   wall_collide  kScaleG + kWallBC + kMoments + kCollisionNode, where the
+//                 discrete collision or the MOOD limiter comes between
+//   final         kScaleG + kMoments
 // and the global sums stay on the device (no host round trip per rescale).
 #include "ab_device.hpp"
 #include "ab_dm.hpp"
@@ -49,8 +51,25 @@ __global__ __launch_bounds__(1024) void k_reduce_mass(int N, const double *__res
         hi = seg[blockIdx.x + 1];
         scal += (size_t)blockIdx.x * S_COUNT;
     }
+    // eight loads in flight per thread while eight are left: the one workgroup
+    // is bound by their latency (64,000 particles: 29 -> 21 us)
+    constexpr int U = 8;
     double s = 0.0, sn = 0.0;
-    for (int i = lo + threadIdx.x; i < hi; i += 1024)
+    int i = lo + (int)threadIdx.x;
+    for (; i + (U - 1) * 1024 < hi; i += U * 1024)
+    {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = pmass[i + u * 1024];
+#pragma unroll
+        for (int u = 0; u < U; ++u) s += v[u];
+        if (!pnew) continue;
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = pnew[i + u * 1024];
+#pragma unroll
+        for (int u = 0; u < U; ++u) sn += v[u];
+    }
+    for (; i < hi; i += 1024)
     {
         s += pmass[i];
         if (pnew) sn += pnew[i];
@@ -89,10 +108,9 @@ __global__ __launch_bounds__(1024) void k_reduce_mass(int N, const double *__res
     }
 }
 
-// kPositivity3D + kNAD3D + kCommit (CudaBackend.cu:882-954, 328-336) for 3-D;
-// kPositivity + kCommit (:304-336) for 2-D. Writes the committed g, the
+// kPositivity3D + kNAD3D + kCommit (CudaBackend.cu:882-954, 328-336) of the
+// step with the discrete collision. Writes the committed g, the
 // limiter bits and the particle's mass.
-template <int DIM>
 __global__ __launch_bounds__(kBlock) void k_limit_commit(DevCloud c, double *__restrict__ g,
                                                          const double *__restrict__ gt,
                                                          const double *__restrict__ rho,
@@ -110,94 +128,63 @@ __global__ __launch_bounds__(kBlock) void k_limit_commit(DevCloud c, double *__r
     double sc = 1.0, sc2 = 1.0;
     bool fires = false, nad = false;
 
-    if constexpr (DIM == 3)
+    const double dv3 = c.dv * c.dv * c.dv;
+    double r[3] = {0.0, 0.0, 0.0};             // mPos, mNeg, mFallback
+    for (int k = lane; k < nodes; k += kWave)
     {
-        const double dv3 = c.dv * c.dv * c.dv;
-        double r[3] = {0.0, 0.0, 0.0};             // mPos, mNeg, mFallback
-        for (int k = lane; k < nodes; k += kWave)
-        {
-            double v = tp[k];
-            if (v >= 0) r[0] += v;
-            else { r[1] += v; r[2] += gp[k]; }
-        }
-        wave_sums<3>(r);
-        fires = (r[1] < -1e-30 && (r[0] + r[1]) > 0);
-        if (fires)
-        {
-            flag += 1.0;
-            double target = r[0] + r[1], replaced = r[0] + r[2];
-            sc = (replaced > 1e-30) ? target / replaced : 0.0;
-        }
-        if (!c.bnd[i])
-        {
-            double rn[1] = {0.0};
-            for (int k = lane; k < nodes; k += kWave)
-            {
-                double v = tp[k];
-                if (fires) v = ((v < 0.0) ? gp[k] : v) * sc;
-                rn[0] += v;
-            }
-            wave_sums<1>(rn);
-            const double rho_new = rn[0] * dv3;
-            const int nn = c.nneigh[i];
-            double rmin = 1e300, rmax = -1e300;
-            for (int k = lane; k < nn; k += kWave)
-            {
-                double q = rho[c.neigh[(size_t)i * AB_MAX_NEIGH + k]];
-                rmin = fmin(rmin, q);
-                rmax = fmax(rmax, q);
-            }
-            rmin = wave_min(rmin);
-            rmax = wave_max(rmax);
-            if (!(rmin > rmax))
-            {
-                double slack = 0.1 * fmax(rmax - rmin, 1e-12) + 1e-9;
-                double lo = rmin - slack, hi = rmax + slack;
-                if (rho_new > hi && rho_new > 1e-30) { nad = true; sc2 = hi / rho_new; }
-                else if (rho_new < lo && rho_new > 1e-30) { nad = true; sc2 = lo / rho_new; }
-                if (nad) flag += 2.0;
-            }
-        }
-        double m[1] = {0.0};
+        double v = tp[k];
+        if (v >= 0) r[0] += v;
+        else { r[1] += v; r[2] += gp[k]; }
+    }
+    wave_sums<3>(r);
+    fires = (r[1] < -1e-30 && (r[0] + r[1]) > 0);
+    if (fires)
+    {
+        flag += 1.0;
+        double target = r[0] + r[1], replaced = r[0] + r[2];
+        sc = (replaced > 1e-30) ? target / replaced : 0.0;
+    }
+    if (!c.bnd[i])
+    {
+        double rn[1] = {0.0};
         for (int k = lane; k < nodes; k += kWave)
         {
             double v = tp[k];
             if (fires) v = ((v < 0.0) ? gp[k] : v) * sc;
-            if (nad) v *= sc2;
-            gp[k] = v;
-            m[0] += v * dv3;
+            rn[0] += v;
         }
-        wave_sums<1>(m);
-        if (lane == 0) { pmass[i] = m[0]; limflag[i] = flag; }
+        wave_sums<1>(rn);
+        const double rho_new = rn[0] * dv3;
+        const int nn = c.nneigh[i];
+        double rmin = 1e300, rmax = -1e300;
+        for (int k = lane; k < nn; k += kWave)
+        {
+            double q = rho[c.neigh[(size_t)i * AB_MAX_NEIGH + k]];
+            rmin = fmin(rmin, q);
+            rmax = fmax(rmax, q);
+        }
+        rmin = wave_min(rmin);
+        rmax = wave_max(rmax);
+        if (!(rmin > rmax))
+        {
+            double slack = 0.1 * fmax(rmax - rmin, 1e-12) + 1e-9;
+            double lo = rmin - slack, hi = rmax + slack;
+            if (rho_new > hi && rho_new > 1e-30) { nad = true; sc2 = hi / rho_new; }
+            else if (rho_new < lo && rho_new > 1e-30) { nad = true; sc2 = lo / rho_new; }
+            if (nad) flag += 2.0;
+        }
     }
-    else
+    double m[1] = {0.0};
+    for (int k = lane; k < nodes; k += kWave)
     {
-        double r[2] = {0.0, 0.0};                  // mPos, mNeg of g1
-        for (int k = lane; k < nodes; k += kWave)
-        {
-            double v = tp[k];
-            if (v >= 0) r[0] += v; else r[1] += v;
-        }
-        wave_sums<2>(r);
-        fires = (r[1] < -1e-30 && r[0] > 1e-30 && (r[0] + r[1]) > 0);
-        if (fires) { flag += 1.0; sc = (r[0] + r[1]) / r[0]; }
-        const double dv2 = c.dv * c.dv;
-        double m[1] = {0.0};
-        for (int k = lane; k < nodes; k += kWave)
-        {
-            double v1 = tp[k], v2 = tp[k + nodes];
-            if (fires)
-            {
-                if (v1 < 0) { v1 = 0; v2 = 0; }
-                else { v1 *= sc; v2 *= sc; }
-            }
-            gp[k] = v1;
-            gp[k + nodes] = v2;
-            m[0] += v1 * dv2;
-        }
-        wave_sums<1>(m);
-        if (lane == 0) { pmass[i] = m[0]; limflag[i] = flag; }
+        double v = tp[k];
+        if (fires) v = ((v < 0.0) ? gp[k] : v) * sc;
+        if (nad) v *= sc2;
+        gp[k] = v;
+        m[0] += v * dv3;
     }
+    wave_sums<1>(m);
+    if (lane == 0) { pmass[i] = m[0]; limflag[i] = flag; }
 }
 
 // kScaleG (massOld/massNew) + kWallBC3D / kMoments3D + kCollisionNode3D
@@ -614,6 +601,247 @@ __global__ __launch_bounds__(kBlock) void k_commit_collide2(DevCloud c, double *
     }
 }
 
+// The 3-D step's kPositivity3D + kNAD3D + kCommit + kScaleG + kWallBC3D /
+// kMoments3D + kCollisionNode3D (CudaBackend.cu:882-954, 328-336, 478-485,
+// 956-1030, 532-569, 1181-1197) in one pass per particle, one wave each, with
+// the rescale between commit and collision left to the end of the step as in
+// k_commit_collide2 (wall density, moments and Maxwellians scale with g). The
+// row is read once and the collided one written once; k_limit_commit<3> and
+// k_wall_collide<3> read three rows and wrote two. What bounded those beside
+// the traffic was an FP64 exponential per node: the velocity grid is a tensor
+// product, so exp(-|v - u|^2 / 2RT) is the product of three factors, 3 Nv
+// exponentials a particle. 40^3 / Nv 10: 332 + 686 -> 286 us, 3.6 TB/s of its one
+// read and one write.
+//
+// NAD compares with the neighbours' densities of the step's start, which must
+// not change while other particles still read them: the wall densities go to
+// rho_wall, and k_final writes rho.
+// U > 0: rows of at most U * 64 nodes stay in registers; U == 0: any row, read
+// again from the cache in each pass, in the same order of sums.
+// mg1, mg2: ceil(2^32 / Nv), ceil(2^32 / Nv^2), exact quotients for k < Nv^3.
+template <int U>
+__global__ __launch_bounds__(kBlock) void k_commit_collide3(
+    DevCloud c, double *__restrict__ g, const double *__restrict__ gt, unsigned mg1, unsigned mg2,
+    double dt, double tau, double R, const double *__restrict__ rho, double *__restrict__ rho_wall,
+    double *ux, double *uy, double *uz, double *T, double *__restrict__ limflag,
+    double *__restrict__ pnew, double *__restrict__ pmass)
+{
+    __shared__ double tab[kBlock / kWave][3][kMaxNv];
+    const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    const int i = xcd_remap(blockIdx.x, gridDim.x) * (kBlock / kWave) + w;
+    if (i >= c.N) return;                              // whole wave: one particle
+    const size_t gs = (size_t)c.gstride;
+    double *gp = g + (size_t)i * gs;
+    const double *tp = gt + (size_t)i * gs;
+    const int nodes = c.nodes, Nv = c.Nv;
+    const double dv3 = c.dv * c.dv * c.dv;
+    const int nu = U > 0 ? U : (nodes + kWave - 1) / kWave;
+
+    double t[U > 0 ? U : 1];
+    if constexpr (U > 0)
+    {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+        {
+            const int k = lane + u * kWave;
+            t[u] = k < nodes ? tp[k] : 0.0;
+        }
+    }
+    const bool wall = c.bnd[i];
+    // the neighbours' densities while the row is on its way
+    double rmin = 1e300, rmax = -1e300;
+    if (!wall)
+    {
+        const int nn = c.nneigh[i];
+        for (int k = lane; k < nn; k += kWave)
+        {
+            const double q = rho[c.neigh[(size_t)i * AB_MAX_NEIGH + k]];
+            rmin = fmin(rmin, q);
+            rmax = fmax(rmax, q);
+        }
+    }
+    double r[3] = {0.0, 0.0, 0.0};                     // mPos, mNeg, mFallback
+#pragma unroll
+    for (int u = 0; u < nu; ++u)
+    {
+        const int k = lane + u * kWave;
+        if (k >= nodes) continue;
+        double v;
+        if constexpr (U > 0) v = t[u]; else v = tp[k];
+        if (v >= 0) r[0] += v;
+        else { r[1] += v; r[2] += gp[k]; }
+    }
+    wave_sums<3>(r);
+    double flag = 0.0, sc = 1.0, sc2 = 1.0;
+    const bool fires = (r[1] < -1e-30 && (r[0] + r[1]) > 0);
+    if (fires)
+    {
+        flag += 1.0;
+        const double target = r[0] + r[1], replaced = r[0] + r[2];
+        sc = (replaced > 1e-30) ? target / replaced : 0.0;
+    }
+    // the committed value of node k (register u)
+    auto committed = [&](int u, int k) {
+        double v;
+        if constexpr (U > 0) v = t[u]; else v = tp[k];
+        if (fires) v = ((v < 0.0) ? gp[k] : v) * sc;
+        return v * sc2;
+    };
+    if (!wall)
+    {
+        double rn = r[0] + r[1];
+        if (fires)
+        {
+            rn = 0.0;
+#pragma unroll
+            for (int u = 0; u < nu; ++u)
+            {
+                const int k = lane + u * kWave;
+                if (k < nodes) rn += committed(u, k);
+            }
+            rn = wave_sum(rn);
+        }
+        const double rho_new = rn * dv3;
+        rmin = wave_min(rmin);
+        rmax = wave_max(rmax);
+        if (!(rmin > rmax))
+        {
+            const double slack = 0.1 * fmax(rmax - rmin, 1e-12) + 1e-9;
+            const double lo = rmin - slack, hi = rmax + slack;
+            bool nad = false;
+            if (rho_new > hi && rho_new > 1e-30) { nad = true; sc2 = hi / rho_new; }
+            else if (rho_new < lo && rho_new > 1e-30) { nad = true; sc2 = lo / rho_new; }
+            if (nad) flag += 2.0;
+        }
+    }
+    if constexpr (U > 0)
+    {
+        // commit: the later passes read the register
+        if (fires || sc2 != 1.0)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+            {
+                const int k = lane + u * kWave;
+                if (k < nodes) t[u] = committed(u, k);
+            }
+    }
+    auto value = [&](int u, int k) { if constexpr (U > 0) return t[u]; else return committed(u, k); };
+    auto node = [&](int k, int &iv, int &jv, int &kv) {
+        kv = (int)__umulhi((unsigned)k, mg2);
+        const int p = k - kv * (Nv * Nv);
+        jv = (int)__umulhi((unsigned)p, mg1);
+        iv = p - jv * Nv;
+    };
+    // the three factors of exp(-|v - u|^2 / (2RT)), one entry per lane and pass
+    auto factors = [&](double ax, double ay, double az, double twoRT) {
+        for (int e = lane; e < 3 * Nv; e += kWave)
+        {
+            const int axis = e / Nv, l = e - axis * Nv;
+            const double d = vnode(c.vlo, c.dv, l) - (axis == 0 ? ax : axis == 1 ? ay : az);
+            tab[w][axis][l] = exp(-(d * d) / twoRT);
+        }
+        wave_lds_sync();
+    };
+    double m = 0.0, mnew = 0.0;
+    if (wall)
+    {
+        const double nx = c.wnx[i], ny = c.wny[i], nz = c.wnz[i];
+        const double Ux = c.wux[i], Uy = c.wuy[i], Uz = c.wuz[i], Tw = c.wt[i];
+        const double RT2w = 2.0 * R * Tw, in = 1.0 / pow(AB_PI * RT2w, 1.5);
+        factors(Ux, Uy, Uz, RT2w);
+        double q[3] = {0.0, 0.0, 0.0};                 // intM, intP, committed mass
+        auto cn_of = [&](int iv, int jv, int kv) {
+            return wall_cn3(vnode(c.vlo, c.dv, iv), vnode(c.vlo, c.dv, jv), vnode(c.vlo, c.dv, kv),
+                            Ux, Uy, Uz, nx, ny, nz);
+        };
+#pragma unroll
+        for (int u = 0; u < nu; ++u)
+        {
+            const int k = lane + u * kWave;
+            if (k >= nodes) continue;
+            int iv, jv, kv;
+            node(k, iv, jv, kv);
+            const double v = value(u, k), cn = cn_of(iv, jv, kv);
+            if (cn < 0.0) q[0] += cn * v;
+            else if (cn > 0.0) q[1] += cn * (tab[w][0][iv] * tab[w][1][jv] * tab[w][2][kv]);
+            q[2] += v;
+        }
+        wave_sums<3>(q);
+        const double intM = q[0] * dv3, intP = q[1] * in * dv3;
+        const double rho_w = (intP > 1e-30) ? (-intM / intP) : 1.0, am = rho_w * in;
+        mnew = q[2] * dv3;
+#pragma unroll
+        for (int u = 0; u < nu; ++u)
+        {
+            const int k = lane + u * kWave;
+            if (k >= nodes) continue;
+            int iv, jv, kv;
+            node(k, iv, jv, kv);
+            double v = value(u, k);
+            if (cn_of(iv, jv, kv) > 0.0) v = am * (tab[w][0][iv] * tab[w][1][jv] * tab[w][2][kv]);
+            gp[k] = v;
+            m += v;
+        }
+        if (lane == 0) { rho_wall[i] = rho_w; ux[i] = Ux; uy[i] = Uy; uz[i] = Uz; T[i] = Tw; }
+    }
+    else
+    {
+        double q[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int u = 0; u < nu; ++u)
+        {
+            const int k = lane + u * kWave;
+            if (k >= nodes) continue;
+            int iv, jv, kv;
+            node(k, iv, jv, kv);
+            const double vx = vnode(c.vlo, c.dv, iv), vy = vnode(c.vlo, c.dv, jv),
+                         vz = vnode(c.vlo, c.dv, kv);
+            const double f = value(u, k);
+            q[0] += f;
+            q[1] += vx * f;
+            q[2] += vy * f;
+            q[3] += vz * f;
+            q[4] += (vx * vx + vy * vy + vz * vz) * f;
+        }
+        wave_sums<5>(q);
+#pragma unroll
+        for (int a = 0; a < 5; ++a) q[a] *= dv3;
+        mnew = q[0];
+        double mrho = rho[i], mux = ux[i], muy = uy[i], muz = uz[i], mT = T[i];
+        if (q[0] > 1e-30)
+        {
+            mrho = q[0];
+            mux = q[1] / q[0];
+            muy = q[2] / q[0];
+            muz = q[3] / q[0];
+            const double t1 = (q[4] / q[0] - (mux * mux + muy * muy + muz * muz)) / (3.0 * R);
+            mT = t1 > 1e-6 ? t1 : 1e-6;
+        }
+        const double lam = dt / tau, coeff = 1.0 / (1.0 + lam);
+        const double twoRT = 2.0 * R * mT, am = lam * mrho / pow(AB_PI * twoRT, 1.5);
+        factors(mux, muy, muz, twoRT);
+#pragma unroll
+        for (int u = 0; u < nu; ++u)
+        {
+            const int k = lane + u * kWave;
+            if (k >= nodes) continue;
+            int iv, jv, kv;
+            node(k, iv, jv, kv);
+            const double f = coeff * (value(u, k) + am * (tab[w][0][iv] * tab[w][1][jv] * tab[w][2][kv]));
+            gp[k] = f;
+            m += f;
+        }
+        if (lane == 0) { ux[i] = mux; uy[i] = muy; uz[i] = muz; T[i] = mT; }
+    }
+    m = wave_sum(m) * dv3;
+    if (lane == 0)
+    {
+        pmass[i] = m;
+        pnew[i] = mnew;
+        limflag[i] = flag;
+    }
+}
+
 // kScaleG (massOld/massColl) + kMoments3D / kMoments (CudaBackend.cu:1773-1788).
 // One wave per particle, four per workgroup: each lane loads four nodes of
 // both layers before it adds any, and the sums are wave reductions, so a
@@ -625,7 +853,7 @@ __global__ __launch_bounds__(kBlock) void k_final(DevCloud c, double *__restrict
                                                   double *uz, double *T,
                                                   double *__restrict__ pmass,
                                                   const int *__restrict__ guard,
-                                                  bool fold_scale1)
+                                                  const double *rho_wall)
 {
     constexpr int kPer = kBlock / kWave;
     const int i = xcd_remap(blockIdx.x, gridDim.x) * kPer + (int)(threadIdx.x / kWave);
@@ -687,7 +915,7 @@ __global__ __launch_bounds__(kBlock) void k_final(DevCloud c, double *__restrict
     if (lane == 0)
     {
         pmass[i] = r[5];
-        if (!inner && fold_scale1) rho[i] *= s1;
+        if (!inner && rho_wall) rho[i] = rho_wall[i] * s1;
         if (inner && r[0] > 1e-30)
         {
             double mux = r[1] / r[0], muy = r[2] / r[0], muz = 0.0, u2;
@@ -855,8 +1083,7 @@ void launch_limit_commit(const DevCloud &c, double *g, const double *gt, const d
                          double *limflag, double *pmass, hipStream_t s)
 {
     const int nb = (c.N + kBlock / kWave - 1) / (kBlock / kWave);
-    if (c.dim == 3) k_limit_commit<3><<<nb, kBlock, 0, s>>>(c, g, gt, rho, limflag, pmass);
-    else k_limit_commit<2><<<nb, kBlock, 0, s>>>(c, g, gt, rho, limflag, pmass);
+    k_limit_commit<<<nb, kBlock, 0, s>>>(c, g, gt, rho, limflag, pmass);
 }
 
 void launch_wall_collide(const DevCloud &c, const DmArgs &dm, double *g, const double *scal,
@@ -874,15 +1101,15 @@ void launch_wall_collide(const DevCloud &c, const DmArgs &dm, double *g, const d
 
 void launch_final(const DevCloud &c, double *g, const double *scal, double R, double *rho,
                   double *ux, double *uy, double *uz, double *T, double *pmass, hipStream_t s,
-                  const int *guard, bool fold_scale1)
+                  const int *guard, const double *rho_wall)
 {
     const int nb = (c.N + kBlock / kWave - 1) / (kBlock / kWave);
     if (c.dim == 3)
         k_final<3><<<nb, kBlock, 0, s>>>(c, g, scal, R, rho, ux, uy, uz, T, pmass, guard,
-                                         fold_scale1);
+                                         rho_wall);
     else
         k_final<2><<<nb, kBlock, 0, s>>>(c, g, scal, R, rho, ux, uy, uz, T, pmass, guard,
-                                         fold_scale1);
+                                         rho_wall);
 }
 
 void launch_commit_collide2(const DevCloud &c, double *g, const double *gt, double dt,
@@ -905,6 +1132,27 @@ void launch_commit_collide2(const DevCloud &c, double *g, const double *gt, doub
     else
         k_commit_collide2<0><<<nb, kBlock, 0, s>>>(c, g, gt, dt, tau, R, rho, ux, uy, T, limflag,
                                                    pnew, pmass);
+}
+
+void launch_commit_collide3(const DevCloud &c, double *g, const double *gt, double dt,
+                            double tau, double R, const double *rho, double *rho_wall, double *ux,
+                            double *uy, double *uz, double *T, double *limflag, double *pnew,
+                            double *pmass, hipStream_t s)
+{
+    const int nb = (c.N + kBlock / kWave - 1) / (kBlock / kWave);
+    const unsigned n1 = (unsigned)c.Nv, n2 = n1 * n1;
+    const unsigned mg1 = (unsigned)((0x100000000ull + n1 - 1) / n1),
+                   mg2 = (unsigned)((0x100000000ull + n2 - 1) / n2);
+    auto go = [&](auto kernel) {
+        kernel<<<nb, kBlock, 0, s>>>(c, g, gt, mg1, mg2, dt, tau, R, rho, rho_wall, ux, uy, uz, T,
+                                     limflag, pnew, pmass);
+    };
+    // rows of up to 1,024 nodes (Nv <= 10) stay in registers
+    const int u = (c.nodes + kWave - 1) / kWave;
+    if (u <= 4) go(k_commit_collide3<4>);
+    else if (u <= 8) go(k_commit_collide3<8>);
+    else if (u <= 16) go(k_commit_collide3<16>);
+    else go(k_commit_collide3<0>);
 }
 
 void launch_mood_check(const DevCloud &c, double *gt, const double *rho, int *mood,
