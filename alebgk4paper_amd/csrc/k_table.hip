@@ -859,15 +859,22 @@ __device__ __forceinline__ void blk_ends(const T *__restrict__ g, const T *__res
     (end_step<T, TX, TY, TOP, CLAMP, U>(a, pb, ca, cb, v, aw, an), ...);
 }
 
-// One wave = a TX x TY block of columns with origin (bx, by), all of the
+// Blocks of width t that cover the interior columns of n.
+__host__ __device__ constexpr int blocks(int n, int t) { return (n - 4 + t - 1) / t; }
+
+// One wave = a TX x TY block of columns with origin (x0, y0), all of the
 // x/y class (cx, cy), x one 64-node chunk. Interior blocks (cx = cy = 2)
 // lie two columns inside the lattice; edge blocks (CLAMP) run along an edge
 // of the lattice, their stencil columns clamped to it.
 template <typename T, int TX, int TY, int K, bool CLAMP, int R = 2, int ZB = 1>
 __device__ __forceinline__ void block_at(const Lat &L, const T *__restrict__ g, T *__restrict__ gt,
-                                         const T *__restrict__ coef, int chunk, int bx, int by,
+                                         const T *__restrict__ coef, int chunk, int x0, int y0,
                                          int cx, int cy, int slab, int voff)
 {
+    // A lattice whose interior is no multiple of the block: the last block is
+    // moved back inside and leaves the columns before (x0, y0) to the block
+    // that owns them.
+    const int bx = TX > 1 ? min(x0, L.nx - 2 - TX) : x0, by = TY > 1 ? min(y0, L.ny - 2 - TY) : y0;
     const size_t plane = (size_t)L.nx * L.ny;
     const size_t c0 = (size_t)chunk * kWave;
     const T *gw = g + c0;
@@ -876,6 +883,7 @@ __device__ __forceinline__ void block_at(const Lat &L, const T *__restrict__ g, 
         return coef + ((size_t)(cx + 5 * (cy + 5 * cz)) * L.nchunk + chunk) * kOff * kWave;
     };
     auto store = [&](int t, int iz, T v) {
+        if (bx + t % TX < x0 || by + t / TX < y0) return;
         bstore(gtw + ((size_t)(bx + t % TX) + (size_t)L.nx * (by + t / TX) + plane * iz) * L.S, voff, v);
     };
     auto end_pair = [&](auto top) {
@@ -923,14 +931,14 @@ __device__ __forceinline__ void block_at(const Lat &L, const T *__restrict__ g, 
     march(cr);
 }
 
-// Interior block blk (row-major over the interior). Requires (nx - 4) % TX
-// == 0 and (ny - 4) % TY == 0.
+// Interior block blk (row-major over the interior). Requires nx - 4 >= TX and
+// ny - 4 >= TY.
 template <typename T, int TX, int TY, int K, int R = 2, int ZB = 1>
 __device__ __forceinline__ void block_wave(const Lat &L, const T *__restrict__ g, T *__restrict__ gt,
                                            const T *__restrict__ coef, int chunk, int blk, int slab,
                                            int voff)
 {
-    const int nbx = (L.nx - 4) / TX;
+    const int nbx = blocks(L.nx, TX);
     block_at<T, TX, TY, K, false, R, ZB>(L, g, gt, coef, chunk, 2 + (blk % nbx) * TX,
                                   2 + (blk / nbx) * TY, 2, 2, slab, voff);
 }
@@ -938,7 +946,7 @@ __device__ __forceinline__ void block_wave(const Lat &L, const T *__restrict__ g
 // The whole transport in one launch: per chunk, the edge columns (z blocks
 // of KE), then the interior blocks (TX x TY columns per wave). One
 // launch keeps the edge waves from running as a second, short and
-// latency-bound grid after the blocks. Where the interior is a multiple of 4
+// latency-bound grid after the blocks. Where the interior is at least 4
 // columns wide, the edge columns along an edge share a class and run as
 // blocks too: 1 x 4 along the x edges (ix = 0, 1, nx-2, nx-1), 4 x 1 along
 // the y edges, and only the 16 corner columns one per wave.
@@ -951,16 +959,13 @@ __device__ __forceinline__ void block_wave(const Lat &L, const T *__restrict__ g
 template <int K>
 __host__ __device__ constexpr int zblocks(int nz) { return (nz - 4 + K - 1) / K; }
 
-__host__ __device__ inline bool edge_blocks(int nx, int ny)
-{
-    return ((nx - 4) & 3) == 0 && ((ny - 4) & 3) == 0;
-}
+__host__ __device__ inline bool edge_blocks(int nx, int ny) { return nx >= 8 && ny >= 8; }
 
 // edge waves per chunk: blocks along the four x edges and four y edges plus
 // the corners, or one wave per edge column
 __host__ __device__ inline int edge_items(int nx, int ny, int slabs = 1)
 {
-    return edge_blocks(nx, ny) ? ((ny - 4) + (nx - 4)) * slabs + 16 : nx * ny - (nx - 4) * (ny - 4);
+    return edge_blocks(nx, ny) ? 4 * (blocks(nx, 4) + blocks(ny, 4)) * slabs + 16 : nx * ny - (nx - 4) * (ny - 4);
 }
 
 // Edge blocks march in z blocks of at most kEdgeK (12 would raise the
@@ -980,7 +985,7 @@ template <typename T, int TX, int TY, int K, int KE, int SLAB, int R = 2>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void k_apply_mix(Lat L, const T *__restrict__ g, T *__restrict__ gt, const T *__restrict__ coef)
 {
-    const int nblk = ((L.nx - 4) / TX) * ((L.ny - 4) / TY);
+    const int nblk = blocks(L.nx, TX) * blocks(L.ny, TY);
     const int nitem = SLAB ? nblk * (zblocks<SLAB * K>(L.nz) + 1) : nblk;
     const int eslabs = edge_slabs(SLAB != 0, L.nz);
     const int per = nitem + edge_items(L.nx, L.ny, eslabs);
@@ -1004,7 +1009,7 @@ void k_apply_mix(Lat L, const T *__restrict__ g, T *__restrict__ gt, const T *__
     static_assert(!SLAB || KB == kEdgeK, "edge slabs are counted in z blocks of kEdgeK");
     if (edge_blocks(L.nx, L.ny))
     {
-        const int qy = (L.ny - 4) / 4, qx = (L.nx - 4) / 4;
+        const int qy = blocks(L.ny, 4), qx = blocks(L.nx, 4);
         const int nblke = 4 * (qx + qy);
         if (e < nblke * eslabs)
         {
@@ -1860,13 +1865,13 @@ void launch_shape(int i, Lat L, const T *g, T *gt, const T *cf, const double *sc
                   hipStream_t s)
 {
     auto waves = [&](int ncol) { return (ncol * L.nchunk + 3) / 4; };
-    const int all = L.nx * L.ny, inner = (L.nx - 4) * (L.ny - 4);
+    const int all = L.nx * L.ny;
     if constexpr (sizeof(T) == 4)
     {
         const ApplyShape sh = kShapes32[i];
         if (sh.TX > 1)
         {
-            const int nblk = inner / (sh.TX * sh.TY);
+            const int nblk = blocks(L.nx, sh.TX) * blocks(L.ny, sh.TY);
             const int nw = (sh.S ? nblk * ((L.nz - 4 + sh.S * sh.K - 1) / (sh.S * sh.K) + 1) : nblk) +
                            edge_items(L.nx, L.ny, edge_slabs(sh.S != 0, L.nz));
             switch (i)
@@ -1896,25 +1901,28 @@ void launch_shape(int i, Lat L, const T *g, T *gt, const T *cf, const double *sc
     }
 }
 
-// A shape applies to this lattice (blocks must tile the interior columns).
+// A shape applies to this lattice (a block must fit into the interior columns).
 template <typename T>
 bool shape_fits(int i, int nx, int ny)
 {
     const ApplyShape sh = shape_at<T>(i);
-    return sh.TX == 1 || ((nx - 4) % sh.TX == 0 && (ny - 4) % sh.TY == 0 && nx > 4 && ny > 4);
+    return sh.TX == 1 || (nx - 4 >= sh.TX && ny - 4 >= sh.TY);
 }
 
-// Default shape before tuning: in FP32 the 2 x 4 column blocks with K = 6
-// in the slab order where they tile the interior (the fastest shape measured,
-// 267 us at 40^3 / Nv 10 and 860 us at 60^3 / Nv 10, against 612 and 1934
-// us for single columns), else the 2 x 2 blocks, else single columns; in
-// FP64 the single-column z block that divides the interior run.
+// Default shape before tuning. FP32: the 2 x 4 column blocks with K = 6 in the
+// slab order, the fastest shape from 10^3 to 60^3 particles whether or not
+// they tile the interior (us against single columns: 264 / 580 at 40^3 / Nv 10,
+// 986 / 2423 at 31^3 / Nv 20, 66 / 125 at 21^3 / Nv 10, 21 / 31 at 10^3 / Nv 10).
+// Single columns in z blocks of 9 where the launch has fewer of them than the
+// chip has SIMDs: every wave then runs alone and the shorter one ends first
+// (18.2 / 22.2 us at 13^3 / Nv 7, 16.4 / 19.4 at 11^3 / Nv 6), and where no block
+// fits. FP64: the single-column z block that divides the interior run.
 template <typename T>
-int default_shape(int nx, int ny, int nz)
+int default_shape(const Lat &L)
 {
     if (sizeof(T) == 4)
-        return shape_fits<T>(5, nx, ny) ? 5 : (shape_fits<T>(3, nx, ny) ? 3 : 0);
-    const int run = nz - 4;
+        return L.nx * L.ny * L.nchunk < 1024 || !shape_fits<T>(5, L.nx, L.ny) ? 1 : 5;
+    const int run = L.nz - 4;
     return run % 9 == 0 ? 0 : (run % 7 == 0 ? 2 : 1);
 }
 
@@ -1928,7 +1936,7 @@ int apply_launch(ab_ctx *ctx, const Lat &L, int shape)
         return AB_ERR_UNSUPPORTED;
     }
     if (shape < 0 || shape >= nshapes<T>() || !shape_fits<T>(shape, L.nx, L.ny))
-        shape = default_shape<T>(ctx->cfg.nx, ctx->cfg.ny, ctx->cfg.nz);
+        shape = default_shape<T>(L);
     launch_shape<T>(shape, L, (const T *)ctx->gs, (T *)ctx->gts, (const T *)ctx->coef, ctx->scal,
                     ctx->stream);
     return hipGetLastError() == hipSuccess ? AB_OK : AB_ERR_HIP;
@@ -2336,7 +2344,7 @@ int table_set_shape(ab_ctx *ctx, int shape)
     if (shape < -1 || shape >= ns) { ctx->err = "transport shape index out of range"; return AB_ERR_ARG; }
     const bool fits = shape < 0 || (is_fp32(ctx) ? shape_fits<float>(shape, ctx->cfg.nx, ctx->cfg.ny)
                                                  : shape_fits<double>(shape, ctx->cfg.nx, ctx->cfg.ny));
-    if (!fits) { ctx->err = "transport shape does not tile this lattice"; return AB_ERR_UNSUPPORTED; }
+    if (!fits) { ctx->err = "transport shape does not fit this lattice"; return AB_ERR_UNSUPPORTED; }
     ctx->apply_shape = shape;
     return AB_OK;
 }
