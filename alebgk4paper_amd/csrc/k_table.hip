@@ -35,6 +35,7 @@
 #include "ab_device.hpp"
 #include "ab_internal.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -239,14 +240,14 @@ __device__ void build_class(const DevCloud &c, int i, int lin, const int *lat, d
 
 template <typename T>
 __global__ void k_build(DevCloud c, const int *__restrict__ rep, const int *__restrict__ lat,
-                        double dt, double h, double tol, int order, T *__restrict__ coef, int S)
+                        double dt, double h, double tol, int order, T *__restrict__ coef, int nchunk)
 {
     const int cls = blockIdx.y;
     const int lin = blockIdx.x * blockDim.x + threadIdx.x;
-    if (lin >= S) return;
+    if (lin >= nchunk * kWave) return;
     // layout [class][64-node chunk][81 offsets][64 nodes]: a wave's 81
     // coefficient rows are one contiguous 81 x 64 block (constant offsets)
-    T *out = coef + ((size_t)cls * (S / kWave) + lin / kWave) * kOff * kWave + (lin % kWave);
+    T *out = coef + ((size_t)cls * nchunk + lin / kWave) * kOff * kWave + (lin % kWave);
     for (int o = 0; o < kOff; ++o) out[(size_t)o * kWave] = T(0);
     if (lin >= c.nodes) return;
     const int i = rep[cls];
@@ -483,6 +484,35 @@ __device__ __forceinline__ void column_of(const Lat &L, int e, bool edges, int &
     }
 }
 
+// The four end planes of a lattice column (ix, iy), one 64-node chunk, in pairs
+// (0, 1) and (nz-2, nz-1): their own classes, coefficients loaded per offset,
+// column values shared.
+template <typename T>
+__device__ __forceinline__ void column_ends(const Lat &L, const T *__restrict__ g, T *__restrict__ gt,
+                                            const T *__restrict__ coef, int chunk, int ix, int iy,
+                                            int voff)
+{
+    const int col = ix + L.nx * iy;
+    const int cx = category(ix, L.nx), cy = category(iy, L.ny);
+    const size_t plane = (size_t)L.nx * L.ny, c0 = (size_t)chunk * kWave;
+    const T *gw = g + c0;
+    T *gtw = gt + c0;
+    auto end_pair = [&](auto top) {
+        constexpr bool TOP = decltype(top)::value;
+        const int iz = TOP ? L.nz - 2 : 0;
+        const T *cfa = coef + ((size_t)(cx + 5 * (cy + 5 * category(iz, L.nz))) * L.nchunk + chunk) * kOff * kWave;
+        const T *cfb = coef + ((size_t)(cx + 5 * (cy + 5 * category(iz + 1, L.nz))) * L.nchunk + chunk) * kOff * kWave;
+        T a0, a1;
+        apply_pair<T, TOP>(gw, cfa, cfb, L, ix, iy, voff, a0, a1,
+                           std::make_integer_sequence<int, kCols>{});
+        bstore(gtw + ((size_t)col + plane * iz) * L.S, voff, a0);
+        bstore(gtw + ((size_t)col + plane * (iz + 1)) * L.S, voff, a1);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    end_pair(std::false_type{});
+    end_pair(std::true_type{});
+}
+
 // One wave = lattice column (ix, iy) x one 64-node chunk: the end-plane
 // pairs, then the interior march in z blocks of K outputs.
 template <typename T, int K>
@@ -498,22 +528,7 @@ __device__ __forceinline__ void column_wave(const Lat &L, const T *__restrict__ 
     const T *gw = g + c0;
     T *gtw = gt + c0;
 
-    // The four end planes, in pairs (0, 1) and (nz-2, nz-1): their own
-    // classes, coefficients loaded per offset, column values shared.
-    auto end_pair = [&](auto top) {
-        constexpr bool TOP = decltype(top)::value;
-        const int iz = TOP ? L.nz - 2 : 0;
-        const T *cfa = coef + ((size_t)(cx + 5 * (cy + 5 * category(iz, L.nz))) * L.nchunk + chunk) * kOff * kWave;
-        const T *cfb = coef + ((size_t)(cx + 5 * (cy + 5 * category(iz + 1, L.nz))) * L.nchunk + chunk) * kOff * kWave;
-        T a0, a1;
-        apply_pair<T, TOP>(gw, cfa, cfb, L, ix, iy, voff, a0, a1,
-                           std::make_integer_sequence<int, kCols>{});
-        bstore(gtw + ((size_t)col + plane * iz) * L.S, voff, a0);
-        bstore(gtw + ((size_t)col + plane * (iz + 1)) * L.S, voff, a1);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    end_pair(std::false_type{});
-    end_pair(std::true_type{});
+    column_ends(L, g, gt, coef, chunk, ix, iy, voff);
 
     // Interior planes iz = 2 .. nz-3 share one class: coefficients in
     // registers
@@ -1038,6 +1053,276 @@ void k_apply_mix(Lat L, const T *__restrict__ g, T *__restrict__ gt, const T *__
     int ix, iy;
     column_of(L, e, true, ix, iy);
     column_wave<T, KE>(L, g, gt, coef, chunk, ix, iy, voff);
+}
+
+// ---- the march through z -----------------------------------------------------
+// A block's planes zb .. ze of the interior z class. Plane by plane the values
+// of the union columns are loaded once each, and every value is added into the
+// outputs of the five planes z - 2 .. z + 2 that it reaches, whose sums wait in
+// registers (acc[a]: output plane p - 2 + a while plane p is read); plane p - 2
+// is complete after plane p. The loads run a ring of columns ahead of the
+// arithmetic, across the plane's end.
+//
+// FP64 runs this: 81 coefficients take 162 registers, so a z block of one
+// column was all that fitted beside them, at 30 loads per output; the march
+// keeps 20 sums for a 2 x 2 block and needs 8. us per transport at 27^3 / Nv 9,
+// 40^3 / Nv 10, 20^3 / Nv 8: 363, 1213, 127 -> 231, 785, 74. FP32 blocks are
+// bound by instruction issue and latency, not by loads: marched (2 x 4, 5.5
+// loads per output) they took 262 us at 40^3 / Nv 10 against 264 in z blocks
+// (9.2), and trimming their first and last planes spilled.
+// A block: TX x TY columns of x/y class (cx, cy), one 64-node chunk. x0, y0: the
+// first column it owns. A lattice whose interior is no multiple of the block:
+// the last block is moved back inside (bx, by) and leaves the columns before
+// (x0, y0) to the block that owns them. Interior blocks (cx = cy = 2) lie two
+// columns inside the lattice; edge blocks (CLAMP) run along an edge of it, their
+// stencil columns clamped to it.
+template <typename T, int TX, int TY>
+struct BlockAt
+{
+    Lat L;
+    const T *gw, *cf;                                  // the chunk's values and coefficients
+    T *gtw;
+    int x0, y0, bx, by, cx, cy, voff;
+    size_t plane;
+    __device__ BlockAt(const Lat &l, const T *g, T *gt, const T *coef, int chunk, int xo, int yo,
+                       int kx, int ky, int v)
+        : L(l), gw(g + (size_t)chunk * kWave), cf(coef + (size_t)chunk * kOff * kWave),
+          gtw(gt + (size_t)chunk * kWave), x0(xo), y0(yo), bx(TX > 1 ? min(xo, l.nx - 2 - TX) : xo),
+          by(TY > 1 ? min(yo, l.ny - 2 - TY) : yo), cx(kx), cy(ky), voff(v),
+          plane((size_t)l.nx * l.ny)
+    {}
+    __device__ __forceinline__ const T *rows(int cz) const
+    {
+        return cf + (size_t)(cx + 5 * (cy + 5 * cz)) * L.nchunk * kOff * kWave;
+    }
+    __device__ __forceinline__ void store(int t, int iz, T v) const
+    {
+        if (bx + t % TX < x0 || by + t / TX < y0) return;
+        bstore(gtw + ((size_t)(bx + t % TX) + (size_t)L.nx * (by + t / TX) + plane * iz) * L.S, voff, v);
+    }
+};
+
+template <int TX, int TY, int MAX>
+constexpr int march_ring()
+{
+    // the longest ring that divides the columns of a plane, so that a column
+    // has the same register on every plane
+    int r = 1;
+    for (int k = 2; k <= MAX; ++k)
+        if (Blk<TX, TY>::NU % k == 0) r = k;
+    return r;
+}
+
+// LO, HI: the sums the plane still reaches (the planes before zb and after ze
+// reach only some of the item's outputs).
+template <typename T, int TX, int TY, int LO, int HI, int U, int... TI>
+__device__ __forceinline__ void march_fma(const T (&cr)[kOff], T v, T (&acc)[5][TX * TY],
+                                          std::integer_sequence<int, TI...>)
+{
+    constexpr UCol uc = Blk<TX, TY>::ucol(U);
+    auto one = [&](auto tic) {
+        constexpr int t = decltype(tic)::value;
+        constexpr int c = col_of(uc.ox - t % TX, uc.oy - t / TX);
+        if constexpr (c >= 0)
+        {
+            constexpr int dc = col_at(c).d, o0 = col_at(c).o0;
+            // input plane p at offset dz = 2 - a of output plane p - 2 + a
+#pragma clang loop unroll(full)
+            for (int dz = -dc; dz <= dc; ++dz)
+                if (2 - dz >= LO && 2 - dz <= HI) acc[2 - dz][t] += cr[o0 + dz + dc] * v;
+        }
+    };
+    (one(std::integral_constant<int, TI>{}), ...);
+}
+
+template <typename T, int TX, int TY, bool CLAMP, int RG, int LO, int HI, int U>
+__device__ __forceinline__ void march_step(const BlkAddr<T, 1> &a, int next, const T (&cr)[kOff],
+                                           T (&v)[RG], T (&acc)[5][TX * TY])
+{
+    constexpr int NU = Blk<TX, TY>::NU, ahead = U + RG - 1;
+    if constexpr (ahead < NU)
+        v[ahead % RG] = bload_so<T>(a.r, a.lin, a.template cofs<ahead, TX, TY, CLAMP>());
+    else
+        v[ahead % RG] = bload_so<T>(a.r, a.lin, a.template cofs<ahead - NU, TX, TY, CLAMP>() + next);
+    march_fma<T, TX, TY, LO, HI, U>(cr, v[U % RG], acc, std::make_integer_sequence<int, TX * TY>{});
+#pragma clang loop unroll(full)
+    for (int k = 0; k < 5; ++k)
+#pragma clang loop unroll(full)
+        for (int t = 0; t < TX * TY; ++t) asm volatile("" : "+v"(acc[k][t])::"memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+template <typename T, int TX, int TY, bool CLAMP, int RG, int... U>
+__device__ __forceinline__ void march_prime(const BlkAddr<T, 1> &a, T (&v)[RG],
+                                            std::integer_sequence<int, U...>)
+{
+    ((v[U] = bload_so<T>(a.r, a.lin, a.template cofs<U, TX, TY, CLAMP>())), ...);
+}
+
+template <typename T, int TX, int TY, bool CLAMP, int RG, int LO, int HI, int... U>
+__device__ __forceinline__ void march_plane(const BlkAddr<T, 1> &a, int next, const T (&cr)[kOff],
+                                            T (&v)[RG], T (&acc)[5][TX * TY],
+                                            std::integer_sequence<int, U...>)
+{
+    (march_step<T, TX, TY, CLAMP, RG, LO, HI, U>(a, next, cr, v, acc), ...);
+}
+
+template <typename T, int TX, int TY, bool CLAMP>
+__device__ __forceinline__ void block_march(const BlockAt<T, TX, TY> &b, int zb, int ze)
+{
+    constexpr int NT = TX * TY, NU = Blk<TX, TY>::NU;
+    constexpr int RG = march_ring<TX, TY, 9>();
+    const Lat &L = b.L;
+    T cr[kOff];
+    const __amdgpu_buffer_rsrc_t rc = brsrc(b.rows(2));
+#pragma unroll
+    for (int o = 0; o < kOff; ++o) cr[o] = bload_so<T>(rc, b.voff, o * kWave * (int)sizeof(T));
+    BlkAddr<T, 1> a;
+    a.lin = b.voff;
+    a.col = L.S * (int)sizeof(T);
+    a.row = L.nx * L.S * (int)sizeof(T);
+    a.bx = b.bx; a.by = b.by; a.nx = L.nx; a.ny = L.ny;
+    // the descriptor's base (bx - 2, by - 2) may lie before the array for an
+    // edge block; every address it serves is inside (offsets are >= 0)
+    const T *base = b.gw + ((ptrdiff_t)(b.bx - 2) + (ptrdiff_t)L.nx * (b.by - 2)) * L.S +
+                    (size_t)(zb - 2) * b.plane * L.S;
+    const int pb = (int)(b.plane * L.S * sizeof(T));
+    T acc[5][NT];
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[k][t] = T(0);
+    T v[RG];
+    a.r = brsrc(base);
+    march_prime<T, TX, TY, CLAMP, RG>(a, v, std::make_integer_sequence<int, RG - 1>{});
+    int p = zb - 2;
+    auto plane = [&](auto lo, auto hi) __attribute__((always_inline)) {
+        a.r = brsrc(base);
+        // past the last plane the ring reads that plane again, for nothing
+        march_plane<T, TX, TY, CLAMP, RG, decltype(lo)::value, decltype(hi)::value>(
+            a, p < ze + 2 ? pb : 0, cr, v, acc, std::make_integer_sequence<int, NU>{});
+        base += b.plane * L.S;
+        if (p - 2 >= zb)
+        {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) b.store(t, p - 2, acc[0][t]);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[k][t] = acc[k + 1][t];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[4][t] = T(0);
+        ++p;
+    };
+    using i0 = std::integral_constant<int, 0>;
+    using i1 = std::integral_constant<int, 1>;
+    using i2 = std::integral_constant<int, 2>;
+    using i3 = std::integral_constant<int, 3>;
+    using i4 = std::integral_constant<int, 4>;
+    if (ze - zb < 3)
+    {
+        while (p <= ze + 2) plane(i0{}, i4{});
+        return;
+    }
+    plane(i4{}, i4{}); plane(i3{}, i4{}); plane(i2{}, i4{}); plane(i1{}, i4{});
+    while (p <= ze - 2) plane(i0{}, i4{});
+    plane(i0{}, i3{}); plane(i0{}, i2{}); plane(i0{}, i1{}); plane(i0{}, i0{});
+}
+
+// The marched transport in one launch. Per chunk: the end planes (0, 1, nz-2,
+// nz-1, classes of their own) column by column; the blocks along the lattice
+// edges, whose columns share a class along the edge (1 x 4 along the x edges, 4 x
+// 1 along the y edges; where the interior is narrower than four, one column
+// each); the corner columns; the interior blocks. Every block's planes are cut
+// into nslab items of at least four planes, so that the launch has waves enough;
+// a cut costs four planes' loads.
+struct MarchItems
+{
+    int nedge, ncorner, nblk, nslab;                   // blocks of each kind, items per block
+    __host__ __device__ int per_chunk(int nx, int ny) const
+    {
+        return nx * ny + (nedge + ncorner + nblk) * nslab;
+    }
+};
+
+template <typename T, int TX, int TY>
+MarchItems march_items(const Lat &L, int nslab)
+{
+    MarchItems m;
+    m.nedge = edge_blocks(L.nx, L.ny) ? 4 * (blocks(L.nx, 4) + blocks(L.ny, 4)) : 0;
+    m.ncorner = edge_blocks(L.nx, L.ny) ? 16 : L.nx * L.ny - (L.nx - 4) * (L.ny - 4);
+    m.nblk = blocks(L.nx, TX) * blocks(L.ny, TY);
+    m.nslab = std::max(1, std::min(nslab, (L.nz - 4) / 4));
+    return m;
+}
+
+template <typename T, int TX, int TY>
+__global__ __launch_bounds__(256, 2)
+void k_apply_march(Lat L, const T *__restrict__ g, T *__restrict__ gt, const T *__restrict__ coef,
+                   MarchItems m)
+{
+    const int per = m.per_chunk(L.nx, L.ny);
+    const int b = xcd_remap(blockIdx.x, gridDim.x);
+    const int wv = __builtin_amdgcn_readfirstlane(b * (int)(blockDim.x / kWave) + (int)threadIdx.x / kWave);
+    const int voff = (threadIdx.x & (kWave - 1)) * (int)sizeof(T);
+    if (wv >= per * L.nchunk) return;
+    const int chunk = wv / per;                             // chunk-major
+    int e = wv % per;
+    const int ncol = L.nx * L.ny;
+    if (e < ncol)
+    {
+        column_ends<T>(L, g, gt, coef, chunk, e % L.nx, e / L.nx, voff);
+        return;
+    }
+    e -= ncol;
+    // item k of a block
+    auto run = [&](auto tx, auto ty, auto clamp, int k, int x0, int y0, int cx, int cy) {
+        constexpr int BX = decltype(tx)::value, BY = decltype(ty)::value;
+        const BlockAt<T, BX, BY> at(L, g, gt, coef, chunk, x0, y0, cx, cy, voff);
+        const int nzi = L.nz - 4;
+        block_march<T, BX, BY, decltype(clamp)::value>(at, 2 + nzi * k / m.nslab,
+                                                       1 + nzi * (k + 1) / m.nslab);
+    };
+    using std::integral_constant;
+    using one = integral_constant<int, 1>;
+    using four = integral_constant<int, 4>;
+    const int pb = m.nslab;
+    if (e < m.nedge * pb)
+    {
+        const int eb = e / pb, k = e % pb, qy = blocks(L.ny, 4), qx = blocks(L.nx, 4);
+        if (eb < 4 * qy)                                    // x edges: 1 x 4 along y
+        {
+            const int side = eb / qy, ix = side < 2 ? side : L.nx - 4 + side;
+            run(one{}, four{}, std::true_type{}, k, ix, 2 + 4 * (eb % qy), category(ix, L.nx), 2);
+            return;
+        }
+        const int f = eb - 4 * qy;                          // y edges: 4 x 1 along x
+        const int side = f / qx, iy = side < 2 ? side : L.ny - 4 + side;
+        run(four{}, one{}, std::true_type{}, k, 2 + 4 * (f % qx), iy, 2, category(iy, L.ny));
+        return;
+    }
+    e -= m.nedge * pb;
+    if (e < m.ncorner * pb)
+    {
+        const int cb = e / pb, k = e % pb;
+        int ix, iy;
+        if (m.nedge)
+        {
+            const int a = cb & 3, c = cb >> 2;
+            ix = a < 2 ? a : L.nx - 4 + a;
+            iy = c < 2 ? c : L.ny - 4 + c;
+        }
+        else column_of(L, cb, true, ix, iy);
+        run(one{}, one{}, std::true_type{}, k, ix, iy, category(ix, L.nx), category(iy, L.ny));
+        return;
+    }
+    e -= m.ncorner * pb;
+    // interior blocks item by item within a slab: the blocks in flight are
+    // neighbours
+    const int k = e / m.nblk, blk = e % m.nblk, nbx = blocks(L.nx, TX);
+    run(integral_constant<int, TX>{}, integral_constant<int, TY>{}, std::false_type{}, k,
+        2 + (blk % nbx) * TX, 2 + (blk / nbx) * TY, 2, 2);
 }
 
 // ---- per-particle limiters, wall, moments, collision -------------------------
@@ -1843,13 +2128,15 @@ bool is_fp32(const ab_ctx *ctx) { return ctx->cfg.precision == AB_PREC_MIXED; }
 // K outputs per z block (values reused across K + 4 planes), W the waves per
 // SIMD the register allocation targets. Every shape does the same products
 // in the same order per output, so the results do not depend on the choice.
-// TX x TY > 1: interior blocks + edge columns; S > 0: the slab order, items of S z blocks
+// TX x TY > 1: interior blocks + edge columns. FP32, S > 0: the slab order, items
+// of S z blocks. FP64: marched through z, S items per block (these sum an output's
+// terms plane by plane).
 struct ApplyShape { int K, W, TX, TY, S; };
 constexpr ApplyShape kShapes32[] = {{12, 3, 1, 1, 0}, {9, 3, 1, 1, 0}, {12, 2, 2, 2, 0},
                                     {12, 2, 2, 2, 1}, {8, 2, 2, 3, 1}, {6, 2, 2, 4, 1},
                                     {6, 2, 2, 4, 2}};
-constexpr ApplyShape kShapes64[] = {{9, 2, 1, 1, 0}, {8, 2, 1, 1, 0}, {7, 2, 1, 1, 0},
-                                    {6, 2, 1, 1, 0}};
+constexpr ApplyShape kShapes64[] = {{9, 2, 1, 1, 0}, {7, 2, 1, 1, 0}, {0, 2, 2, 2, 1},
+                                    {0, 2, 2, 2, 2}};
 constexpr int kMaxBlockPlanes = kMaxZBlockPlanes;
 
 template <typename T>
@@ -1890,14 +2177,14 @@ void launch_shape(int i, Lat L, const T *g, T *gt, const T *cf, const double *sc
     }
     else
     {
-        const int nb = waves(all);
-        switch (i)
+        const ApplyShape sh = kShapes64[i];
+        if (sh.TX > 1)
         {
-        case 0: k_apply<T, 9, 2><<<nb, 256, 0, s>>>(L, g, gt, cf, scal); break;
-        case 1: k_apply<T, 8, 2><<<nb, 256, 0, s>>>(L, g, gt, cf, scal); break;
-        case 2: k_apply<T, 7, 2><<<nb, 256, 0, s>>>(L, g, gt, cf, scal); break;
-        default: k_apply<T, 6, 2><<<nb, 256, 0, s>>>(L, g, gt, cf, scal); break;
+            const MarchItems m = march_items<T, 2, 2>(L, sh.S);
+            k_apply_march<T, 2, 2><<<waves(m.per_chunk(L.nx, L.ny)), 256, 0, s>>>(L, g, gt, cf, m);
         }
+        else if (i == 1) k_apply<T, 7, 2><<<waves(all), 256, 0, s>>>(L, g, gt, cf, scal);
+        else k_apply<T, 9, 2><<<waves(all), 256, 0, s>>>(L, g, gt, cf, scal);
     }
 }
 
@@ -1916,14 +2203,14 @@ bool shape_fits(int i, int nx, int ny)
 // Single columns in z blocks of 9 where the launch has fewer of them than the
 // chip has SIMDs: every wave then runs alone and the shorter one ends first
 // (18.2 / 22.2 us at 13^3 / Nv 7, 16.4 / 19.4 at 11^3 / Nv 6), and where no block
-// fits. FP64: the single-column z block that divides the interior run.
+// fits. FP64: the marched 2 x 2 blocks by the same rule (29 / 37 us at 13^3 / Nv 7,
+// 51 / 46 at 10^3 / Nv 10).
 template <typename T>
 int default_shape(const Lat &L)
 {
     if (sizeof(T) == 4)
         return L.nx * L.ny * L.nchunk < 1024 || !shape_fits<T>(5, L.nx, L.ny) ? 1 : 5;
-    const int run = L.nz - 4;
-    return run % 9 == 0 ? 0 : (run % 7 == 0 ? 2 : 1);
+    return shape_fits<T>(2, L.nx, L.ny) && L.nx * L.ny * L.nchunk >= 1024 ? 2 : 0;
 }
 
 template <typename T>
@@ -2145,16 +2432,17 @@ int table_setup(ab_ctx *ctx)
 static int table_build(ab_ctx *ctx, double dt)
 {
     const double tol = ctx->cfg.mls_tol > 0 ? ctx->cfg.mls_tol : 1e-12;
-    dim3 grid((ctx->S + 255) / 256, kNcls);
+    const int nchunk = (ctx->nodes + kWave - 1) / kWave;
+    dim3 grid((nchunk * kWave + 255) / 256, kNcls);
     ab::DevCloud c = ctx->view();
     if (is_fp32(ctx))
         k_build<float><<<grid, 256, 0, ctx->stream>>>(c, ctx->cls, ctx->lat, dt, ctx->cfg.radius,
                                                       tol, ctx->cfg.mls_order, (float *)ctx->coef,
-                                                      ctx->S);
+                                                      nchunk);
     else
         k_build<double><<<grid, 256, 0, ctx->stream>>>(c, ctx->cls, ctx->lat, dt,
                                                        ctx->cfg.radius, tol, ctx->cfg.mls_order,
-                                                       (double *)ctx->coef, ctx->S);
+                                                       (double *)ctx->coef, nchunk);
     return hipGetLastError() == hipSuccess ? AB_OK : AB_ERR_HIP;
 }
 
@@ -2217,7 +2505,7 @@ int table_step(ab_ctx *ctx, double dt)
         int rc = table_prepare(ctx, dt);
         if (rc) return rc;
     }
-    Lat L{ctx->cfg.nx, ctx->cfg.ny, ctx->cfg.nz, ctx->S, ctx->S / kWave};
+    Lat L{ctx->cfg.nx, ctx->cfg.ny, ctx->cfg.nz, ctx->S, (ctx->nodes + kWave - 1) / kWave};
     ab::DevCloud c = ctx->view();
     hipStream_t s = ctx->stream;
     auto tic = [&]() { prof_begin(ctx); };
@@ -2288,7 +2576,7 @@ int table_autotune(ab_ctx *ctx, double dt, int reps, int cap, char (*names)[32],
         int rc = table_prepare(ctx, dt);
         if (rc) return rc;
     }
-    Lat L{ctx->cfg.nx, ctx->cfg.ny, ctx->cfg.nz, ctx->S, ctx->S / kWave};
+    Lat L{ctx->cfg.nx, ctx->cfg.ny, ctx->cfg.nz, ctx->S, (ctx->nodes + kWave - 1) / kWave};
     const bool f32 = is_fp32(ctx);
     const int ns = f32 ? nshapes<float>() : nshapes<double>();
     hipEvent_t e0, e1;
@@ -2322,7 +2610,8 @@ int table_autotune(ab_ctx *ctx, double dt, int reps, int cap, char (*names)[32],
         if (names && i < cap)
         {
             const ApplyShape sh = f32 ? shape_at<float>(i) : shape_at<double>(i);
-            if (sh.TX > 1)
+            if (sh.TX > 1 && !f32) snprintf(names[i], 32, "B%dx%d/M%d", sh.TX, sh.TY, sh.S);
+            else if (sh.TX > 1)
                 snprintf(names[i], 32, "B%dx%d/K%d%s", sh.TX, sh.TY, sh.K,
                          sh.S == 2 ? "/S2" : (sh.S ? "/S" : ""));
             else snprintf(names[i], 32, "K%d/W%d", sh.K, sh.W);
