@@ -53,7 +53,7 @@ void free_cloud(ab_ctx *c)
     void *ptrs[] = {c->x, c->y, c->z, c->bnd, c->wnx, c->wny, c->wnz, c->wux, c->wuy, c->wuz,
                     c->wt, c->mvx, c->mvy, c->mvz, c->rho, c->ux, c->uy, c->uz, c->T,
                     c->neigh, c->nneigh, c->ilist, c->blist, c->g, c->gt, c->limflag,
-                    c->mlsflag, c->mlsovr, c->pmass, c->pnew, c->prho, c->vox, c->vcount, c->vstart, c->vlist,
+                    c->mlsflag, c->mlsovr, c->pmass, c->pnew, c->prho, c->pcol, c->vox, c->vcount, c->vstart, c->vlist,
                     c->bmom, c->bidx, c->bwu, c->bbody, c->bcnt, c->bcon, c->bpar, c->bout,
                     c->bid, c->dm_alpha, c->dm_pass, c->dm_res, c->dm_rec,
                     c->mood, c->moodfail, c->inst, c->ih, c->seg};
@@ -67,7 +67,7 @@ void free_cloud(ab_ctx *c)
     c->mvx = c->mvy = c->mvz = nullptr;
     c->rho = c->ux = c->uy = c->uz = c->T = nullptr;
     c->neigh = c->nneigh = c->ilist = c->blist = nullptr;
-    c->g = c->gt = c->limflag = c->mlsovr = c->pmass = c->pnew = c->prho = nullptr;
+    c->g = c->gt = c->limflag = c->mlsovr = c->pmass = c->pnew = c->prho = c->pcol = nullptr;
     c->mlsflag = nullptr;
     c->vox = c->vcount = c->vstart = c->vlist = nullptr;
     c->bmom = c->bcon = c->bwu = c->bpar = c->bout = nullptr;
@@ -86,7 +86,7 @@ int alloc_cloud(ab_ctx *c)
     int rc = 0;
     double **dd[] = {&c->x, &c->y, &c->z, &c->wnx, &c->wny, &c->wnz, &c->wux, &c->wuy, &c->wuz,
                      &c->wt, &c->mvx, &c->mvy, &c->mvz, &c->rho, &c->ux, &c->uy, &c->uz, &c->T,
-                     &c->limflag, &c->mlsovr, &c->pmass, &c->pnew, &c->prho};
+                     &c->limflag, &c->mlsovr, &c->pmass, &c->pnew, &c->prho, &c->pcol};
     for (double **p : dd) if ((rc = dalloc(c, p, N))) return rc;
     if ((rc = dalloc(c, &c->bnd, N))) return rc;
     if ((rc = dalloc(c, &c->neigh, N * AB_MAX_NEIGH))) return rc;
@@ -184,11 +184,8 @@ int fp64_transport(ab_ctx *c, double dt, bool diag)
     diag = diag || c->cfg.mls_clamp;
     if (c->dim == 3) return stencil_transport(c, dt, tol, diag);
     launch_transport_fp64(v, c->g, c->gt, dt, c->cfg.radius, c->cfg.mls_order, tol,
-                          c->cfg.mls_clamp, c->mlsflag, c->mlsovr, c->ilist, c->n_int, false,
-                          diag, c->stream);
-    launch_transport_fp64(v, c->g, c->gt, dt, c->cfg.radius, c->cfg.mls_order, tol,
-                          c->cfg.mls_clamp, c->mlsflag, c->mlsovr, c->blist, c->n_bnd, true,
-                          diag, c->stream);
+                          c->cfg.mls_clamp, c->mlsflag, c->mlsovr, c->ilist, c->n_int, c->blist,
+                          c->n_bnd, diag, c->stream);
     return hipGetLastError() == hipSuccess ? AB_OK : AB_ERR_HIP;
 }
 
@@ -198,31 +195,32 @@ int fp64_step(ab_ctx *c, double dt, bool diag)
     hipStream_t s = c->stream;
     Timer tm(c);
     int rc;
+    // positivity, NAD, commit, wall and collision in one pass, both rescales in
+    // the end-of-step one and all mass sums in one reduction; the discrete
+    // collision keeps its separate passes
+    const bool fused = c->cfg.collision == AB_COLLISION_CONTINUOUS;
+    double *rho_wall = c->dim == 3 ? c->prho : c->rho;
     tm.tic();
     if (!c->mass_valid) launch_mass_partials(v, c->g, c->pmass, s);
-    launch_reduce_mass(c->N, c->pmass, c->scal, R_MASS_OLD, 0, s, c->seg, c->nbatch);
+    if (!fused) launch_reduce_mass(c->N, c->pmass, c->scal, R_MASS_OLD, 0, s, c->seg, c->nbatch);
     if (diag && (rc = zero_step_flags(c))) return rc;   // else nothing reads them
     tm.toc(ST_REDUCE);
     tm.tic();
     if ((rc = fp64_transport(c, dt, diag))) return rc;
     tm.toc(ST_TRANSPORT);
-    // positivity, NAD, commit, wall and collision in one pass, both rescales in
-    // the end-of-step one; the discrete collision keeps its separate passes
-    const bool fused = c->cfg.collision == AB_COLLISION_CONTINUOUS;
-    double *rho_wall = c->dim == 3 ? c->prho : c->rho;
     if (fused)
     {
         tm.tic();
         if (c->dim == 3)
             launch_commit_collide3(v, c->g, c->gt, dt, c->cfg.tau, c->cfg.R, c->rho, rho_wall, c->ux,
-                                   c->uy, c->uz, c->T, c->limflag, c->pnew, c->pmass, s);
+                                   c->uy, c->uz, c->T, c->limflag, c->pnew, c->pcol, s);
         else
             launch_commit_collide2(v, c->g, c->gt, dt, c->cfg.tau, c->cfg.R, c->rho, c->ux, c->uy,
-                                   c->T, c->limflag, c->pnew, c->pmass, s);
+                                   c->T, c->limflag, c->pnew, c->pcol, s);
         tm.toc(ST_WALL_COLLIDE);
         tm.tic();
-        launch_reduce_mass(c->N, c->pmass, c->scal, R_MASS_FUSED, c->cfg.no_mass_fix, s, c->seg,
-                           c->nbatch, c->pnew);
+        launch_reduce_mass(c->N, c->pcol, c->scal, R_MASS_FUSED, c->cfg.no_mass_fix, s, c->seg,
+                           c->nbatch, c->pnew, c->pmass);
         tm.toc(ST_REDUCE);
     }
     else
@@ -276,7 +274,7 @@ int fp64_step_mood(ab_ctx *c, double dt, bool diag)
     launch_mood_check(v, c->gt, c->rho, c->mood, c->limflag, s);
     const double tol = c->cfg.mls_tol > 0 ? c->cfg.mls_tol : 1e-12;
     launch_transport_fp64(v, c->g, c->gt, dt, c->cfg.radius, 1, tol, c->cfg.mls_clamp,
-                          c->mlsflag, c->mlsovr, c->ilist, c->n_int, false,
+                          c->mlsflag, c->mlsovr, c->ilist, c->n_int, nullptr, 0,
                           diag || c->cfg.mls_clamp, s, c->mood);
     launch_mood_commit(v, c->g, c->gt, c->mood, c->limflag, c->pmass, s);
     tm.toc(ST_LIMIT_COMMIT);
@@ -404,12 +402,12 @@ int relayout_cloud(ab_ctx *c, const int *src, int n)
     constexpr int nc = sizeof(carried) / sizeof(carried[0]);
     double *od[nc];
     for (int k = 0; k < nc; ++k) { od[k] = *carried[k]; *carried[k] = nullptr; }
-    double *og = c->g, *ogt = c->gt, *olim = c->limflag, *oovr = c->mlsovr, *opm = c->pmass, *opn = c->pnew, *opr = c->prho;
+    double *og = c->g, *ogt = c->gt, *olim = c->limflag, *oovr = c->mlsovr, *opm = c->pmass, *opn = c->pnew, *opr = c->prho, *opc = c->pcol;
     double *oalpha = c->dm_alpha, *ores = c->dm_res;
     int *opass = c->dm_pass, *omls = c->mlsflag, *omood = c->mood, *omf = c->moodfail;
     int *onb = c->neigh, *onn = c->nneigh, *oil = c->ilist, *obl = c->blist, *obid = c->bid;
     unsigned char *obnd = c->bnd;
-    c->g = c->gt = c->limflag = c->mlsovr = c->pmass = c->pnew = c->prho = nullptr;
+    c->g = c->gt = c->limflag = c->mlsovr = c->pmass = c->pnew = c->prho = c->pcol = nullptr;
     c->dm_alpha = c->dm_res = nullptr;
     c->dm_pass = c->mlsflag = c->mood = c->moodfail = nullptr;
     c->neigh = c->nneigh = c->ilist = c->blist = c->bid = nullptr;
@@ -447,7 +445,7 @@ int relayout_cloud(ab_ctx *c, const int *src, int n)
         if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
         { c->err = "cloud re-layout: gather failed"; rc = AB_ERR_HIP; }
     }
-    void *old[] = {og, ogt, olim, oovr, opm, opn, opr, oalpha, ores, opass, omls, omood, omf,
+    void *old[] = {og, ogt, olim, oovr, opm, opn, opr, opc, oalpha, ores, opass, omls, omood, omf,
                    onb, onn, oil, obl, obnd, obid, c->vox, c->vlist, c->dm_rec};
     for (void *p : old) if (p) (void)hipFree(p);
     for (int k = 0; k < nc; ++k) if (od[k]) (void)hipFree(od[k]);

@@ -62,9 +62,9 @@ enum ScalarSlot
     S_COUNT = 8
 };
 
-// R_MASS_FUSED: the committed masses (second array) and the collided
-// masses of the unscaled rows (first array) of the 2-D table step's fused
-// commit and collision, giving both scales at once.
+// R_MASS_FUSED: the collided masses of the unscaled rows (first array), the
+// committed masses (second) and the step's starting masses (third) of the fused
+// commit and collision, giving all scales at once.
 enum ReduceMode { R_MASS_OLD = 0, R_MASS_NEW = 1, R_MASS_COLL = 2, R_MASS_FUSED = 3 };
 
 // Stages timed by ab_profile, in report order.
@@ -113,6 +113,7 @@ struct ab_ctx
     double *pmass = nullptr;       // per-particle partial sums
     double *pnew = nullptr;        // committed mass per particle of the fused commit and collision
     double *prho = nullptr;        // its wall densities (3-D)
+    double *pcol = nullptr;        // its collided masses
     double *scal = nullptr;        // ab::ScalarSlot
     bool mass_valid = false;       // pmass holds the current g's masses
     // Bumped whenever the device arrays are freed, re-allocated or refilled
@@ -256,12 +257,14 @@ void prof_end(ab_ctx *c, int stage);
 void prof_flush(ab_ctx *c);
 
 // ---- k_mls.hip -------------------------------------------------------------
-// diag: the flags and overshoots of the step statistics (and the clamp).
+// The interior particles il and the boundary particles bl. diag: the flags and
+// overshoots of the step statistics (and the clamp). only (may be null): the
+// interior particles to act on. dev (may be null): the lists' lengths on the
+// device.
 void launch_transport_fp64(const DevCloud &c, const double *g, double *gt, double dt,
                            double h, int order, double tol, int clamp, int *mlsflag,
-                           double *mlsovr, const int *list, int nlist, bool boundary, bool diag,
-                           hipStream_t s, const int *only = nullptr,
-                           const int *nlist_dev = nullptr);
+                           double *mlsovr, const int *il, int ni, const int *bl, int nb, bool diag,
+                           hipStream_t s, const int *only = nullptr, const int *dev = nullptr);
 
 // ---- k_stencil.hip ---------------------------------------------------------
 // The 3-D transport with the normal equations shared by congruent stencils.
@@ -286,7 +289,7 @@ void launch_mass_partials(const DevCloud &c, const double *g, double *pmass, hip
 // seg[0..nseg], scalars S_COUNT apart); else one over all N.
 void launch_reduce_mass(int N, const double *pmass, double *scal, int mode, int nofix,
                         hipStream_t s, const int *seg = nullptr, int nseg = 1,
-                        const double *pnew = nullptr);
+                        const double *pnew = nullptr, const double *pold = nullptr);
 void launch_limit_commit(const DevCloud &c, double *g, const double *gt, const double *rho,
                          double *limflag, double *pmass, hipStream_t s);
 // guard (may be null): when given, the launch acts only if *guard is set,

@@ -41,9 +41,10 @@ __global__ __launch_bounds__(kBlock) void k_mass_partials(DevCloud c, const doub
 __global__ __launch_bounds__(1024) void k_reduce_mass(int N, const double *__restrict__ pmass,
                                                       double *scal, int mode, int nofix,
                                                       const int *__restrict__ seg,
-                                                      const double *__restrict__ pnew)
+                                                      const double *__restrict__ pnew,
+                                                      const double *__restrict__ pold)
 {
-    __shared__ double sh[1024 / kWave], shn[1024 / kWave];
+    __shared__ double sh[1024 / kWave], shn[1024 / kWave], sho[1024 / kWave];
     int lo = 0, hi = N;
     if (seg)
     {
@@ -53,45 +54,47 @@ __global__ __launch_bounds__(1024) void k_reduce_mass(int N, const double *__res
     }
     // eight loads in flight per thread while eight are left: the one workgroup
     // is bound by their latency (64,000 particles: 29 -> 21 us)
-    constexpr int U = 8;
-    double s = 0.0, sn = 0.0;
-    int i = lo + (int)threadIdx.x;
-    for (; i + (U - 1) * 1024 < hi; i += U * 1024)
-    {
-        double v[U];
+    auto total = [&](const double *__restrict__ p) {
+        constexpr int U = 8;
+        double t = 0.0;
+        int i = lo + (int)threadIdx.x;
+        for (; i + (U - 1) * 1024 < hi; i += U * 1024)
+        {
+            double v[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = pmass[i + u * 1024];
+            for (int u = 0; u < U; ++u) v[u] = p[i + u * 1024];
 #pragma unroll
-        for (int u = 0; u < U; ++u) s += v[u];
-        if (!pnew) continue;
-#pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = pnew[i + u * 1024];
-#pragma unroll
-        for (int u = 0; u < U; ++u) sn += v[u];
-    }
-    for (; i < hi; i += 1024)
-    {
-        s += pmass[i];
-        if (pnew) sn += pnew[i];
-    }
+            for (int u = 0; u < U; ++u) t += v[u];
+        }
+        for (; i < hi; i += 1024) t += p[i];
+        return t;
+    };
+    double s = total(pmass), sn = pnew ? total(pnew) : 0.0, so = pold ? total(pold) : 0.0;
     s = wave_sum(s);
     sn = wave_sum(sn);
-    if ((threadIdx.x & (kWave - 1)) == 0) { sh[threadIdx.x / kWave] = s; shn[threadIdx.x / kWave] = sn; }
+    so = wave_sum(so);
+    if ((threadIdx.x & (kWave - 1)) == 0)
+    {
+        sh[threadIdx.x / kWave] = s;
+        shn[threadIdx.x / kWave] = sn;
+        sho[threadIdx.x / kWave] = so;
+    }
     __syncthreads();
     if (threadIdx.x == 0)
     {
-        double t = 0.0, tn = 0.0;
-        for (int q = 0; q < 1024 / kWave; ++q) { t += sh[q]; tn += shn[q]; }
+        double t = 0.0, tn = 0.0, to = 0.0;
+        for (int q = 0; q < 1024 / kWave; ++q) { t += sh[q]; tn += shn[q]; to += sho[q]; }
         if (mode == R_MASS_FUSED)
         {
             // massOld / massNew, the collided mass after that rescale, and the
             // one end-of-step factor that the unscaled collided rows need:
             // massOld / massColl * massOld / massNew = massOld / t
-            const double s1 = (tn > 1e-30) ? scal[S_MASS_OLD] / tn : 1.0;
+            const double s1 = (tn > 1e-30) ? to / tn : 1.0;
+            scal[S_MASS_OLD] = to;
             scal[S_MASS_NEW] = tn;
             scal[S_SCALE1] = s1;
             scal[S_MASS_COLL] = s1 * t;
-            scal[S_SCALE2] = (!nofix && s1 * t > 1e-30) ? scal[S_MASS_OLD] / t : s1;
+            scal[S_SCALE2] = (!nofix && s1 * t > 1e-30) ? to / t : s1;
         }
         else if (mode == R_MASS_OLD)
             scal[S_MASS_OLD] = t;
@@ -1074,9 +1077,10 @@ void launch_mass_partials(const DevCloud &c, const double *g, double *pmass, hip
 }
 
 void launch_reduce_mass(int N, const double *pmass, double *scal, int mode, int nofix,
-                        hipStream_t s, const int *seg, int nseg, const double *pnew)
+                        hipStream_t s, const int *seg, int nseg, const double *pnew,
+                        const double *pold)
 {
-    k_reduce_mass<<<seg ? nseg : 1, 1024, 0, s>>>(N, pmass, scal, mode, nofix, seg, pnew);
+    k_reduce_mass<<<seg ? nseg : 1, 1024, 0, s>>>(N, pmass, scal, mode, nofix, seg, pnew, pold);
 }
 
 void launch_limit_commit(const DevCloud &c, double *g, const double *gt, const double *rho,

@@ -154,27 +154,39 @@ __device__ __forceinline__ void transport3d_item(const DevCloud &c, const double
     }
 }
 
-// nlist_dev: the list's length on the device (the stencil classification
-// leaves what it cannot share there), else nlist. The workgroups stride over
-// the (particle, 256 nodes) items, so the grid needs no host count.
-template <int P, bool BND, bool DIAG>
+// The interior particles il (P basis functions), then the boundary particles bl
+// (linear basis), in one launch. dev: the lists' lengths on the device (the
+// stencil classification leaves what it cannot share there), else ni and nb.
+// The workgroups stride over the (particle, 256 nodes) items, so the grid needs
+// no host count.
+template <int P, bool DIAG>
 __global__ __launch_bounds__(kBlock) void k_transport3d(DevCloud c, const double *__restrict__ g,
                                                         double *__restrict__ gt, double dt,
                                                         double h, double tol, int clamp,
                                                         int *mlsflag, double *mlsovr,
-                                                        const int *__restrict__ list, int nlist,
-                                                        const int *__restrict__ nlist_dev,
+                                                        const int *__restrict__ il, int ni,
+                                                        const int *__restrict__ bl, int nb,
+                                                        const int *__restrict__ dev,
                                                         int nchunk, const int *__restrict__ only)
 {
     __shared__ double se[AB_MAX_NEIGH][4];
     __shared__ int sj[AB_MAX_NEIGH];
-    const int nitem = (nlist_dev ? *nlist_dev : nlist) * nchunk;
-    for (int item = xcd_remap(blockIdx.x, gridDim.x); item < nitem; item += gridDim.x)
+    const int nint = (dev ? dev[0] : ni) * nchunk, nall = nint + (dev ? dev[1] : nb) * nchunk;
+    for (int item = xcd_remap(blockIdx.x, gridDim.x); item < nall; item += gridDim.x)
     {
-        const int i = list[item / nchunk];
-        if (only && !only[i]) continue;      // whole block: one particle
-        transport3d_item<P, BND, DIAG>(c, g, gt, dt, h, tol, clamp, mlsflag, mlsovr, i,
-                                       item % nchunk, se, sj);
+        if (item < nint)
+        {
+            const int i = il[item / nchunk];
+            if (only && !only[i]) continue;      // whole block: one particle
+            transport3d_item<P, false, DIAG>(c, g, gt, dt, h, tol, clamp, mlsflag, mlsovr, i,
+                                             item % nchunk, se, sj);
+        }
+        else
+        {
+            const int e = item - nint;
+            transport3d_item<4, true, DIAG>(c, g, gt, dt, h, tol, clamp, mlsflag, mlsovr,
+                                            bl[e / nchunk], e % nchunk, se, sj);
+        }
     }
 }
 
@@ -239,7 +251,7 @@ __device__ __forceinline__ void solve_pivoted(double (&A)[P * P], double (&r1)[P
     o2 = s2[0];
 }
 
-// kCopyGt + kTransportNode, 2-D Chu layers (Solver/CudaBackend.cu:199-300).
+// One item (particle i, 256 nodes) of kCopyGt + kTransportNode, 2-D Chu layers (Solver/CudaBackend.cu:199-300).
 // The reference solves by Gauss elimination with partial pivoting. A is
 // symmetric positive definite, so elimination without pivoting is as stable
 // and gives the same solution to rounding; where a pivot falls below 1e-9 of
@@ -247,17 +259,12 @@ __device__ __forceinline__ void solve_pivoted(double (&A)[P * P], double (&r1)[P
 // the pivoted elimination runs instead, so what it does with a singular
 // matrix stays what it was.
 template <int P, bool BND>
-__global__ __launch_bounds__(kBlock) void k_transport2d(DevCloud c, const double *__restrict__ g,
-                                                        double *__restrict__ gt, double dt,
-                                                        double h, const int *__restrict__ list,
-                                                        int nchunk, const int *__restrict__ only)
+__device__ __forceinline__ void transport2d_item(const DevCloud &c, const double *__restrict__ g,
+                                                 double *__restrict__ gt, double dt, double h,
+                                                 int i, int chunk, double (&se)[AB_MAX_NEIGH][2],
+                                                 int (&sj)[AB_MAX_NEIGH])
 {
-    __shared__ double se[AB_MAX_NEIGH][2];
-    __shared__ int sj[AB_MAX_NEIGH];
-    const int b = xcd_remap(blockIdx.x, gridDim.x);
-    const int i = list[b / nchunk];
-    if (only && !only[i]) return;            // whole block: one particle
-    const int lin = (b % nchunk) * kBlock + threadIdx.x;
+    const int lin = chunk * kBlock + threadIdx.x;
     const int nn = c.nneigh[i];
     if (c.inst) h = c.ih[c.inst[i]];
     const double ih = 1.0 / h;
@@ -373,38 +380,54 @@ __global__ __launch_bounds__(kBlock) void k_transport2d(DevCloud c, const double
     gt[(size_t)i * gs + lin + Nv2] = o2;
 }
 
+// The interior particles il (P basis functions), then the boundary particles bl
+// (linear basis), in one launch: on a small cloud the boundary's own launch
+// would cost as much again as its work.
+template <int P>
+__global__ __launch_bounds__(kBlock) void k_transport2d(DevCloud c, const double *__restrict__ g,
+                                                        double *__restrict__ gt, double dt,
+                                                        double h, const int *__restrict__ il,
+                                                        int ni, const int *__restrict__ bl,
+                                                        int nchunk, const int *__restrict__ only)
+{
+    __shared__ double se[AB_MAX_NEIGH][2];
+    __shared__ int sj[AB_MAX_NEIGH];
+    const int b = xcd_remap(blockIdx.x, gridDim.x), p = b / nchunk, chunk = b % nchunk;
+    if (p < ni)
+    {
+        const int i = il[p];
+        if (only && !only[i]) return;            // whole block: one particle
+        transport2d_item<P, false>(c, g, gt, dt, h, i, chunk, se, sj);
+    }
+    else transport2d_item<3, true>(c, g, gt, dt, h, bl[p - ni], chunk, se, sj);
+}
+
 }  // namespace
 
 void launch_transport_fp64(const DevCloud &c, const double *g, double *gt, double dt, double h,
                            int order, double tol, int clamp, int *mlsflag, double *mlsovr,
-                           const int *list, int nlist, bool boundary, bool diag, hipStream_t s,
-                           const int *only, const int *nlist_dev)
+                           const int *il, int ni, const int *bl, int nb, bool diag, hipStream_t s,
+                           const int *only, const int *dev)
 {
-    if (nlist <= 0) return;
+    if (ni + nb <= 0) return;
     const int nchunk = (c.nodes + kBlock - 1) / kBlock;
-    const int nb = nlist * nchunk;
+    const int all = (ni + nb) * nchunk;
     if (c.dim == 3)
     {
-        // with a count on the device the grid is what fills the chip, not the
-        // list's upper bound: most of it would find nothing to do
-        const int grid = nlist_dev ? std::min(nb, kFillBlocks) : nb;
+        // with the counts on the device the grid is what fills the chip, not
+        // the lists' upper bounds: most of it would find nothing to do
+        const int grid = dev ? std::min(all, kFillBlocks) : all;
         auto go = [&](auto kernel) {
-            kernel<<<grid, kBlock, 0, s>>>(c, g, gt, dt, h, tol, clamp, mlsflag, mlsovr, list,
-                                           nlist, nlist_dev, nchunk, only);
+            kernel<<<grid, kBlock, 0, s>>>(c, g, gt, dt, h, tol, clamp, mlsflag, mlsovr, il, ni,
+                                           bl, nb, dev, nchunk, only);
         };
-        if (boundary) { if (diag) go(k_transport3d<4, true, true>); else go(k_transport3d<4, true, false>); }
-        else if (order >= 2) { if (diag) go(k_transport3d<10, false, true>); else go(k_transport3d<10, false, false>); }
-        else { if (diag) go(k_transport3d<4, false, true>); else go(k_transport3d<4, false, false>); }
+        if (order >= 2) { if (diag) go(k_transport3d<10, true>); else go(k_transport3d<10, false>); }
+        else { if (diag) go(k_transport3d<4, true>); else go(k_transport3d<4, false>); }
     }
+    else if (order >= 2)
+        k_transport2d<6><<<all, kBlock, 0, s>>>(c, g, gt, dt, h, il, ni, bl, nchunk, only);
     else
-    {
-        if (boundary)
-            k_transport2d<3, true><<<nb, kBlock, 0, s>>>(c, g, gt, dt, h, list, nchunk, only);
-        else if (order >= 2)
-            k_transport2d<6, false><<<nb, kBlock, 0, s>>>(c, g, gt, dt, h, list, nchunk, only);
-        else
-            k_transport2d<3, false><<<nb, kBlock, 0, s>>>(c, g, gt, dt, h, list, nchunk, only);
-    }
+        k_transport2d<3><<<all, kBlock, 0, s>>>(c, g, gt, dt, h, il, ni, bl, nchunk, only);
 }
 
 }  // namespace ab

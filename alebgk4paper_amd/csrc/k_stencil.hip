@@ -882,9 +882,8 @@ int stencil_transport(ab_ctx *c, double dt, double tol, bool diag)
                                                         c->st_slot, nchunk);
     }
     launch_transport_fp64(v, c->g, c->gt, dt, f.radius, f.mls_order, tol, f.mls_clamp, c->mlsflag,
-                          c->mlsovr, c->st_int, c->n_int, false, diag, s, nullptr, c->st_n + N_INT);
-    launch_transport_fp64(v, c->g, c->gt, dt, f.radius, f.mls_order, tol, f.mls_clamp, c->mlsflag,
-                          c->mlsovr, c->st_bnd, c->n_bnd, true, diag, s, nullptr, c->st_n + N_BND);
+                          c->mlsovr, c->st_int, c->n_int, c->st_bnd, c->n_bnd, diag, s, nullptr,
+                          c->st_n + N_INT);
     return hipGetLastError() == hipSuccess ? AB_OK : AB_ERR_HIP;
 }
 
