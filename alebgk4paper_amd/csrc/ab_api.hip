@@ -182,7 +182,7 @@ int fp64_transport(ab_ctx *c, double dt, bool diag)
     const double tol = c->cfg.mls_tol > 0 ? c->cfg.mls_tol : 1e-12;
     DevCloud v = c->view();
     diag = diag || c->cfg.mls_clamp;
-    if (c->dim == 3) return stencil_transport(c, dt, tol, diag);
+    if (stencil_shared(c)) return stencil_transport(c, dt, tol, diag);
     launch_transport_fp64(v, c->g, c->gt, dt, c->cfg.radius, c->cfg.mls_order, tol,
                           c->cfg.mls_clamp, c->mlsflag, c->mlsovr, c->ilist, c->n_int, c->blist,
                           c->n_bnd, diag, c->stream);
@@ -359,7 +359,7 @@ int graph_coefficients(ab_ctx *c, double dt)
         if (rc) return rc;
     }
     // likewise the stencil classes, which a captured step does not look for
-    if (c->dim == 3 && !table_mode(c) && !c->st_valid)
+    if (!table_mode(c) && stencil_shared(c) && !c->st_valid)
     {
         int rc = stencil_prepare(c);
         if (rc) return rc;

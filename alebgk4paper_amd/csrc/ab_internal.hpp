@@ -270,6 +270,8 @@ void launch_transport_fp64(const DevCloud &c, const double *g, double *gt, doubl
 // The 3-D transport with the normal equations shared by congruent stencils.
 // stencil_prepare: the classes of the current cloud (after every change of
 // positions, lists, flags, wall or mesh velocities: st_valid).
+// stencil_shared: whether this cloud is large enough for it.
+bool stencil_shared(const ab_ctx *ctx);
 int stencil_transport(ab_ctx *ctx, double dt, double tol, bool diag);
 int stencil_prepare(ab_ctx *ctx);
 void stencil_free(ab_ctx *ctx);

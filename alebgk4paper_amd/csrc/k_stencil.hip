@@ -590,6 +590,18 @@ struct Wave                                            // what the loads of an i
     size_t gs;
 };
 
+// Rows in flight: the loads of row U + D - 1 are issued before the products of
+// row U. Short pieces have registers for deeper rings, and are what a small
+// cloud's launch waits for.
+template <int YN, int R>
+constexpr int depth() { return R >= 8 && YN > 1 ? 2 : (R >= 4 ? 3 : 4); }
+
+// Where the coefficients of the stencil row at oy are kept until the last run of
+// the patch has met it: by oy (the same row of the next plane comes after
+// that), or in the ring of a single run.
+template <int YN, int R>
+constexpr int coef_at(int U, int oy) { return YN > 1 ? oy + 2 : U % depth<YN, R>(); }
+
 // Values of patch row U into v, and into cm the coefficients of the stencil row
 // that the first run meets there (the later runs meet it at later rows).
 template <int YN, int R, int U>
@@ -611,19 +623,20 @@ __device__ __forceinline__ void patch_load(const Wave &w, const int (&first)[YN]
         constexpr Row k = kRowTab.r[row_of(q.y, q.oz)];
 #pragma clang loop unroll(full)
         for (int j = 0; j <= 2 * k.d; ++j)
-            cm[q.y + 2][j] = (w.cf + (size_t)(k.o0 + j) * kWave)[w.lane];
+            cm[coef_at<YN, R>(U, q.y)][j] = (w.cf + (size_t)(k.o0 + j) * kWave)[w.lane];
     }
 }
 
 template <int YN, int R, bool DIAG, int U>
 __device__ __forceinline__ void patch_step(const Wave &w, const int (&first)[YN],
-                                           double (&v)[2][R + 4], double (&cm)[5][5],
-                                           double (&acc)[YN][R], double (&gmin)[DIAG ? R : 1],
+                                           double (&v)[depth<YN, R>()][R + 4],
+                                           double (&cm)[5][5], double (&acc)[YN][R], double (&gmin)[DIAG ? R : 1],
                                            double (&gmax)[DIAG ? R : 1])
 {
     constexpr auto q = Patch<YN>::tab.r[U];
-    constexpr int B = U & 1;
-    if constexpr (U + 1 < Patch<YN>::tab.n) patch_load<YN, R, U + 1>(w, first, v[1 - B], cm);
+    constexpr int D = depth<YN, R>(), B = U % D;
+    if constexpr (U + D - 1 < Patch<YN>::tab.n)
+        patch_load<YN, R, U + D - 1>(w, first, v[(U + D - 1) % D], cm);
 #pragma clang loop unroll(full)
     for (int k = 0; k < YN; ++k)
     {
@@ -634,7 +647,7 @@ __device__ __forceinline__ void patch_step(const Wave &w, const int (&first)[YN]
         for (int j = 0; j <= 4; ++j)
         {
             if (j > 2 * d) continue;
-            const double cj = cm[q.y - k + 2][j];
+            const double cj = cm[coef_at<YN, R>(U, q.y - k)][j];
 #pragma clang loop unroll(full)
             for (int r = 0; r < R; ++r) acc[k][r] += cj * v[B][r + j + q.d - d];
             if constexpr (DIAG)
@@ -666,8 +679,11 @@ __device__ __forceinline__ void patch_rows(const Wave &w, const int (&first)[YN]
                                            double (&gmax)[DIAG ? R : 1],
                                            std::integer_sequence<int, U...>)
 {
-    double v[2][R + 4], cm[5][5];
+    constexpr int D = depth<YN, R>();
+    double v[D][R + 4], cm[5][5];
     patch_load<YN, R, 0>(w, first, v[0], cm);
+    if constexpr (D > 2) patch_load<YN, R, 1>(w, first, v[1], cm);
+    if constexpr (D > 3) patch_load<YN, R, 2>(w, first, v[2], cm);
     (patch_step<YN, R, DIAG, U>(w, first, v, cm, acc, gmin, gmax), ...);
 }
 
@@ -807,6 +823,19 @@ void stencil_free(ab_ctx *c)
     c->st_follow = nullptr;
     c->st_coef = nullptr;
     c->st_valid = false;
+}
+
+// The shared path has a floor of about 150 us (the coefficients' chain of dependent
+// FP64 operations, the longest items, the corner particles), the per-particle
+// path takes 15 us and 0.28 us per 1,000 interior quadratic (or 3,300 linear)
+// values. They meet at 500,000: us shared / per particle 205 / 116 at 337,000
+// (10^3 / Nv 8), 214 / 183 at 418,000 (12^3 / Nv 7), 160 / 231 at 546,000 (13^3 /
+// Nv 7), 170 / 304 at 1.04 million (14^3 / Nv 8); linear 152 / 133 at 421,000, 158 /
+// 193 at 629,000.
+bool stencil_shared(const ab_ctx *c)
+{
+    const double w = (c->cfg.mls_order >= 2 ? 1.0 : 0.3) * c->n_int + 0.3 * c->n_bnd;
+    return c->dim == 3 && w * c->nodes >= 5e5;
 }
 
 // Classes, runs and lists of the cloud as it is now, on its stream, without a

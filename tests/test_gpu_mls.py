@@ -47,11 +47,11 @@ def test_transport_on_a_jittered_cloud(name, nx, nv, order):
     assert (np.abs(sol.gt() - want) / scale).max() < 1e-12
 
 
-@pytest.mark.parametrize("amp", [0.0, 0.15])
-def test_step_statistics_match_oracle_and_change_nothing(amp):
+@pytest.mark.parametrize("nx,nv,amp", [(9, 5, 0.0), (9, 5, 0.15), (13, 7, 0.0)])
+def test_step_statistics_match_oracle_and_change_nothing(nx, nv, amp):
     """Flags and overshoots of the transport with stats; the same state, bit
     for bit, without them."""
-    case, cl, ocl, dt = _jittered("cavity3d", 9, 5, 2, amp)
+    case, cl, ocl, dt = _jittered("cavity3d", nx, nv, 2, amp)
     _, fl, ov = O.transport(ocl, cl.g, dt, cl.cfg.radius, 2, flags=True)
     a, b = A.Solver(cl, precision=A.PREC_FP64), A.Solver(cl, precision=A.PREC_FP64)
     st = a.step(dt, stats=True)
@@ -63,11 +63,11 @@ def test_step_statistics_match_oracle_and_change_nothing(amp):
     assert abs(st["mls_ovr_sum"] - ov.sum()) <= 1e-12 * np.abs(cl.g).sum() + 1e-9 * ov.sum()
 
 
-@pytest.mark.parametrize("name", ["cavity3d", "cavity2d"])
-def test_values_outside_the_support_do_not_enter(name):
+@pytest.mark.parametrize("name,nx,nv", [("cavity3d", 9, 5), ("cavity3d", 13, 7), ("cavity2d", 9, 5)])
+def test_values_outside_the_support_do_not_enter(name, nx, nv):
     """A neighbour that is not finite reaches exactly the nodes whose foot
     point has it in its support, as in the oracle."""
-    case, cl, ocl, dt = _jittered(name, 9, 5, 2, 0.0)
+    case, cl, ocl, dt = _jittered(name, nx, nv, 2, 0.0)
     p = cl.N // 2
     cl.g[p] = np.nan
     cl.g[p + 1] = np.inf
@@ -159,10 +159,12 @@ def _variant(kind, nx, nv, order):
 
 
 @pytest.mark.parametrize("kind,nx,nv,order", [
-    ("lattice", 13, 5, 2), ("lattice", 18, 4, 1), ("lattice", 5, 5, 2), ("lattice", 7, 9, 2),
-    ("few", 13, 5, 2), ("tiny", 12, 5, 2), ("permuted", 11, 5, 2), ("holes", 14, 4, 2),
-    ("twice", 11, 4, 2), ("mesh", 12, 5, 2), ("lid", 12, 5, 2)])
+    ("lattice", 13, 7, 2), ("lattice", 18, 7, 1), ("lattice", 7, 15, 2), ("lattice", 10, 5, 2),
+    ("few", 13, 7, 2), ("tiny", 13, 7, 2), ("permuted", 13, 7, 2), ("holes", 14, 7, 2),
+    ("twice", 13, 7, 2), ("mesh", 13, 7, 2), ("lid", 13, 7, 2)])
 def test_shared_stencils_match_oracle(kind, nx, nv, order):
+    """All but 10^3 / Nv 5 are above the 500,000 values from which stencils are
+    shared."""
     print(f"[mls] shared stencils {kind} {nx} Nv {nv} order {order}", flush=True)
     case, cl, ocl, dt = _variant(kind, nx, nv, order)
     sol = A.Solver(cl, precision=A.PREC_FP64)
@@ -176,7 +178,7 @@ def test_stencils_follow_the_cloud():
     """After a transport, particles move and gain a mesh velocity
     (ab_set_wall_state); the next transport, eager and as a replay of a graph
     captured before, sees them."""
-    case, cl, ocl, dt = _variant("lattice", 11, 4, 2)
+    case, cl, ocl, dt = _variant("lattice", 13, 7, 2)
     sols = [A.Solver(cl, precision=A.PREC_FP64) for _ in range(3)]
     graph = A.Graph([sols[1]], dt, 1)
     for s in sols[:2]:
@@ -200,7 +202,7 @@ def test_stencils_follow_the_cloud():
     cl.mesh = np.zeros((cl.N, 3))
     cl.mesh[p] = mv
     nb, nn = sols[0].neighbours()
-    ocl = O.Cloud(3, 4, cl.cfg.vmin, (cl.cfg.vmax - cl.cfg.vmin) / 3, cl.x, cl.y, cl.z, cl.boundary,
+    ocl = O.Cloud(3, 7, cl.cfg.vmin, (cl.cfg.vmax - cl.cfg.vmin) / 6, cl.x, cl.y, cl.z, cl.boundary,
                   cl.wall, nb, nn, cl.mesh)
     st = O.State(ocl, cl.g, cl.mom)
     O.step(ocl, st, dt, case.tau, case.R, cl.cfg.radius, 2)
