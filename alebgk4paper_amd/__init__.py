@@ -407,7 +407,7 @@ class ABBodyTask(C.Structure):
 
 def body_step_many(solvers, dt, bodies, geos, doms):
     """ab_body_step_many: the moving-body block of several solvers at once
-    (one host thread per cloud). bodies[k]: solver k's ABRigidBody list,
+    (each part of the block for all clouds, so their round trips overlap). bodies[k]: solver k's ABRigidBody list,
     updated in place; geos[k]: its (dx, dy, dz, minDist); doms[k]: its box as
     box() gives it. Returns the (removed, merged, added) counts per solver."""
     n = len(solvers)

@@ -54,7 +54,7 @@ void free_cloud(ab_ctx *c)
                     c->wt, c->mvx, c->mvy, c->mvz, c->rho, c->ux, c->uy, c->uz, c->T,
                     c->neigh, c->nneigh, c->ilist, c->blist, c->g, c->gt, c->limflag,
                     c->mlsflag, c->mlsovr, c->pmass, c->pnew, c->prho, c->pcol, c->vox, c->vcount, c->vstart, c->vlist,
-                    c->bmom, c->bidx, c->bwu, c->bbody, c->bcnt, c->bcon, c->bpar, c->bout,
+                    c->bmom, c->bidx, c->bwu, c->bbody, c->bcnt, c->bcon, c->bpar, c->bout, c->bblk,
                     c->bid, c->dm_alpha, c->dm_pass, c->dm_res, c->dm_rec,
                     c->mood, c->moodfail, c->inst, c->ih, c->seg};
     for (void *p : ptrs) if (p) (void)hipFree(p);
@@ -71,7 +71,8 @@ void free_cloud(ab_ctx *c)
     c->mlsflag = nullptr;
     c->vox = c->vcount = c->vstart = c->vlist = nullptr;
     c->bmom = c->bcon = c->bwu = c->bpar = c->bout = nullptr;
-    c->bidx = c->bbody = c->bcnt = nullptr;
+    c->bidx = c->bbody = c->bcnt = c->bblk = nullptr;
+    c->bblk_cap = 0;
     c->bmom_cap = 0;
     c->bid = nullptr;
     table_free(c);
@@ -649,6 +650,7 @@ int ab_destroy(ab_ctx *c)
     free_cloud(c);
     mlp_free(c);
     for (void *p : c->cm_pool) if (p) (void)hipFree(p);
+    if (c->mail) (void)hipHostFree(c->mail);
     if (c->scal) (void)hipFree(c->scal);
     for (auto e : c->evpool) if (e) (void)hipEventDestroy(e);
     if (c->ev0) (void)hipEventDestroy(c->ev0);

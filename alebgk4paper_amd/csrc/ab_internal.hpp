@@ -221,6 +221,9 @@ struct ab_ctx
     // results; a counter
     int bmom_cap = 0;
     int *bidx = nullptr, *bbody = nullptr, *bcnt = nullptr;
+    int *bblk = nullptr;           // counts per 1,024 particles of the surface list
+    int bblk_cap = 0;
+    double *mail = nullptr;        // pinned host memory: results of a body step's parts
     double *bmom = nullptr, *bcon = nullptr, *bwu = nullptr;
     double *bpar = nullptr, *bout = nullptr;
 
@@ -364,5 +367,13 @@ void table_free(ab_ctx *ctx);
 // boundary lists from the boundary flags.
 int relayout_cloud(ab_ctx *ctx, const int *src, int n);
 int rebuild_lists(ab_ctx *ctx);
+
+// ---- k_cloud.hip -------------------------------------------------------------
+// What the cloud management would change, counted without a host
+// synchronisation, and its bookkeeping where that is nothing.
+int cloud_probe(ab_ctx *ctx, int nbodies, const ab_body *bodies, double dx, double min_dist,
+                const double dom[6], const int *surf, int nsurf, const double box[6], int *removed,
+                int *merged, int *added);
+void cloud_unchanged(ab_ctx *ctx);
 
 }  // namespace ab

@@ -62,53 +62,76 @@ struct ShapeBody
     double v[3], om[3], angv;
 };
 
-constexpr int kParDoubles = (int)(sizeof(ShapeBody) / sizeof(double)) + 1;
-static_assert(sizeof(LoadBody) <= kParDoubles * sizeof(double), "parameter slot");
-static_assert(sizeof(MoveBody) <= kParDoubles * sizeof(double), "parameter slot");
+// The contact's shift of a body's surface.
+struct ShiftBody { double d[3]; int on; };
+
+// Counters of a body step: surface particles, those of no body, and what the
+// cloud management found to remove, to merge and to refill.
+enum { C_SURF = 0, C_BAD, C_REMOVE, C_MERGE, C_REFILL, kCounts = 8 };
+
+// Per-body parameters as a kernel argument.
+template <typename T>
+struct Par
+{
+    T b[kMaxBodies];
+    __host__ __device__ const T &operator[](int k) const { return b[k]; }
+};
+
+constexpr int kParDoubles = (int)(sizeof(LoadBody) / sizeof(double));
 
 // Stable list of the body-surface particles (boundary, body id >= 0) in
-// particle order; one workgroup of 1024 threads over contiguous ranges.
-// With idx == nullptr only the counts are written: count[0] the surface
-// particles, count[1] those whose body id is nb or more (no such body).
-__global__ __launch_bounds__(1024) void k_surface_list(int n, int nb,
-                                                       const unsigned char *__restrict__ bnd,
-                                                       const int *__restrict__ bid,
-                                                       int *__restrict__ idx,
-                                                       int *__restrict__ body,
-                                                       int *__restrict__ count)
+// particle order. count[0]: the surface particles, count[1]: those whose body id
+// is nb or more (no such body); the counters of the cloud management start at
+// zero. At most cap entries are written. k_surface_count: the same two counts of
+// each 1,024 particles; k_surface_place: the list from them.
+constexpr int kListBlock = 1024;
+int list_blocks(int n) { return std::max(1, (n + kListBlock - 1) / kListBlock); }
+
+__global__ __launch_bounds__(kListBlock) void k_surface_count(int n, int nb,
+                                                              const unsigned char *__restrict__ bnd,
+                                                              const int *__restrict__ bid,
+                                                              int *__restrict__ blk)
 {
-    __shared__ int sh[1024];
-    __shared__ int bad;
-    const int t = threadIdx.x;
-    if (t == 0) bad = 0;
-    const int per = (n + 1023) / 1024, lo = min(t * per, n), hi = min(lo + per, n);
-    int cnt = 0, nbad = 0;
-    for (int i = lo; i < hi; ++i)
-    {
-        cnt += (bnd[i] && bid[i] >= 0);
-        nbad += (bnd[i] && bid[i] >= nb);
-    }
+    const int i = blockIdx.x * kListBlock + threadIdx.x;
+    const bool surf = i < n && bnd[i] && bid[i] >= 0, bad = i < n && bnd[i] && bid[i] >= nb;
+    const int cs = __syncthreads_count(surf), cb = __syncthreads_count(bad);
+    if (threadIdx.x == 0) { blk[2 * blockIdx.x] = cs; blk[2 * blockIdx.x + 1] = cb; }
+}
+
+__global__ __launch_bounds__(kListBlock) void k_surface_place(int n,
+                                                              const unsigned char *__restrict__ bnd,
+                                                              const int *__restrict__ bid,
+                                                              const int *__restrict__ blk, int cap,
+                                                              int *__restrict__ idx,
+                                                              int *__restrict__ body,
+                                                              int *__restrict__ count)
+{
+    __shared__ int sh[kListBlock / kWave], base, total, bad;
+    const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
+    if (t == 0) base = total = bad = 0;
     __syncthreads();
+    int before = 0, all = 0, nbad = 0;
+    for (int q = t; q < (int)gridDim.x; q += kListBlock)
+    {
+        const int c = blk[2 * q];
+        all += c;
+        nbad += blk[2 * q + 1];
+        if (q < (int)blockIdx.x) before += c;
+    }
+    if (before) atomicAdd(&base, before);
+    if (all) atomicAdd(&total, all);
     if (nbad) atomicAdd(&bad, nbad);
-    sh[t] = cnt;
+    const int i = blockIdx.x * kListBlock + t;
+    const bool surf = i < n && bnd[i] && bid[i] >= 0;
+    const unsigned long long m = __ballot(surf);
+    if (lane == 0) sh[w] = __popcll(m);
     __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1)
-    {
-        const int v = t >= o ? sh[t - o] : 0;
-        __syncthreads();
-        sh[t] += v;
-        __syncthreads();
-    }
-    if (t == 1023) { count[0] = sh[1023]; count[1] = bad; }
-    if (!idx) return;
-    int pos = sh[t] - cnt;
-    for (int i = lo; i < hi; ++i)
-        if (bnd[i] && bid[i] >= 0)
-        {
-            idx[pos] = i;
-            body[pos] = bid[i];
-            ++pos;
-        }
+    int pos = base + __popcll(m & ((1ull << lane) - 1ull));
+    for (int q = 0; q < w; ++q) pos += sh[q];
+    if (surf && pos < cap) { idx[pos] = i; body[pos] = bid[i]; }
+    // (an unknown body id empties the list: the passes over it index the bodies)
+    if (blockIdx.x == 0 && t < kCounts)
+        count[t] = t == C_SURF ? (bad ? 0 : total) : (t == C_BAD ? bad : 0);
 }
 
 // Raw moments of the listed particles. Table storage holds g = L (M0 + d);
@@ -116,8 +139,9 @@ __global__ __launch_bounds__(1024) void k_surface_list(int n, int nb,
 template <typename T>
 __global__ void k_body_moments(DevCloud c, const T *__restrict__ g, int stride, const double *lazy,
                                const double *__restrict__ m0, const int *__restrict__ idx, int n,
-                               double *__restrict__ mom)
+                               double *__restrict__ mom, const int *__restrict__ dev = nullptr)
 {
+    if (dev) n = min(n, *dev);
     const int k = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
     const int lane = threadIdx.x & (kWave - 1);
     if (k >= n) return;
@@ -146,13 +170,17 @@ __global__ void k_body_moments(DevCloud c, const T *__restrict__ g, int stride, 
 // Force and torque contributions of each listed surface particle
 // (BodyDynamics.cpp:41-94) for a wall velocity U taken from the cloud's wall
 // state (umode 0), from wu (umode 1), or from the rigid motion of its body
-// (umode 2, setSurfaceVelocity :103-125).
+// (umode 2, setSurfaceVelocity :103-125). dev (may be null): the list's length
+// on the device, at most n of it.
+template <typename P>
 __global__ void k_surface_loads(DevCloud c, int n, const int *__restrict__ idx,
                                 const int *__restrict__ body, const double *__restrict__ mom,
                                 const double *__restrict__ wu, int umode,
-                                const LoadBody *__restrict__ lb, double *__restrict__ con)
+                                P lb, double *__restrict__ con,
+                                const int *__restrict__ dev = nullptr)
 {
 #pragma clang fp contract(off)
+    if (dev) n = min(n, *dev);
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
     const int i = idx[k];
@@ -200,10 +228,16 @@ __global__ void k_surface_loads(DevCloud c, int n, const int *__restrict__ idx,
 
 // One workgroup per body: the sum of its surface particles' contributions,
 // each thread over a strided share of the list, then a fixed tree.
+// dev: as in k_surface_loads; with cnt, the counters to mail.
 __global__ __launch_bounds__(256) void k_body_sum(int n, const int *__restrict__ body,
                                                   const double *__restrict__ con,
-                                                  double *__restrict__ out)
+                                                  double *__restrict__ out,
+                                                  const int *__restrict__ dev = nullptr,
+                                                  const int *__restrict__ cnt = nullptr,
+                                                  int *mail = nullptr)
 {
+    if (dev) n = min(n, *dev);
+    if (cnt && blockIdx.x == 0 && threadIdx.x < kCounts) mail[threadIdx.x] = cnt[threadIdx.x];
     __shared__ double sh[6][256];
     const int b = blockIdx.x, t = threadIdx.x;
     double a[6] = {0, 0, 0, 0, 0, 0};
@@ -228,7 +262,7 @@ __global__ __launch_bounds__(256) void k_body_sum(int n, const int *__restrict__
 // (BodyDynamics.cpp:405-440).
 __global__ void k_surface_move(int dim, int n, const int *__restrict__ idx,
                                const int *__restrict__ body, double dt,
-                               const MoveBody *__restrict__ mb, double *x, double *y, double *z)
+                               Par<MoveBody> mb, double *x, double *y, double *z)
 {
 #pragma clang fp contract(off)
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -302,19 +336,25 @@ __global__ __launch_bounds__(256) void k_body_extent(int n, const int *__restric
 }
 
 // The contact's rigid shift of a body's surface (BodyDynamics.cpp:588-594);
-// shift = 3 per body, applied only to bodies flagged in shift[3 nb + b].
-__global__ void k_surface_shift(int n, int nb, const int *__restrict__ idx,
-                                const int *__restrict__ body, const double *__restrict__ shift,
+// applied only to the bodies that it touches.
+__global__ void k_surface_shift(int n, const int *__restrict__ idx,
+                                const int *__restrict__ body, Par<ShiftBody> shift,
                                 double *x, double *y, double *z)
 {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
-    const int b = body[k];
-    if (shift[3 * nb + b] == 0.0) return;
+    const ShiftBody &S = shift[body[k]];
+    if (!S.on) return;
     const int i = idx[k];
-    x[i] += shift[3 * b];
-    y[i] += shift[3 * b + 1];
-    z[i] += shift[3 * b + 2];
+    x[i] += S.d[0];
+    y[i] += S.d[1];
+    z[i] += S.d[2];
+}
+
+// The cloud management's counters to the host's mailbox.
+__global__ void k_mail_counts(const int *__restrict__ cnt, int *mail)
+{
+    if (threadIdx.x < kCounts) mail[threadIdx.x] = cnt[threadIdx.x];
 }
 
 // getNormal / getNormal3 of the four shapes (Geometry.hpp:116-122,
@@ -372,7 +412,7 @@ __device__ void shape_normal(const ShapeBody &b, double x, double y, double z, d
 // normal, wall velocity v + w x r, and the mesh velocity that moves the
 // transport's foot points with the surface.
 __global__ void k_surface_refresh(DevCloud c, int n, const int *__restrict__ idx,
-                                  const int *__restrict__ body, const ShapeBody *__restrict__ sb,
+                                  const int *__restrict__ body, Par<ShapeBody> sb,
                                   double *wnx, double *wny, double *wnz, double *wux, double *wuy,
                                   double *wuz, double *mvx, double *mvy, double *mvz)
 {
@@ -413,6 +453,9 @@ __global__ void k_surface_refresh(DevCloud c, int n, const int *__restrict__ idx
         }                                                                               \
     } while (0)
 
+// Surface particles the scratch holds at least.
+constexpr int kMinSurf = 512;
+
 // Scratch of the body passes for ns surface particles (grown, kept).
 int body_scratch(ab_ctx *c, int ns)
 {
@@ -420,7 +463,7 @@ int body_scratch(ab_ctx *c, int ns)
     {
         if (hipMalloc((void **)&c->bpar, sizeof(double) * kParDoubles * kMaxBodies) != hipSuccess ||
             hipMalloc((void **)&c->bout, sizeof(double) * 8 * kMaxBodies) != hipSuccess ||
-            hipMalloc((void **)&c->bcnt, 2 * sizeof(int)) != hipSuccess)
+            hipMalloc((void **)&c->bcnt, kCounts * sizeof(int)) != hipSuccess)
         { c->err = "body scratch: device allocation failed"; return AB_ERR_NOMEM; }
     }
     if (ns <= c->bmom_cap) return AB_OK;
@@ -429,7 +472,7 @@ int body_scratch(ab_ctx *c, int ns)
     c->bidx = c->bbody = nullptr;
     c->bmom = c->bcon = c->bwu = nullptr;
     c->bmom_cap = 0;
-    const size_t n = (size_t)std::max(ns, 64);
+    const size_t n = (size_t)std::max(ns, kMinSurf);
     if (hipMalloc((void **)&c->bidx, sizeof(int) * n) != hipSuccess ||
         hipMalloc((void **)&c->bbody, sizeof(int) * n) != hipSuccess ||
         hipMalloc((void **)&c->bmom, sizeof(double) * 10 * n) != hipSuccess ||
@@ -440,7 +483,40 @@ int body_scratch(ab_ctx *c, int ns)
     return AB_OK;
 }
 
-void launch_moments(ab_ctx *c, const int *idx, int n, double *mom)
+// The per-1,024 counts of the surface list, for the current N, and the mailbox.
+int body_list_scratch(ab_ctx *c)
+{
+    if (!c->mail &&
+        hipHostMalloc((void **)&c->mail, sizeof(double) * (kCounts + 7 * kMaxBodies),
+                      hipHostMallocPortable) != hipSuccess)
+    { c->err = "body scratch: host allocation failed"; return AB_ERR_NOMEM; }
+    const int nl = list_blocks(c->N);
+    if (nl <= c->bblk_cap) return AB_OK;
+    if (c->bblk) (void)hipFree(c->bblk);
+    c->bblk = nullptr;
+    c->bblk_cap = 0;
+    if (hipMalloc((void **)&c->bblk, sizeof(int) * 2 * (size_t)nl) != hipSuccess)
+    { c->err = "body scratch: device allocation failed"; return AB_ERR_NOMEM; }
+    c->bblk_cap = nl;
+    return AB_OK;
+}
+
+// The bodies as the cloud management takes them.
+void managed_bodies(ab_body *cb, const ab_rigid_body *bodies, int nb)
+{
+    for (int b = 0; b < nb; ++b)
+    {
+        const ab_rigid_body &B = bodies[b];
+        std::memset(&cb[b], 0, sizeof cb[b]);
+        cb[b].shape = B.shape;
+        for (int a = 0; a < 3; ++a) cb[b].c[a] = B.c[a];
+        cb[b].size = B.size;
+        cb[b].o[0] = B.o[0]; cb[b].o[1] = B.o[1];
+        for (int a = 0; a < 9; ++a) cb[b].rm[a] = B.rm[a];
+    }
+}
+
+void launch_moments(ab_ctx *c, const int *idx, int n, double *mom, const int *dev = nullptr)
 {
     if (n <= 0) return;
     const int nb = (n * kWave + 255) / 256;
@@ -448,13 +524,13 @@ void launch_moments(ab_ctx *c, const int *idx, int n, double *mom)
     const bool tab = c->cfg.precision != AB_PREC_FP64 && c->dim == 3;
     if (!tab)
         k_body_moments<double><<<nb, 256, 0, c->stream>>>(v, c->g, c->gstride, nullptr, nullptr,
-                                                          idx, n, mom);
+                                                          idx, n, mom, dev);
     else if (c->cfg.precision == AB_PREC_MIXED)
         k_body_moments<float><<<nb, 256, 0, c->stream>>>(v, (const float *)c->gs, c->S,
-                                                         c->scal + S_LAZY, c->m0, idx, n, mom);
+                                                         c->scal + S_LAZY, c->m0, idx, n, mom, dev);
     else
         k_body_moments<double><<<nb, 256, 0, c->stream>>>(v, (const double *)c->gs, c->S,
-                                                          c->scal + S_LAZY, c->m0, idx, n, mom);
+                                                          c->scal + S_LAZY, c->m0, idx, n, mom, dev);
 }
 
 // Loads of nb bodies from the moments of n listed surface particles:
@@ -682,11 +758,76 @@ extern "C" int ab_body_loads_static(ab_ctx *c, int nsurf, const int *surf_idx,
     return body_loads_on(c, B, nsurf, surf_idx, surf_body, nbodies, body_c, body_area, wu, out);
 }
 
-extern "C" int ab_body_step(ab_ctx *c, double dt, int nb, ab_rigid_body *bodies, double dx,
-                            double min_dist, const double dom[6], double *loads_out, int *n_new,
-                            int counts[3])
+namespace ab {
+namespace {
+
+// The moving-body block of one cloud, cut where the host needs results of the
+// device: start, predict, move, contact, end. Each part but the last enqueues
+// work whose results a kernel writes into the context's mailbox (pinned host
+// memory), and the next part begins by waiting for them, so several clouds'
+// blocks run one part after another over all of them and wait together. What
+// bounds a block is the round trips, not its kernels: four of them, where the
+// block as separate calls with copies had twelve (a step of 16 cavities with a
+// free circle, 31 to 50 points a side, Nv 16, with the fluid steps: 8.1 -> 4.1
+// ms; of cavity3d-cube 40^3, Nv 10: 3.4 -> 3.0 ms).
+struct BodyBlock
 {
-    if (!c) return AB_ERR_ARG;
+    ab_ctx *c;
+    double dt;
+    int nb;
+    ab_rigid_body *bodies;
+    double dx, min_dist;
+    const double *dom;
+    double *loads;
+    int *n_new, *counts;
+    bool live = false;                 // the block has parts left to run
+    int ns = 0;
+    Par<LoadBody> lb{};
+    double L0[6 * kMaxBodies], L1[6 * kMaxBodies];
+
+    int *mail_counts() const { return (int *)c->mail; }
+    double *mail() const { return c->mail + kCounts; }   // doubles after the counters
+    int wait() const
+    {
+        BCHK(c, hipStreamSynchronize(c->stream));
+        return AB_OK;
+    }
+    int surface_loads(int umode, int n, const int *dev, double *out);
+    int list();
+    int start();
+    int predict();
+    int move();
+    int contact();
+    int end();
+};
+
+int BodyBlock::surface_loads(int umode, int n, const int *dev, double *out)
+{
+    hipStream_t s = c->stream;
+    if (n > 0)
+        k_surface_loads<<<(n + 255) / 256, 256, 0, s>>>(c->view(), n, c->bidx, c->bbody, c->bmom,
+                                                        nullptr, umode, lb, c->bcon, dev);
+    k_body_sum<<<nb, 256, 0, s>>>(n, c->bbody, c->bcon, out, dev, dev ? c->bcnt : nullptr,
+                                  mail_counts());
+    BCHK(c, hipGetLastError());
+    return AB_OK;
+}
+
+// The surface list in particle order, its raw moments and the loads at the
+// current wall state (BodyDynamics.cpp:353).
+int BodyBlock::list()
+{
+    hipStream_t s = c->stream;
+    const int nl = list_blocks(c->N);
+    k_surface_count<<<nl, kListBlock, 0, s>>>(c->N, nb, c->bnd, c->bid, c->bblk);
+    k_surface_place<<<nl, kListBlock, 0, s>>>(c->N, c->bnd, c->bid, c->bblk, c->bmom_cap, c->bidx,
+                                              c->bbody, c->bcnt);
+    launch_moments(c, c->bidx, c->bmom_cap, c->bmom, c->bcnt);
+    return surface_loads(0, c->bmom_cap, c->bcnt, mail());
+}
+
+int BodyBlock::start()
+{
     if (counts) counts[0] = counts[1] = counts[2] = 0;
     if (n_new) *n_new = c->N;
     if (nb < 0 || nb > kMaxBodies || (nb && !bodies) || !dom || !(dt > 0.0) ||
@@ -701,53 +842,45 @@ extern "C" int ab_body_step(ab_ctx *c, double dt, int nb, ab_rigid_body *bodies,
         if (bodies[b].shape < AB_BODY_SQUARE || bodies[b].shape > AB_BODY_CUBE ||
             bodies[b].npts <= 0 || !(bodies[b].mass > 0.0) || !(bodies[b].size > 0.0))
         { c->err = "ab_body_step: invalid body"; return AB_ERR_ARG; }
-    c->st_valid = false;           // the surface moves
-    hipStream_t s = c->stream;
-    const bool d3 = c->dim == 3;
     int rc;
-    // host sources of asynchronous copies: alive until the calls below have
-    // synchronised the stream
-    MoveBody mb[kMaxBodies];
-    ShapeBody sb[kMaxBodies];
-    double sh[4 * kMaxBodies];
-    if ((rc = body_scratch(c, 0))) return rc;
-    // the surface list, in particle order
-    k_surface_list<<<1, 1024, 0, s>>>(c->N, nb, c->bnd, c->bid, nullptr, nullptr, c->bcnt);
-    int cnt2[2] = {0, 0};
-    BCHK(c, hipMemcpyAsync(cnt2, c->bcnt, sizeof cnt2, hipMemcpyDeviceToHost, s));
-    BCHK(c, hipStreamSynchronize(s));
-    const int ns = cnt2[0];
-    if (cnt2[1])
+    if ((rc = body_scratch(c, kMinSurf)) || (rc = body_list_scratch(c))) return rc;
+    for (int b = 0; b < nb; ++b)
     {
-        c->err = "ab_body_step: " + std::to_string(cnt2[1]) +
+        for (int a = 0; a < 3; ++a) lb.b[b].c[a] = bodies[b].c[a];
+        lb.b[b].area = area(bodies[b]);
+    }
+    live = true;
+    return list();
+}
+
+// The loads arrive; the predictor (BodyDynamics.cpp:367-395; 2-D spin lives in
+// the z component) and the loads at the predicted wall velocities, same g
+// (:398-399).
+int BodyBlock::predict()
+{
+    int rc = wait();
+    if (rc) return rc;
+    ns = mail_counts()[C_SURF];
+    if (const int bad = mail_counts()[C_BAD])
+    {
+        c->err = "ab_body_step: " + std::to_string(bad) +
                  " surface particles carry a body id with no body given";
         return AB_ERR_ARG;
     }
-    if ((rc = body_scratch(c, ns))) return rc;
-    k_surface_list<<<1, 1024, 0, s>>>(c->N, nb, c->bnd, c->bid, c->bidx, c->bbody, c->bcnt);
-    launch_moments(c, c->bidx, ns, c->bmom);
-    BCHK(c, hipGetLastError());
-
-    // 1. loads at the current wall state (BodyDynamics.cpp:353)
-    LoadBody lb[kMaxBodies];
-    std::memset(lb, 0, sizeof lb);
-    for (int b = 0; b < nb; ++b)
+    if (ns > c->bmom_cap)
     {
-        for (int a = 0; a < 3; ++a) lb[b].c[a] = bodies[b].c[a];
-        lb[b].area = area(bodies[b]);
+        // more than the scratch held: a larger one, and the list again
+        if ((rc = body_scratch(c, ns)) || (rc = list()) || (rc = wait())) return rc;
     }
-    double L0[6 * kMaxBodies], L1[6 * kMaxBodies];
-    if ((rc = loads(c, c->bidx, c->bbody, ns, c->bmom, nullptr, 0, lb, nb, L0, c->bcon, c->bpar,
-                    c->bout)))
-        return rc;
-
-    // 2. predictor (:367-395); 2-D spin lives in the z component
+    c->st_valid = false;               // the surface moves
+    const bool d3 = c->dim == 3;
+    std::memcpy(L0, mail(), sizeof(double) * 6 * nb);
     for (int b = 0; b < nb; ++b)
     {
         const ab_rigid_body &B = bodies[b];
         const double I = inertia(B);
         const double *F = L0 + 6 * b, *T = F + 3;
-        LoadBody &l = lb[b];
+        LoadBody &l = lb.b[b];
         l.v[0] = B.vel[0] + F[0] * dt / B.mass;
         l.v[1] = B.vel[1] + F[1] * dt / B.mass;
         l.v[2] = d3 ? B.vel[2] + F[2] * dt / B.mass : 0.0;
@@ -772,52 +905,51 @@ extern "C" int ab_body_step(ab_ctx *c, double dt, int nb, ab_rigid_body *bodies,
             l.w[2] = d3 ? B.om[2] : B.angular_vel;
         }
     }
-    // 3. corrector loads at the predicted wall velocities, same g (:398-399)
-    if ((rc = loads(c, c->bidx, c->bbody, ns, c->bmom, nullptr, 2, lb, nb, L1, c->bcon, c->bpar,
-                    c->bout)))
-        return rc;
-    if (loads_out)
+    return surface_loads(2, ns, nullptr, mail());
+}
+
+// The corrector loads arrive; the rigid motion of the surface with the old
+// state (:405-440), Newton-Euler with the averaged loads (:451-519), and the
+// surface's extents.
+int BodyBlock::move()
+{
+    if (int rc = wait()) return rc;
+    hipStream_t s = c->stream;
+    const bool d3 = c->dim == 3;
+    std::memcpy(L1, mail(), sizeof(double) * 6 * nb);
+    if (loads)
         for (int b = 0; b < nb; ++b)
         {
-            std::memcpy(loads_out + 12 * b, L0 + 6 * b, 6 * sizeof(double));
-            std::memcpy(loads_out + 12 * b + 6, L1 + 6 * b, 6 * sizeof(double));
+            std::memcpy(loads + 12 * b, L0 + 6 * b, 6 * sizeof(double));
+            std::memcpy(loads + 12 * b + 6, L1 + 6 * b, 6 * sizeof(double));
         }
-
-    // 4. rigid motion of the surface with the old state (:405-440)
+    Par<MoveBody> mb{};
+    for (int b = 0; b < nb; ++b)
     {
-        std::memset(mb, 0, sizeof mb);
-        for (int b = 0; b < nb; ++b)
+        const ab_rigid_body &B = bodies[b];
+        MoveBody &m = mb.b[b];
+        for (int a = 0; a < 3; ++a) { m.c[a] = B.c[a]; m.v[a] = B.vel[a]; }
+        if (d3)
         {
-            const ab_rigid_body &B = bodies[b];
-            MoveBody &m = mb[b];
-            for (int a = 0; a < 3; ++a) { m.c[a] = B.c[a]; m.v[a] = B.vel[a]; }
-            if (d3)
+            const double wmag = std::sqrt(B.om[0] * B.om[0] + B.om[1] * B.om[1] + B.om[2] * B.om[2]);
+            m.rot = wmag > 1e-300;
+            if (m.rot)
             {
-                const double wmag = std::sqrt(B.om[0] * B.om[0] + B.om[1] * B.om[1] + B.om[2] * B.om[2]);
-                m.rot = wmag > 1e-300;
-                if (m.rot)
-                {
-                    for (int a = 0; a < 3; ++a) m.a[a] = B.om[a] / wmag;
-                    const double th = wmag * dt;
-                    m.cs = std::cos(th); m.sn = std::sin(th);
-                    m.omc = 1.0 - m.cs;
-                }
-            }
-            else
-            {
-                const double th = B.angular_vel * dt;
+                for (int a = 0; a < 3; ++a) m.a[a] = B.om[a] / wmag;
+                const double th = wmag * dt;
                 m.cs = std::cos(th); m.sn = std::sin(th);
+                m.omc = 1.0 - m.cs;
             }
         }
-        BCHK(c, hipMemcpyAsync(c->bpar, mb, sizeof(MoveBody) * nb, hipMemcpyHostToDevice, s));
-        if (ns > 0)
-            k_surface_move<<<(ns + 255) / 256, 256, 0, s>>>(c->dim, ns, c->bidx, c->bbody, dt,
-                                                            (const MoveBody *)c->bpar, c->x, c->y,
-                                                            c->z);
-        BCHK(c, hipGetLastError());
+        else
+        {
+            const double th = B.angular_vel * dt;
+            m.cs = std::cos(th); m.sn = std::sin(th);
+        }
     }
-
-    // 5. Newton-Euler with the averaged loads (:451-519)
+    if (ns > 0)
+        k_surface_move<<<(ns + 255) / 256, 256, 0, s>>>(c->dim, ns, c->bidx, c->bbody, dt, mb, c->x,
+                                                        c->y, c->z);
     for (int b = 0; b < nb; ++b)
     {
         ab_rigid_body &B = bodies[b];
@@ -860,96 +992,133 @@ extern "C" int ab_body_step(ab_ctx *c, double dt, int nb, ab_rigid_body *bodies,
         }
         if (d3) B.angular_vel = B.om[2];
     }
+    k_body_extent<<<nb, 256, 0, s>>>(ns, c->bidx, c->bbody, c->x, c->y, c->z, mail());
+    BCHK(c, hipGetLastError());
+    return AB_OK;
+}
 
-    // 5b. box-wall contact (:550-610)
+// The extents arrive; box-wall contact (:550-610), the surface wall state from
+// the new positions and state (:615-638), and what the cloud management around
+// the moved bodies (Solver.cpp:379-398) would find to do.
+int BodyBlock::contact()
+{
+    if (int rc = wait()) return rc;
+    hipStream_t s = c->stream;
+    const bool d3 = c->dim == 3;
+    double ext[7 * kMaxBodies];
+    std::memcpy(ext, mail(), sizeof(double) * 7 * nb);
+    // dom = xleft, xright, ybottom, ytop, zfront, zback
+    const double gap = 0.4 * std::fabs(dx);
+    const double xlo = std::min(dom[0], dom[1]), xhi = std::max(dom[0], dom[1]);
+    const double ylo = std::min(dom[2], dom[3]), yhi = std::max(dom[2], dom[3]);
+    const double zlo = std::min(dom[5], dom[4]), zhi = std::max(dom[5], dom[4]);
+    Par<ShiftBody> sh{};
+    bool any = false;
+    // the bounds of the whole surface, as k_bbox finds them
+    double box[6] = {1e300, -1e300, 1e300, -1e300, 1e300, -1e300};
+    for (int b = 0; b < nb; ++b)
     {
-        double ext[7 * kMaxBodies];
-        k_body_extent<<<nb, 256, 0, s>>>(ns, c->bidx, c->bbody, c->x, c->y, c->z, c->bout);
-        BCHK(c, hipGetLastError());
-        BCHK(c, hipMemcpyAsync(ext, c->bout, sizeof(double) * 7 * nb, hipMemcpyDeviceToHost, s));
-        BCHK(c, hipStreamSynchronize(s));
-        // dom = xleft, xright, ybottom, ytop, zfront, zback
-        const double gap = 0.4 * std::fabs(dx);
-        const double xlo = std::min(dom[0], dom[1]), xhi = std::max(dom[0], dom[1]);
-        const double ylo = std::min(dom[2], dom[3]), yhi = std::max(dom[2], dom[3]);
-        const double zlo = std::min(dom[5], dom[4]), zhi = std::max(dom[5], dom[4]);
-        std::memset(sh, 0, sizeof sh);
-        bool any = false;
-        for (int b = 0; b < nb; ++b)
+        const double *e = ext + 7 * b;
+        if (e[6] == 0.0) continue;
+        const double sx = std::max(0.0, (xlo + gap) - e[0]) - std::max(0.0, e[1] - (xhi - gap));
+        const double sy = std::max(0.0, (ylo + gap) - e[2]) - std::max(0.0, e[3] - (yhi - gap));
+        const double sz = d3 ? std::max(0.0, (zlo + gap) - e[4]) - std::max(0.0, e[5] - (zhi - gap))
+                             : 0.0;
+        const bool on = !(sx == 0.0 && sy == 0.0 && sz == 0.0);
+        const double d[3] = {on ? sx : 0.0, on ? sy : 0.0, on ? sz : 0.0};
+        for (int a = 0; a < 3; ++a)
         {
-            const double *e = ext + 7 * b;
-            if (e[6] == 0.0) continue;
-            const double sx = std::max(0.0, (xlo + gap) - e[0]) - std::max(0.0, e[1] - (xhi - gap));
-            const double sy = std::max(0.0, (ylo + gap) - e[2]) - std::max(0.0, e[3] - (yhi - gap));
-            const double sz = d3 ? std::max(0.0, (zlo + gap) - e[4]) - std::max(0.0, e[5] - (zhi - gap))
-                                 : 0.0;
-            if (sx == 0.0 && sy == 0.0 && sz == 0.0) continue;
-            ab_rigid_body &B = bodies[b];
-            B.c[0] += sx; B.c[1] += sy; B.c[2] += sz;
-            sh[3 * b] = sx; sh[3 * b + 1] = sy; sh[3 * b + 2] = sz;
-            sh[3 * nb + b] = 1.0;
-            any = true;
-            if (sx > 0.0 && B.vel[0] < 0.0) B.vel[0] = 0.0;
-            if (sx < 0.0 && B.vel[0] > 0.0) B.vel[0] = 0.0;
-            if (sy > 0.0 && B.vel[1] < 0.0) B.vel[1] = 0.0;
-            if (sy < 0.0 && B.vel[1] > 0.0) B.vel[1] = 0.0;
-            if (d3)
-            {
-                if (sz > 0.0 && B.vel[2] < 0.0) B.vel[2] = 0.0;
-                if (sz < 0.0 && B.vel[2] > 0.0) B.vel[2] = 0.0;
-            }
+            // (a shift rounds every position the same way, so the shifted
+            // extent is the extent of the shifted positions)
+            box[2 * a] = std::min(box[2 * a], on ? e[2 * a] + d[a] : e[2 * a]);
+            box[2 * a + 1] = std::max(box[2 * a + 1], on ? e[2 * a + 1] + d[a] : e[2 * a + 1]);
         }
-        if (any)
+        if (!on) continue;
+        ab_rigid_body &B = bodies[b];
+        B.c[0] += sx; B.c[1] += sy; B.c[2] += sz;
+        for (int a = 0; a < 3; ++a) sh.b[b].d[a] = d[a];
+        sh.b[b].on = 1;
+        any = true;
+        if (sx > 0.0 && B.vel[0] < 0.0) B.vel[0] = 0.0;
+        if (sx < 0.0 && B.vel[0] > 0.0) B.vel[0] = 0.0;
+        if (sy > 0.0 && B.vel[1] < 0.0) B.vel[1] = 0.0;
+        if (sy < 0.0 && B.vel[1] > 0.0) B.vel[1] = 0.0;
+        if (d3)
         {
-            BCHK(c, hipMemcpyAsync(c->bout, sh, sizeof(double) * 4 * nb, hipMemcpyHostToDevice, s));
-            k_surface_shift<<<(ns + 255) / 256, 256, 0, s>>>(ns, nb, c->bidx, c->bbody, c->bout,
-                                                             c->x, c->y, c->z);
-            BCHK(c, hipGetLastError());
+            if (sz > 0.0 && B.vel[2] < 0.0) B.vel[2] = 0.0;
+            if (sz < 0.0 && B.vel[2] > 0.0) B.vel[2] = 0.0;
         }
     }
-
-    // 6. surface wall state from the new positions and state (:615-638)
-    {
-        std::memset(sb, 0, sizeof sb);
-        for (int b = 0; b < nb; ++b)
-        {
-            const ab_rigid_body &B = bodies[b];
-            ShapeBody &q = sb[b];
-            q.shape = B.shape;
-            q.size = B.size;
-            q.angv = B.angular_vel;
-            for (int a = 0; a < 3; ++a) { q.c[a] = B.c[a]; q.v[a] = B.vel[a]; q.om[a] = B.om[a]; }
-            q.o[0] = B.o[0]; q.o[1] = B.o[1];
-            for (int a = 0; a < 9; ++a) q.rm[a] = B.rm[a];
-        }
-        BCHK(c, hipMemcpyAsync(c->bpar, sb, sizeof(ShapeBody) * nb, hipMemcpyHostToDevice, s));
-        if (ns > 0)
-            k_surface_refresh<<<(ns + 255) / 256, 256, 0, s>>>(
-                c->view(), ns, c->bidx, c->bbody, (const ShapeBody *)c->bpar, c->wnx, c->wny,
-                c->wnz, c->wux, c->wuy, c->wuz, c->mvx, c->mvy, c->mvz);
-        BCHK(c, hipGetLastError());
-        BCHK(c, hipStreamSynchronize(s));
-    }
-
-    // 7. cloud management around the moved bodies (Solver.cpp:379-398)
-    ab_body cb[kMaxBodies];
+    if (any && ns > 0)
+        k_surface_shift<<<(ns + 255) / 256, 256, 0, s>>>(ns, c->bidx, c->bbody, sh, c->x, c->y, c->z);
+    Par<ShapeBody> sb{};
     for (int b = 0; b < nb; ++b)
     {
         const ab_rigid_body &B = bodies[b];
-        std::memset(&cb[b], 0, sizeof cb[b]);
-        cb[b].shape = B.shape;
-        for (int a = 0; a < 3; ++a) cb[b].c[a] = B.c[a];
-        cb[b].size = B.size;
-        cb[b].o[0] = B.o[0]; cb[b].o[1] = B.o[1];
-        for (int a = 0; a < 9; ++a) cb[b].rm[a] = B.rm[a];
+        ShapeBody &q = sb.b[b];
+        q.shape = B.shape;
+        q.size = B.size;
+        q.angv = B.angular_vel;
+        for (int a = 0; a < 3; ++a) { q.c[a] = B.c[a]; q.v[a] = B.vel[a]; q.om[a] = B.om[a]; }
+        q.o[0] = B.o[0]; q.o[1] = B.o[1];
+        for (int a = 0; a < 9; ++a) q.rm[a] = B.rm[a];
     }
+    if (ns > 0)
+        k_surface_refresh<<<(ns + 255) / 256, 256, 0, s>>>(c->view(), ns, c->bidx, c->bbody, sb,
+                                                           c->wnx, c->wny, c->wnz, c->wux, c->wuy,
+                                                           c->wuz, c->mvx, c->mvy, c->mvz);
+    BCHK(c, hipGetLastError());
+    ab_body cb[kMaxBodies];
+    managed_bodies(cb, bodies, nb);
+    if (int rc = cloud_probe(c, nb, cb, dx, min_dist, dom, c->bidx, ns, box, c->bcnt + C_REMOVE,
+                             c->bcnt + C_MERGE, c->bcnt + C_REFILL))
+        return rc;
+    k_mail_counts<<<1, kWave, 0, s>>>(c->bcnt, mail_counts());
+    BCHK(c, hipGetLastError());
+    return AB_OK;
+}
+
+// Nothing to remove, merge or refill: the cloud stays and its lists are already
+// rebuilt. Else the cloud management, from its start.
+int BodyBlock::end()
+{
+    if (int rc = wait()) return rc;
+    const int *k = mail_counts();
+    if (!k[C_REMOVE] && !k[C_MERGE] && !k[C_REFILL])
+    {
+        cloud_unchanged(c);
+        return AB_OK;
+    }
+    ab_body cb[kMaxBodies];
+    managed_bodies(cb, bodies, nb);
     return ab_cloud_manage(c, nb, cb, nullptr, dx, min_dist, dom, n_new, counts);
 }
 
-// Several clouds' moving-body blocks in one call, one context after another
-// on the calling thread. (One host thread per context overlapped the
-// instances' synchronisations, but crashed inside the runtime's kernel
-// launch when a profiler traced the 16 threads; it is not used.)
+using Part = int (BodyBlock::*)();
+constexpr Part kParts[] = {&BodyBlock::start, &BodyBlock::predict, &BodyBlock::move,
+                           &BodyBlock::contact, &BodyBlock::end};
+
+}  // namespace
+}  // namespace ab
+
+extern "C" int ab_body_step(ab_ctx *c, double dt, int nb, ab_rigid_body *bodies, double dx,
+                            double min_dist, const double dom[6], double *loads_out, int *n_new,
+                            int counts[3])
+{
+    if (!c) return AB_ERR_ARG;
+    BodyBlock b{c, dt, nb, bodies, dx, min_dist, dom, loads_out, n_new, counts};
+    for (Part p : kParts)
+    {
+        if (p != kParts[0] && !b.live) break;
+        if (int rc = (b.*p)()) return rc;
+    }
+    return AB_OK;
+}
+
+// Several clouds' moving-body blocks in one call, on the calling thread: each
+// part of the block for all of them, so that their round trips overlap. (One
+// host thread per context overlapped them too, but crashed inside the runtime's
+// kernel launch when a profiler traced the 16 threads.)
 extern "C" int ab_body_step_many(int n, ab_ctx *const *ctxs, const ab_body_task *tasks)
 {
     if (n <= 0 || n > 64 || !ctxs || !tasks) return AB_ERR_ARG;
@@ -960,17 +1129,35 @@ extern "C" int ab_body_step_many(int n, ab_ctx *const *ctxs, const ab_body_task 
             if (ctxs[q] == ctxs[k]) { ctxs[k]->err = "ab_body_step_many: a context appears twice"; return AB_ERR_ARG; }
     }
     std::vector<int> rcs(n, AB_OK);
-    int cur = 0;
-    const bool have = hipGetDevice(&cur) == hipSuccess;
+    std::vector<BodyBlock> blocks;
+    blocks.reserve(n);
     for (int k = 0; k < n; ++k)
     {
-        ab_ctx *c = ctxs[k];
         const ab_body_task &t = tasks[k];
-        if (hipSetDevice(c->device) != hipSuccess)
-        { c->err = "ab_body_step_many: hipSetDevice failed"; rcs[k] = AB_ERR_HIP; continue; }
-        rcs[k] = ab_body_step(c, t.dt, t.nbodies, t.bodies, t.dx, t.min_dist, t.dom, t.loads,
-                              t.n_new, t.counts);
+        blocks.push_back(BodyBlock{ctxs[k], t.dt, t.nbodies, t.bodies, t.dx, t.min_dist, t.dom,
+                                   t.loads, t.n_new, t.counts});
     }
+    // tasks that share bodies follow one another, as separate calls would
+    bool shared = false;
+    for (int k = 0; k < n; ++k)
+        for (int q = 0; q < k; ++q)
+            shared = shared || (tasks[k].bodies < tasks[q].bodies + std::max(0, tasks[q].nbodies) &&
+                                tasks[q].bodies < tasks[k].bodies + std::max(0, tasks[k].nbodies));
+    int cur = 0;
+    const bool have = hipGetDevice(&cur) == hipSuccess;
+    auto run = [&](int k, Part p) {
+        ab_ctx *c = ctxs[k];
+        if (rcs[k] || (p != kParts[0] && !blocks[k].live)) return;
+        if (hipSetDevice(c->device) != hipSuccess)
+        { c->err = "ab_body_step_many: hipSetDevice failed"; rcs[k] = AB_ERR_HIP; }
+        else rcs[k] = (blocks[k].*p)();
+    };
+    if (shared)
+        for (int k = 0; k < n; ++k)
+            for (Part p : kParts) run(k, p);
+    else
+        for (Part p : kParts)
+            for (int k = 0; k < n; ++k) run(k, p);
     if (have) (void)hipSetDevice(cur);               // the caller's device as it was
     for (int k = 0; k < n; ++k)
         if (rcs[k]) return rcs[k];

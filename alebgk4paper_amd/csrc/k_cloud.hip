@@ -160,11 +160,12 @@ __global__ void k_surface_flags(int n, const unsigned char *__restrict__ bnd,
 }
 
 // manageRemove (CloudManagement.cpp:17-69): keep[i] = 0 for an interior
-// particle inside a body or within 0.4 dx of a body-surface particle.
+// particle inside a body or within 0.4 dx of a body-surface particle. With
+// found, only their number is taken (also in k_merge_cand and k_sites).
 __global__ void k_remove(int n, const double *__restrict__ x, const double *__restrict__ y,
                          const double *__restrict__ z, const unsigned char *__restrict__ bnd,
                          Bodies B, int d3, const int *__restrict__ surf, int nsurf, double hug2,
-                         unsigned char *__restrict__ keep)
+                         unsigned char *__restrict__ keep, int *found = nullptr)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -179,7 +180,8 @@ __global__ void k_remove(int n, const double *__restrict__ x, const double *__re
             drop = dist2(px, py, pz, x[q], y[q], z[q], d3) < hug2;
         }
     }
-    keep[i] = drop ? 0 : 1;
+    if (found) { if (drop) atomicAdd(found, 1); }
+    else keep[i] = drop ? 0 : 1;
 }
 
 // mergeCloseParticles, the candidates (CloudManagement.cpp:87-99): an
@@ -187,7 +189,8 @@ __global__ void k_remove(int n, const double *__restrict__ x, const double *__re
 __global__ void k_merge_cand(int n, const double *__restrict__ x, const double *__restrict__ y,
                              const double *__restrict__ z, const unsigned char *__restrict__ bnd,
                              const int *__restrict__ neigh, const int *__restrict__ nneigh,
-                             int d3, double min2, unsigned char *__restrict__ cand)
+                             int d3, double min2, unsigned char *__restrict__ cand,
+                             int *found = nullptr)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -202,7 +205,8 @@ __global__ void k_merge_cand(int n, const double *__restrict__ x, const double *
             c = dist2(x[i], y[i], z[i], x[j], y[j], z[j], d3) < min2;
         }
     }
-    cand[i] = c ? 1 : 0;
+    if (found) { if (c) atomicAdd(found, 1); }
+    else cand[i] = c ? 1 : 0;
 }
 
 // mergeCloseParticles, the greedy pass (CloudManagement.cpp:87-111) over the
@@ -310,7 +314,8 @@ __global__ __launch_bounds__(256) void k_sites(Sites S, int n, const double *__r
                                                const double *__restrict__ z, Bodies B, int d3,
                                                const int *__restrict__ surf, int nsurf,
                                                double hole2, double clr2,
-                                               unsigned char *__restrict__ ok)
+                                               unsigned char *__restrict__ ok,
+                                               int *found = nullptr)
 {
     const int s = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
     const int lane = threadIdx.x & (kWave - 1);
@@ -327,7 +332,10 @@ __global__ __launch_bounds__(256) void k_sites(Sites S, int n, const double *__r
         hug = dist2(x[q], y[q], z[q], xm, ym, zm, d3) < clr2;
     }
     const bool bad = __ballot(near || hug) != 0;
-    if (lane == 0) ok[s] = (!bad && !in_any(B, xm, ym, zm, d3)) ? 1 : 0;
+    if (lane != 0) return;
+    const bool fill = !bad && !in_any(B, xm, ym, zm, d3);
+    if (found) { if (fill) atomicAdd(found, 1); }
+    else ok[s] = fill ? 1 : 0;
 }
 
 // manageRefill's additions (CloudManagement.cpp:210-243), one block, the
@@ -537,7 +545,97 @@ int apply_keep(ab_ctx *c, Scratch &sc, const unsigned char *keep, int **body)
     return ab_rebuild_neighbours(c);
 }
 
+// The bodies as the kernels take them; false: an unknown shape.
+bool dev_bodies(Bodies &B, int nbodies, const ab_body *bodies)
+{
+    B.n = nbodies;
+    for (int k = 0; k < nbodies; ++k)
+    {
+        const ab_body &b = bodies[k];
+        if (b.shape < AB_BODY_SQUARE || b.shape > AB_BODY_CUBE) return false;
+        DevBody &d = B.b[k];
+        d.shape = b.shape; d.cx = b.c[0]; d.cy = b.c[1]; d.cz = b.c[2]; d.size = b.size;
+        d.ox = b.o[0]; d.oy = b.o[1];
+        for (int m = 0; m < 9; ++m) d.rm[m] = b.rm[m];
+    }
+    return true;
+}
+
+// The refill's site range around the surface's bounds hb, as
+// CloudManagement.cpp:156-171 computes it.
+Sites site_range(const double hb[6], const double dom[6], double dxl, bool d3)
+{
+    const double margin = 3.5 * dxl;
+    double bx0 = hb[0] - margin, bx1 = hb[1] + margin;
+    double by0 = hb[2] - margin, by1 = hb[3] + margin;
+    double bz0 = hb[4] - margin, bz1 = hb[5] + margin;
+    const int nxs = (int)std::llround((dom[1] - dom[0]) / dxl);
+    const int nys = (int)std::llround((dom[3] - dom[2]) / dxl);
+    const int nzs = d3 ? (int)std::llround((dom[5] - dom[4]) / dxl) : 0;
+    const int i0 = std::max(1, (int)std::ceil((bx0 - dom[0]) / dxl));
+    const int i1 = std::min(nxs - 1, (int)std::floor((bx1 - dom[0]) / dxl));
+    const int j0 = std::max(1, (int)std::ceil((by0 - dom[2]) / dxl));
+    const int j1 = std::min(nys - 1, (int)std::floor((by1 - dom[2]) / dxl));
+    const int k0 = d3 ? std::max(1, (int)std::ceil((bz0 - dom[4]) / dxl)) : 0;
+    const int k1 = d3 ? std::min(nzs - 1, (int)std::floor((bz1 - dom[4]) / dxl)) : 0;
+    Sites S{};
+    S.i0 = i0; S.j0 = j0; S.k0 = k0;
+    S.nx = std::max(0, i1 - i0 + 1);
+    S.ny = std::max(0, j1 - j0 + 1);
+    const int nz = std::max(0, k1 - k0 + 1);
+    S.n = S.nx * S.ny * nz;
+    S.xleft = dom[0]; S.ybottom = dom[2]; S.zfront = dom[4]; S.dxl = dxl;
+    return S;
+}
+
 }  // namespace
+
+namespace ab {
+
+// Counts what ab_cloud_manage would remove, merge and refill, without a host
+// synchronisation: its three tests on the cloud as it is, with the neighbour
+// rebuild that follows the removal. Where all three counts come out zero, this
+// was the whole management.
+int cloud_probe(ab_ctx *c, int nbodies, const ab_body *bodies, double dx, double min_dist,
+                const double dom[6], const int *surf, int nsurf, const double box[6], int *removed,
+                int *merged, int *added)
+{
+    Bodies B{};
+    if (!dev_bodies(B, nbodies, bodies))
+    { c->err = "ab_cloud_manage: unknown body shape"; return AB_ERR_ARG; }
+    c->st_valid = false;
+    hipStream_t s = c->stream;
+    const int N = c->N;
+    const bool d3 = c->dim == 3;
+    const double dxl = std::fabs(dx), hug2 = std::pow(0.4 * dxl, 2), min2 = min_dist * min_dist;
+    const double hole2 = std::pow(0.8 * dxl, 2), clr2 = std::pow(0.6 * dxl, 2);
+    if (N)
+        k_remove<<<(N + 255) / 256, 256, 0, s>>>(N, c->x, c->y, c->z, c->bnd, B, d3, surf, nsurf,
+                                                 hug2, nullptr, removed);
+    CMCHK(c, hipGetLastError());
+    if (int rc = ab_rebuild_neighbours(c)) return rc;
+    if (min2 > 0.0 && N > 0)
+        k_merge_cand<<<(N + 255) / 256, 256, 0, s>>>(N, c->x, c->y, c->z, c->bnd, c->neigh,
+                                                     c->nneigh, d3, min2, nullptr, merged);
+    if (nsurf > 0)
+    {
+        const Sites S = site_range(box, dom, dxl, d3);
+        if (S.n > 0)
+            k_sites<<<(S.n + 3) / 4, 256, 0, s>>>(S, N, c->x, c->y, c->z, B, d3, surf, nsurf, hole2,
+                                                  clr2, nullptr, added);
+    }
+    CMCHK(c, hipGetLastError());
+    return AB_OK;
+}
+
+// The source map of a management that left the cloud as it was.
+void cloud_unchanged(ab_ctx *c)
+{
+    c->cm_src.resize(c->N);
+    for (int i = 0; i < c->N; ++i) c->cm_src[i] = i;
+}
+
+}  // namespace ab
 
 extern "C" int ab_cloud_manage(ab_ctx *c, int nbodies, const ab_body *bodies, const int *body_id,
                                double dx, double min_dist, const double dom[6], int *n_new,
@@ -553,17 +651,8 @@ extern "C" int ab_cloud_manage(ab_ctx *c, int nbodies, const ab_body *bodies, co
         !(dx != 0.0) || !std::isfinite(dx))
     { c->err = "ab_cloud_manage: invalid argument"; return AB_ERR_ARG; }
     Bodies B{};
-    B.n = nbodies;
-    for (int k = 0; k < nbodies; ++k)
-    {
-        const ab_body &b = bodies[k];
-        if (b.shape < AB_BODY_SQUARE || b.shape > AB_BODY_CUBE)
-        { c->err = "ab_cloud_manage: unknown body shape"; return AB_ERR_ARG; }
-        DevBody &d = B.b[k];
-        d.shape = b.shape; d.cx = b.c[0]; d.cy = b.c[1]; d.cz = b.c[2]; d.size = b.size;
-        d.ox = b.o[0]; d.oy = b.o[1];
-        for (int m = 0; m < 9; ++m) d.rm[m] = b.rm[m];
-    }
+    if (!dev_bodies(B, nbodies, bodies))
+    { c->err = "ab_cloud_manage: unknown body shape"; return AB_ERR_ARG; }
     c->st_valid = false;
     const int N0 = c->N;
     c->cm_src.resize(N0);
@@ -663,27 +752,7 @@ extern "C" int ab_cloud_manage(ab_ctx *c, int nbodies, const ab_body *bodies, co
             double hb[6];
             CMCHK(c, hipMemcpyAsync(hb, box, sizeof hb, hipMemcpyDeviceToHost, s));
             CMCHK(c, hipStreamSynchronize(s));
-            // the site range, as CloudManagement.cpp:156-171 computes it
-            const double margin = 3.5 * dxl;
-            double bx0 = hb[0] - margin, bx1 = hb[1] + margin;
-            double by0 = hb[2] - margin, by1 = hb[3] + margin;
-            double bz0 = hb[4] - margin, bz1 = hb[5] + margin;
-            const int nxs = (int)std::llround((dom[1] - dom[0]) / dxl);
-            const int nys = (int)std::llround((dom[3] - dom[2]) / dxl);
-            const int nzs = d3 ? (int)std::llround((dom[5] - dom[4]) / dxl) : 0;
-            const int i0 = std::max(1, (int)std::ceil((bx0 - dom[0]) / dxl));
-            const int i1 = std::min(nxs - 1, (int)std::floor((bx1 - dom[0]) / dxl));
-            const int j0 = std::max(1, (int)std::ceil((by0 - dom[2]) / dxl));
-            const int j1 = std::min(nys - 1, (int)std::floor((by1 - dom[2]) / dxl));
-            const int k0 = d3 ? std::max(1, (int)std::ceil((bz0 - dom[4]) / dxl)) : 0;
-            const int k1 = d3 ? std::min(nzs - 1, (int)std::floor((bz1 - dom[4]) / dxl)) : 0;
-            Sites S{};
-            S.i0 = i0; S.j0 = j0; S.k0 = k0;
-            S.nx = std::max(0, i1 - i0 + 1);
-            S.ny = std::max(0, j1 - j0 + 1);
-            const int nz = std::max(0, k1 - k0 + 1);
-            S.n = S.nx * S.ny * nz;
-            S.xleft = dom[0]; S.ybottom = dom[2]; S.zfront = dom[4]; S.dxl = dxl;
+            const Sites S = site_range(hb, dom, dxl, d3);
             if (S.n > 0)
             {
                 const int N = c->N;
