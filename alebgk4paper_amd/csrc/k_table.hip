@@ -15,7 +15,8 @@
 // includes exactly these; self included for the gated nodes), grouped in 21
 // (ox, oy) columns of 5 or 3 z-offsets.
 //
-// Step (four kernels, six with the discrete collision; no host synchronisation):
+// Step (four kernels, six with the discrete collision; no host
+// synchronisation):
 //   k_apply      dt = sum_o C d  (stored deviation, below) one wave = 64 nodes of a
 //                lattice column (ix, iy); marches along z in blocks of K
 //                outputs with the class coefficients in registers and each
@@ -24,12 +25,14 @@
 //                pre-transport value), NAD, then the diffuse wall (boundary)
 //                or moments + BGK collision (interior), written back in place
 //                of g unscaled; FP64 partial sums per particle. With the
-//                discrete collision it stops after the moments, k_dm_solve
-//                (one thread per particle) finds the discrete Maxwellian and
+//                discrete collision it takes the interior only and stops
+//                after the moments, k_dm_wall (one thread per particle) finds
+//                the discrete Maxwellian and takes the boundary, and
 //                k_collide (one wave per particle) applies the collision.
-//   k_reduce     mass sums -> the two global rescale factors, folded into one
-//                lazy factor the stored g carries into the next step.
-//   k_finalize   per-particle rho, u, T of the step's end.
+//   k_reduce_stage  mass sums over ranges of particles.
+//   k_finalize   the two global rescale factors, folded into one lazy factor
+//                the stored g carries into the next step; per-particle rho, u,
+//                T of the step's end.
 // Homogeneity makes the lazy factor exact: wall, moments (u, T) and
 // collision are all homogeneous of degree 1 in a uniform rescale of g.
 #include "ab_device.hpp"
@@ -1782,9 +1785,10 @@ enum PostSlot { P_SC2, P_OKM, P_RAW, P_D = P_RAW + 5, P_COUNT = P_D + 5 };
 // register (the row's buffer descriptors are uniform); -1 past the list.
 // Consecutive blocks go to different XCDs (no remap): a wave reads only its
 // own row.
-__device__ __forceinline__ int list_particle(const int *__restrict__ list, int n)
+// (block: of the list, four particles each.)
+__device__ __forceinline__ int list_particle(const int *__restrict__ list, int n, int block)
 {
-    const int w = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / kWave);
+    const int w = __builtin_amdgcn_readfirstlane((block * blockDim.x + threadIdx.x) / kWave);
     return w < n ? __builtin_amdgcn_readfirstlane(list[w]) : -1;
 }
 
@@ -1797,21 +1801,28 @@ __device__ __forceinline__ int list_particle_rev(const int *__restrict__ list, i
     return w < n ? __builtin_amdgcn_readfirstlane(list[n - 1 - w]) : -1;
 }
 
-// One wave per boundary particle (the boundary list): positivity and the
-// diffuse wall. Partials: [0] committed mass, [1] mass after the wall, [2]
-// the wall density, [6] limiter bits.
+// The boundary list, one wave per particle: positivity and the diffuse wall.
+// Partials: [0] committed mass, [1] mass after the wall, [2] the wall density,
+// [6] limiter bits.
 template <typename T>
-__global__ __launch_bounds__(256) void k_wall(DevCloud c, Lat L, T *__restrict__ g,
-                                              T *__restrict__ gt, Ref ref,
-                                              const double *__restrict__ scal, double R,
-                                              double *__restrict__ part,
-                                              const int *__restrict__ blist, int nb)
+struct WallArgs
 {
-    const int i = list_particle(blist, nb);
+    T *g, *gt;
+    const int *blist;
+    int nb;
+    int blocks;               // ceil(nb / 4)
+};
+
+template <typename T>
+__device__ __forceinline__ void wall_block(const DevCloud &c, const Lat &L, const Ref &ref,
+                                           const double *scal, double R, double *part,
+                                           const WallArgs<T> &W, int block)
+{
+    const int i = list_particle(W.blist, W.nb, block);
     const int lane = threadIdx.x & (kWave - 1);
     if (i < 0) return;
     const double Lo = scal[S_LAZY];
-    const Row<T> row(g + (size_t)i * L.S, gt + (size_t)i * L.S, ref, lane, c.Nv, c.vlo, c.dv);
+    const Row<T> row(W.g + (size_t)i * L.S, W.gt + (size_t)i * L.S, ref, lane, c.Nv, c.vlo, c.dv);
     double out[kPart] = {0, 0, 0, 0, 0, 0, 0, 0};
     post_boundary<T>(c, i, row, ref, Lo, R, out);
     if (lane < kPart - 1) part[(size_t)i * kPart + lane] = out[lane];
@@ -1819,20 +1830,33 @@ __global__ __launch_bounds__(256) void k_wall(DevCloud c, Lat L, T *__restrict__
 
 // One wave per interior particle (the interior list): positivity, NAD and
 // moments; then (continuous collision) the BGK collision in the same kernel,
-// or (DM) the raw moments and the NAD factor are handed to k_dm_solve, which
-// derives the committed state one thread per particle, and k_collide.
+// or (DM) the raw moments and the NAD factor are handed to k_dm_wall, which
+// derives the committed state one thread per particle, and k_collide. The
+// first W.blocks blocks take the boundary list (none with DM: there k_dm_wall
+// takes it; the wall's registers would cost k_post<T, true> a wave per SIMD).
+// Boundary and interior in one launch: neither waits for the other's last wave
+// (a step, FP32, continuous: 13^3 Nv 7 77 -> 70 us, with the reduction's launch
+// saved too; 31^3 Nv 20 1681 -> 1635 us). Three waves per SIMD as before: FP64
+// spills 48 bytes for it in the limiters' repair path.
 // Partials: [0] committed mass, [1..5] moments after the collision, [6]
 // limiter bits.
 template <typename T, bool DM>
-__global__ __launch_bounds__(256) void k_post(DevCloud c, Lat L, T *__restrict__ g,
-                                              T *__restrict__ gt, Ref ref,
-                                              const double *__restrict__ rho,
-                                              const double *__restrict__ scal, double dt,
-                                              double tau, double R, double *__restrict__ part,
-                                              double *__restrict__ pst,
-                                              const int *__restrict__ ilist, int ni)
+__global__ __launch_bounds__(256, 3) void k_post(DevCloud c, Lat L, T *__restrict__ g,
+                                                 T *__restrict__ gt, Ref ref,
+                                                 const double *__restrict__ rho,
+                                                 const double *__restrict__ scal, double dt,
+                                                 double tau, double R, double *__restrict__ part,
+                                                 double *__restrict__ pst,
+                                                 const int *__restrict__ ilist, int ni,
+                                                 WallArgs<T> W)
 {
-    const int i = list_particle(ilist, ni);
+    if constexpr (!DM)
+        if ((int)blockIdx.x < W.blocks)
+        {
+            wall_block<T>(c, L, ref, scal, R, part, W, blockIdx.x);
+            return;
+        }
+    const int i = list_particle(ilist, ni, DM ? blockIdx.x : blockIdx.x - W.blocks);
     const int lane = threadIdx.x & (kWave - 1);
     if (i < 0) return;
     const double Lo = scal[S_LAZY];
@@ -1875,10 +1899,10 @@ __global__ __launch_bounds__(256) void k_post(DevCloud c, Lat L, T *__restrict__
 // wave's 64 particles on MFMA; every lane takes part), then Newton on the
 // separable grid sums until the relative residual passes. A converged
 // solution replaces the collision target exponent.
-__global__ __launch_bounds__(256) void k_dm_solve(int N, const unsigned char *__restrict__ bnd,
-                                                  DmArgs dm, Ref ref, const double *__restrict__ scal,
-                                                  double R, int Nv, double vlo, double dv,
-                                                  double *__restrict__ pst)
+__device__ __forceinline__ void dm_block(int N, const unsigned char *__restrict__ bnd,
+                                         const DmArgs &dm, const Ref &ref,
+                                         const double *__restrict__ scal, double R, int Nv,
+                                         double vlo, double dv, double *__restrict__ pst)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const size_t n = N;
@@ -1967,7 +1991,24 @@ __global__ __launch_bounds__(256) void k_dm_solve(int N, const unsigned char *__
     }
 }
 
-// The collision of the interior particles towards the target k_dm_solve left
+// The Newton solves, and in blocks of their own (the last W.blocks) the
+// boundary list: the solves are one block per CU waiting on serial chains, the
+// wall is row traffic, and neither reads what the other writes. Two waves per
+// SIMD with the solves' registers, where the wall alone had three: 27^3 Nv 9 in
+// FP64 with the discrete collision 367 -> 357 us a step, 40^3 Nv 10 in FP32 the
+// same (537 -> 535).
+template <typename T>
+__global__ __launch_bounds__(256) void k_dm_wall(DevCloud c, Lat L, DmArgs dm, Ref ref,
+                                                 const double *__restrict__ scal, double R,
+                                                 double *__restrict__ part,
+                                                 double *__restrict__ pst, WallArgs<T> W)
+{
+    const int solves = gridDim.x - W.blocks;
+    if ((int)blockIdx.x < solves) dm_block(c.N, c.bnd, dm, ref, scal, R, c.Nv, c.vlo, c.dv, pst);
+    else wall_block<T>(c, L, ref, scal, R, part, W, (int)blockIdx.x - solves);
+}
+
+// The collision of the interior particles towards the target k_dm_wall left
 // (one wave per particle, the list in reverse: k_post read it forwards);
 // partials [1..5].
 template <typename T>
@@ -1997,12 +2038,16 @@ __global__ __launch_bounds__(256) void k_collide(DevCloud c, Lat L, T *__restric
 }
 
 // Global sums of the partials -> the two rescale factors of cudaStep
-// (:1706-1710, :1773-1780), folded into the lazy factor. Two stages with a
-// fixed partition (deterministic): kRedBlocks blocks sum contiguous particle
-// ranges, then one block combines them.
+// (:1706-1710, :1773-1780), folded into the lazy factor, and the moments. The
+// sums have a fixed partition (deterministic): kRedBlocks blocks sum contiguous
+// particle ranges, then every block of k_finalize combines them for itself (4
+// KB from L2, where a launch of its own for it cost 2.4 us and a gap). red:
+// the pairs of sums, then the starting mass as k_reduce_stage found it.
 constexpr int kRedBlocks = 256;
+constexpr int kRedSize = 2 * kRedBlocks + 1;
 
 __global__ __launch_bounds__(256) void k_reduce_stage(int N, const double *__restrict__ part,
+                                                      const double *__restrict__ scal,
                                                       double *__restrict__ red)
 {
     __shared__ double sh[2 * (256 / kWave)];
@@ -2015,48 +2060,56 @@ __global__ __launch_bounds__(256) void k_reduce_stage(int N, const double *__res
         v[1] += part[(size_t)i * kPart + 1];
     }
     block_sum<2>(v, sh);
-    if (threadIdx.x == 0) { red[2 * blockIdx.x] = v[0]; red[2 * blockIdx.x + 1] = v[1]; }
+    if (threadIdx.x == 0)
+    {
+        red[2 * blockIdx.x] = v[0];
+        red[2 * blockIdx.x + 1] = v[1];
+        if (blockIdx.x == 0) red[2 * kRedBlocks] = scal[S_MASS_OLD];
+    }
 }
 
-__global__ __launch_bounds__(256) void k_reduce(const double *__restrict__ red, double *scal,
-                                                int nofix)
+__global__ __launch_bounds__(256) void k_finalize(DevCloud c, const double *__restrict__ part,
+                                                  const double *__restrict__ red, double *scal,
+                                                  int nofix, double R, double *rho, double *ux,
+                                                  double *uy, double *uz, double *T,
+                                                  double *limflag)
 {
-    __shared__ double sh[2 * (256 / kWave)];
-    double v[2] = {0.0, 0.0};
-    for (int b = threadIdx.x; b < kRedBlocks; b += 256) { v[0] += red[2 * b]; v[1] += red[2 * b + 1]; }
+    __shared__ double sh[2 * (256 / kWave)], fac[2];
+    double v[2] = {red[2 * threadIdx.x], red[2 * threadIdx.x + 1]};
+    static_assert(kRedBlocks == 256, "one pair of sums per thread");
     block_sum<2>(v, sh);
     if (threadIdx.x == 0)
     {
         const double mNew = v[0], hsum = v[1];
-        const double mOld = scal[S_MASS_OLD];
+        const double mOld = red[2 * kRedBlocks];
         const double s1 = (mNew > 1e-30) ? mOld / mNew : 1.0;
         const double mColl = s1 * hsum;
         const double s2 = (!nofix && mColl > 1e-30) ? mOld / mColl : 1.0;
-        scal[S_MASS_START] = mOld;
-        scal[S_MASS_NEW] = mNew;
-        scal[S_SCALE1] = s1;
-        scal[S_MASS_COLL] = mColl;
-        scal[S_SCALE2] = s2;
-        scal[S_LAZY] = s1 * s2;
-        scal[S_MASS_OLD] = s2 * mColl;          // the next step's starting mass
+        fac[0] = s1;
+        fac[1] = s1 * s2;
+        if (blockIdx.x == 0)
+        {
+            scal[S_MASS_START] = mOld;
+            scal[S_MASS_NEW] = mNew;
+            scal[S_SCALE1] = s1;
+            scal[S_MASS_COLL] = mColl;
+            scal[S_SCALE2] = s2;
+            scal[S_LAZY] = s1 * s2;
+            scal[S_MASS_OLD] = s2 * mColl;      // the next step's starting mass
+        }
     }
-}
-
-__global__ void k_finalize(DevCloud c, const double *__restrict__ part,
-                           const double *__restrict__ scal, double R, double *rho, double *ux,
-                           double *uy, double *uz, double *T, double *limflag)
-{
+    __syncthreads();
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= c.N) return;
     const double *p = part + (size_t)i * kPart;
     limflag[i] = p[6];
     if (c.bnd[i])
     {
-        rho[i] = scal[S_SCALE1] * p[2];
+        rho[i] = fac[0] * p[2];
         ux[i] = c.wux[i]; uy[i] = c.wuy[i]; uz[i] = c.wuz[i]; T[i] = c.wt[i];
         return;
     }
-    const double r = scal[S_LAZY] * p[1];
+    const double r = fac[1] * p[1];
     if (r > 1e-30)
     {
         const double mux = p[2] / p[1], muy = p[3] / p[1], muz = p[4] / p[1];
@@ -2373,7 +2426,7 @@ int table_setup(ab_ctx *ctx)
               && hipMalloc((void **)&ctx->m0, sizeof(double) * ctx->S) == hipSuccess
               && hipMalloc((void **)&ctx->m0x, sizeof(double) * kMaxNv) == hipSuccess
               && hipMalloc((void **)&ctx->m0xy, sizeof(double) * kMaxNv * kMaxNv) == hipSuccess
-              && hipMalloc((void **)&ctx->red, sizeof(double) * 2 * kRedBlocks) == hipSuccess
+              && hipMalloc((void **)&ctx->red, sizeof(double) * kRedSize) == hipSuccess
               && (ctx->cfg.collision != AB_COLLISION_DISCRETE
                   || hipMalloc((void **)&ctx->pst, sizeof(double) * P_COUNT * (size_t)N) == hipSuccess);
         if (!a) { table_free(ctx); ctx->err = "table setup: device allocation failed"; return AB_ERR_NOMEM; }
@@ -2540,35 +2593,36 @@ int table_step(ab_ctx *ctx, double dt)
     auto post = [&](auto *gs) {
         using T = std::remove_pointer_t<decltype(gs)>;
         T *gts = (T *)ctx->gts;
-        if (nb)
-            k_wall<T><<<nbb, 256, 0, s>>>(c, L, gs, gts, ref, ctx->scal, ctx->cfg.R, ctx->part,
-                                          ctx->blist, nb);
-        if (!ni) return;
+        const WallArgs<T> W{gs, gts, ctx->blist, nb, nbb};
         if (!dm.on)
         {
-            k_post<T, false><<<nbi, 256, 0, s>>>(c, L, gs, gts, ref, ctx->rho, ctx->scal, dt,
-                                                 ctx->cfg.tau, ctx->cfg.R, ctx->part, nullptr,
-                                                 ctx->ilist, ni);
+            if (nbi + nbb)
+                k_post<T, false><<<nbi + nbb, 256, 0, s>>>(c, L, gs, gts, ref, ctx->rho, ctx->scal,
+                                                           dt, ctx->cfg.tau, ctx->cfg.R, ctx->part,
+                                                           nullptr, ctx->ilist, ni, W);
             return;
         }
-        k_post<T, true><<<nbi, 256, 0, s>>>(c, L, gs, gts, ref, ctx->rho, ctx->scal, dt,
-                                            ctx->cfg.tau, ctx->cfg.R, ctx->part, ctx->pst,
-                                            ctx->ilist, ni);
-        k_dm_solve<<<nbs, 256, 0, s>>>(ctx->N, c.bnd, dm, ref, ctx->scal, ctx->cfg.R, ctx->Nv,
-                                       ctx->vlo, ctx->dv, ctx->pst);
-        k_collide<T><<<nbi, 256, 0, s>>>(c, L, gs, gts, ref, ctx->scal, dt, ctx->cfg.tau,
-                                         ctx->pst, ctx->part, ctx->ilist, ni);
+        if (ni)
+            k_post<T, true><<<nbi, 256, 0, s>>>(c, L, gs, gts, ref, ctx->rho, ctx->scal, dt,
+                                                ctx->cfg.tau, ctx->cfg.R, ctx->part, ctx->pst,
+                                                ctx->ilist, ni, WallArgs<T>{});
+        const int solves = ni ? nbs : 0;
+        if (solves + nbb)
+            k_dm_wall<T><<<solves + nbb, 256, 0, s>>>(c, L, dm, ref, ctx->scal, ctx->cfg.R,
+                                                      ctx->part, ctx->pst, W);
+        if (ni)
+            k_collide<T><<<nbi, 256, 0, s>>>(c, L, gs, gts, ref, ctx->scal, dt, ctx->cfg.tau,
+                                             ctx->pst, ctx->part, ctx->ilist, ni);
     };
     if (is_fp32(ctx)) post((float *)ctx->gs);
     else post((double *)ctx->gs);
     toc(ST_WALL_COLLIDE);
     dm_step_done(ctx);
     tic();
-    k_reduce_stage<<<kRedBlocks, 256, 0, s>>>(ctx->N, ctx->part, ctx->red);
-    k_reduce<<<1, 256, 0, s>>>(ctx->red, ctx->scal, ctx->cfg.no_mass_fix);
-    k_finalize<<<(ctx->N + 255) / 256, 256, 0, s>>>(c, ctx->part, ctx->scal, ctx->cfg.R,
-                                                    ctx->rho, ctx->ux, ctx->uy, ctx->uz,
-                                                    ctx->T, ctx->limflag);
+    k_reduce_stage<<<kRedBlocks, 256, 0, s>>>(ctx->N, ctx->part, ctx->scal, ctx->red);
+    k_finalize<<<std::max(1, nbs), 256, 0, s>>>(c, ctx->part, ctx->red, ctx->scal,
+                                                ctx->cfg.no_mass_fix, ctx->cfg.R, ctx->rho,
+                                                ctx->ux, ctx->uy, ctx->uz, ctx->T, ctx->limflag);
     toc(ST_FINAL);
     return hipGetLastError() == hipSuccess ? AB_OK : AB_ERR_HIP;
 }
