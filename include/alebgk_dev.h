@@ -337,8 +337,8 @@ int ab_body_step(ab_ctx *ctx, double dt, int nbodies, ab_rigid_body *bodies, dou
  * of the block runs for every context before the next, on the calling thread
  * (whose current device is restored), so that the contexts' waits overlap;
  * tasks that share bodies run one after another. Each cloud ends exactly as
- * ab_body_step alone leaves it. Returns the first failing task's status (its message in that context's
- * ab_last_error). n <= 64. */
+ * ab_body_step alone leaves it. Returns the first failing task's status (its
+ * message in that context's ab_last_error). n <= 64. */
 typedef struct ab_body_task {
     double dt;
     int nbodies;
