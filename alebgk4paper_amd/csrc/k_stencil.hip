@@ -296,7 +296,11 @@ __global__ void k_st_cut(int N, const int *__restrict__ key, const unsigned char
 }
 
 // The piece one lattice row up (+y) from the piece at i that can share its
-// loads: same class and length, every row of it the next row of i's. -1: none.
+// loads: same class and length, and every stencil row of it that the table of
+// i's run has one row further up (oy + 1) is that row. A patch reads row (y, oz)
+// through the first of its runs whose 21 rows reach it, so a box that ends at
+// oy = 1 forms no patch: there row oy = 1 of a later run would be read through
+// row oy = 2 of an earlier one, which has none. -1: none.
 __device__ __forceinline__ int piece_up(int i, const int *__restrict__ key, const int *__restrict__ rb,
                                         const unsigned char *__restrict__ plen)
 {
@@ -309,8 +313,8 @@ __device__ __forceinline__ int piece_up(int i, const int *__restrict__ key, cons
     {
         const Row q = kRowsDev.r[r];
         const int up = q.oy < 2 ? kRowsDev.of[(q.oy + 3) + 5 * (q.oz + 2)] : -1;
-        if (up >= 0 && in_box(k, 0, q.oy, q.oz) && in_box(k, 0, q.oy + 1, q.oz))
-            ok = ok && b[r] == a[up];
+        if (up >= 0 && in_box(k, 0, q.oy, q.oz))
+            ok = ok && in_box(k, 0, q.oy + 1, q.oz) && b[r] == a[up];
     }
     return ok ? t : -1;
 }

@@ -207,3 +207,73 @@ def test_stencils_follow_the_cloud():
     st = O.State(ocl, cl.g, cl.mom)
     O.step(ocl, st, dt, case.tau, case.R, cl.cfg.radius, 2)
     assert np.abs(sols[0].g() - st.g).max() < 1e-10 * np.abs(st.g).max()
+
+
+def _ball_lists(n, reach, chebyshev=None):
+    """Neighbour lists of an n[0] x n[1] x n[2] lattice: the sites nearer than
+    reach spacings, or (chebyshev) at most that many lattice steps away per axis."""
+    ix, iy, iz = (a.ravel() for a in np.meshgrid(*[np.arange(k) for k in n], indexing="ij"))
+    at = np.empty(n, np.int64)
+    p = ix + n[0] * (iy + n[1] * iz)
+    at[ix, iy, iz] = p
+    N = len(p)
+    neigh, nn = np.zeros((N, A.MAX_NEIGH), np.int32), np.zeros(N, np.int32)
+    m = int(np.ceil(reach)) if chebyshev is None else chebyshev
+    for oz in range(-m, m + 1):
+        for oy in range(-m, m + 1):
+            for ox in range(-m, m + 1):
+                if (ox, oy, oz) == (0, 0, 0) or \
+                        (chebyshev is None and ox * ox + oy * oy + oz * oz >= reach * reach):
+                    continue
+                jx, jy, jz = ix + ox, iy + oy, iz + oz
+                ok = (jx >= 0) & (jx < n[0]) & (jy >= 0) & (jy < n[1]) & (jz >= 0) & (jz < n[2])
+                i = p[ok]
+                neigh[i, nn[i]] = at[jx[ok], jy[ok], jz[ok]]
+                nn[i] += 1
+    return neigh, nn
+
+
+def _against_oracle(cl, ocl, dt, order, tol):
+    """Transport (over a gt that held NaN), the step's statistics, and the step
+    with and without them."""
+    R = cl.cfg.radius
+    want, fl, ov = O.transport(ocl, cl.g, dt, R, order, flags=True)
+    sol, g = A.Solver(cl, precision=A.PREC_FP64), cl.g
+    cl.g = np.full_like(g, np.nan)
+    sol.upload(cl)
+    sol.transport_only(dt)
+    assert np.isnan(sol.gt()).all()
+    cl.g = g
+    sol.upload(cl)
+    sol.transport_only(dt)
+    scale = np.abs(g).max(axis=1, keepdims=True)
+    err = np.abs(sol.gt() - want) / scale
+    assert not (err >= tol).any() and not np.isnan(err).any(), \
+        f"{(~(err < tol)).sum()} of {err.size} outputs, largest {np.nanmax(err):.2e}"
+    st = sol.step(dt, stats=True)
+    other = A.Solver(cl, precision=A.PREC_FP64)
+    other.step(dt)
+    assert np.array_equal(sol.g(), other.g())
+    assert st["n_mls_degenerate"] == int((fl & 1).astype(bool).sum())
+    assert abs(st["mls_ovr_sum"] - ov.sum()) <= tol * np.abs(g).sum() + 1e-9 * ov.sum()
+
+
+# radius in lattice spacings, lists: sites nearer than this many spacings, or the
+# 26 nearest. From sqrt(3) to 2 (and with the 26 nearest) every interior particle's
+# stencil reaches one step to each side, so stencils of runs one above the other
+# have fewer rows in common than at 2.5.
+@pytest.mark.parametrize("nx,order,radius,lists", [
+    (13, 2, 1.8, 1.8), (13, 2, 1.95, 1.95), (18, 1, 1.8, 1.8), (13, 2, 2.5, "26 nearest"),
+    (18, 1, 2.5, "26 nearest"), (13, 2, 2.1, 2.1), (13, 2, 2.5, 2.5), (18, 1, 1.3, 1.3),
+    (13, 2, 2.9, 2.9)])
+def test_shared_stencils_of_other_reach(nx, order, radius, lists):
+    print(f"[mls] shared stencils {nx} order {order} radius {radius} lists {lists}", flush=True)
+    case, cl, *_ = setup("cavity3d", nx, 7, order=order)
+    dx = 1e-6 / (nx - 1)
+    cl.cfg.radius = radius * dx
+    cl.neigh, cl.nneigh = _ball_lists((nx,) * 3, 0, 1) if lists == "26 nearest" else \
+        _ball_lists((nx,) * 3, lists)
+    # quadratic fits on the 26 nearest with weights down to 1e-3 at radius 1.8 amplify
+    # rounding about ten times more than at 2.5
+    _against_oracle(cl, _oracle_cloud(cl, cl.neigh, cl.nneigh), 0.3 * dx / 1303.0, order,
+                    1e-12 if radius > 2 else 1e-11)
