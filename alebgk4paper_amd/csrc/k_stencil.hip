@@ -334,14 +334,47 @@ __device__ __forceinline__ int bin_of(const DevCloud &c, const Bins &b, int i)
     return iy * b.nz + iz;
 }
 
-// Items: patches of kPatch pieces one above the other in y, aligned to lattice
-// rows 2, 6, 10, ..., where all of them are there, else single pieces. Counted
-// per bin (COUNT), then placed from the bin's start; the particles of no class
-// into their lists.
+// The place in its patch that a piece of key k asks for: its lattice row counted
+// from the key's first particle, which keeps lattice rows 2, 6, 10, ... first
+// and, wherever the lattice lies, y differences near whole spacings.
+__device__ __forceinline__ int patch_place(const DevCloud &c, const Bins &bins, int i, int r)
+{
+    return (int)rint((c.y[i] - c.y[r]) * bins.isy) & (kPatch - 1);
+}
+
+// Whether the piece at base is the first of a patch, its pieces into at: places
+// 0 .. kPatch - 1 in turn, each linked to the next upwards (piece_up) and
+// downwards. So a piece belongs to one patch at most, the one that its own links
+// lead down to, and every piece that asks gets the same answer, whatever the
+// spacing that the places are counted with.
+__device__ __forceinline__ bool patch_at(const DevCloud &c, const Bins &bins, int base,
+                                         const int *__restrict__ key, const int *__restrict__ rb,
+                                         const int *__restrict__ rep,
+                                         const unsigned char *__restrict__ plen, int (&at)[kPatch])
+{
+    at[0] = base;
+    if (key[base] < 0 || !plen[base]) return false;
+    const int r = rep[key[base]];
+    if (patch_place(c, bins, base, r) != 0) return false;
+    for (int q = 1; q < kPatch; ++q)
+    {
+        const int t = piece_up(at[q - 1], key, rb, plen);
+        if (t < 0 || patch_place(c, bins, t, r) != q ||
+            rb[(size_t)t * kRowPad + row_of(-1, 0)] != at[q - 1])
+            return false;
+        at[q] = t;
+    }
+    return true;
+}
+
+// Items: patches of kPatch pieces one above the other in y, where all of them
+// are there, else single pieces. Counted per bin (COUNT), then placed from the
+// bin's start; the particles of no class into their lists.
 template <bool COUNT>
 __global__ void k_st_emit(DevCloud c, Bins bins, const int *__restrict__ key,
-                          const int *__restrict__ rb, const unsigned char *__restrict__ plen,
-                          int *bin, int *__restrict__ item, int *__restrict__ irr_int,
+                          const int *__restrict__ rb, const int *__restrict__ rep,
+                          const unsigned char *__restrict__ plen, int *bin,
+                          int *__restrict__ item, int *__restrict__ irr_int,
                           int *__restrict__ irr_bnd, int *n)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -354,21 +387,11 @@ __global__ void k_st_emit(DevCloud c, Bins bins, const int *__restrict__ key,
         return;
     }
     if (!plen[i]) return;
-    // the piece's place in its patch, and the patch's first piece
-    const int place = ((int)rint((c.y[i] - bins.y0) * bins.isy) - 2) & (kPatch - 1);
+    const int place = patch_place(c, bins, i, rep[key[i]]);
     int base = i;
-    for (int q = 0; q < place && base >= 0; ++q)
-    {
-        const int t = rb[(size_t)base * kRowPad + row_of(-1, 0)];
-        base = t != base && plen[t] ? t : -1;
-    }
-    int at[kPatch] = {base, -1, -1, -1};
-    for (int q = 1; q < kPatch && base >= 0; ++q)
-    {
-        at[q] = piece_up(at[q - 1], key, rb, plen);
-        if (at[q] < 0) base = -1;
-    }
-    const bool patch = base >= 0 && at[place] == i;
+    for (int q = 0; q < place; ++q) base = rb[(size_t)base * kRowPad + row_of(-1, 0)];
+    int at[kPatch];
+    const bool patch = patch_at(c, bins, base, key, rb, rep, plen, at) && at[place] == i;
     if (patch && place) return;                        // its first piece places the patch
     const int k = atomicAdd(&bin[bin_of(c, bins, i)], 1);
     if (COUNT) return;
@@ -880,11 +903,11 @@ int stencil_prepare(ab_ctx *c)
     unsigned char *plen = c->st_follow + N;
     k_st_follow<<<nt, 256, 0, s>>>(c->N, c->st_key, c->st_rb, c->st_follow, plen);
     k_st_cut<<<nt, 256, 0, s>>>(c->N, c->st_key, c->st_follow, plen);
-    k_st_emit<true><<<nt, 256, 0, s>>>(v, bins, c->st_key, c->st_rb, plen, c->st_bin, c->st_run,
-                                       c->st_int, c->st_bnd, c->st_n);
+    k_st_emit<true><<<nt, 256, 0, s>>>(v, bins, c->st_key, c->st_rb, c->st_rep, plen, c->st_bin,
+                                       c->st_run, c->st_int, c->st_bnd, c->st_n);
     k_st_scan<<<1, 1024, 0, s>>>(nbin, c->st_bin, c->st_n);
-    k_st_emit<false><<<nt, 256, 0, s>>>(v, bins, c->st_key, c->st_rb, plen, c->st_bin, c->st_run,
-                                        c->st_int, c->st_bnd, c->st_n);
+    k_st_emit<false><<<nt, 256, 0, s>>>(v, bins, c->st_key, c->st_rb, c->st_rep, plen, c->st_bin,
+                                        c->st_run, c->st_int, c->st_bnd, c->st_n);
     if (hipGetLastError() != hipSuccess) { c->err = "FP64 transport: classification failed"; return AB_ERR_HIP; }
     c->st_valid = true;
     return AB_OK;
