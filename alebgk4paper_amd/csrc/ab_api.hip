@@ -53,7 +53,7 @@ void free_cloud(ab_ctx *c)
     void *ptrs[] = {c->x, c->y, c->z, c->bnd, c->wnx, c->wny, c->wnz, c->wux, c->wuy, c->wuz,
                     c->wt, c->mvx, c->mvy, c->mvz, c->rho, c->ux, c->uy, c->uz, c->T,
                     c->neigh, c->nneigh, c->ilist, c->blist, c->g, c->gt, c->limflag,
-                    c->mlsflag, c->mlsovr, c->pmass, c->pnew, c->prho, c->pcol, c->vox, c->vcount, c->vstart, c->vlist,
+                    c->mlsflag, c->mlsovr, c->pmass, c->pnew, c->vox, c->vcount, c->vstart, c->vlist,
                     c->bmom, c->bidx, c->bwu, c->bbody, c->bcnt, c->bcon, c->bpar, c->bout, c->bblk,
                     c->bid, c->dm_alpha, c->dm_pass, c->dm_res, c->dm_rec,
                     c->mood, c->moodfail, c->inst, c->ih, c->seg};
@@ -68,6 +68,7 @@ void free_cloud(ab_ctx *c)
     c->rho = c->ux = c->uy = c->uz = c->T = nullptr;
     c->neigh = c->nneigh = c->ilist = c->blist = nullptr;
     c->g = c->gt = c->limflag = c->mlsovr = c->pmass = c->pnew = c->prho = c->pcol = nullptr;
+    c->pnew_cap = 0;
     c->mlsflag = nullptr;
     c->vox = c->vcount = c->vstart = c->vlist = nullptr;
     c->bmom = c->bcon = c->bwu = c->bpar = c->bout = nullptr;
@@ -87,8 +88,20 @@ int alloc_cloud(ab_ctx *c)
     int rc = 0;
     double **dd[] = {&c->x, &c->y, &c->z, &c->wnx, &c->wny, &c->wnz, &c->wux, &c->wuy, &c->wuz,
                      &c->wt, &c->mvx, &c->mvy, &c->mvz, &c->rho, &c->ux, &c->uy, &c->uz, &c->T,
-                     &c->limflag, &c->mlsovr, &c->pmass, &c->pnew, &c->prho, &c->pcol};
+                     &c->limflag, &c->mlsovr, &c->pmass};
     for (double **p : dd) if ((rc = dalloc(c, p, N))) return rc;
+    if (N > c->pnew_cap)
+    {
+        // one array, kept by a re-layout while it is long enough
+        if (c->pnew) (void)hipFree(c->pnew);
+        c->pnew = c->prho = c->pcol = nullptr;
+        c->pnew_cap = 0;
+        const size_t cap = N + N / 16;
+        if ((rc = dalloc(c, &c->pnew, 3 * cap))) return rc;
+        c->pnew_cap = cap;
+        c->prho = c->pnew + cap;
+        c->pcol = c->prho + cap;
+    }
     if ((rc = dalloc(c, &c->bnd, N))) return rc;
     if ((rc = dalloc(c, &c->neigh, N * AB_MAX_NEIGH))) return rc;
     if ((rc = dalloc(c, &c->nneigh, N))) return rc;
@@ -390,7 +403,9 @@ __global__ void k_gather_bid(const int *__restrict__ src, int *__restrict__ dst,
 
 // Re-lays the cloud out for n particles: particle i takes the state of old
 // particle src[i] (src: n entries on the device), or zero where src[i] < 0
-// (a particle the caller fills in). The per-step scratch starts at zero;
+// (a particle the caller fills in). The per-step scratch starts at zero, but for
+// what every step writes before it reads it: that and the stencil classes' arrays
+// stay where they are while they hold n particles (a free synchronises the device);
 // the neighbour-search scratch and the training-row ring, sized by N, are
 // dropped. Neighbour lists and the interior/boundary lists are left to the
 // caller.
@@ -403,20 +418,19 @@ int relayout_cloud(ab_ctx *c, const int *src, int n)
     constexpr int nc = sizeof(carried) / sizeof(carried[0]);
     double *od[nc];
     for (int k = 0; k < nc; ++k) { od[k] = *carried[k]; *carried[k] = nullptr; }
-    double *og = c->g, *ogt = c->gt, *olim = c->limflag, *oovr = c->mlsovr, *opm = c->pmass, *opn = c->pnew, *opr = c->prho, *opc = c->pcol;
+    double *og = c->g, *ogt = c->gt, *olim = c->limflag, *oovr = c->mlsovr, *opm = c->pmass;
     double *oalpha = c->dm_alpha, *ores = c->dm_res;
     int *opass = c->dm_pass, *omls = c->mlsflag, *omood = c->mood, *omf = c->moodfail;
     int *onb = c->neigh, *onn = c->nneigh, *oil = c->ilist, *obl = c->blist, *obid = c->bid;
     unsigned char *obnd = c->bnd;
-    c->g = c->gt = c->limflag = c->mlsovr = c->pmass = c->pnew = c->prho = c->pcol = nullptr;
-    c->dm_alpha = c->dm_res = nullptr;
+    c->g = c->gt = c->limflag = c->mlsovr = c->pmass = c->dm_alpha = c->dm_res = nullptr;
     c->dm_pass = c->mlsflag = c->mood = c->moodfail = nullptr;
     c->neigh = c->nneigh = c->ilist = c->blist = c->bid = nullptr;
     c->bnd = nullptr;
     const int oldN = c->N;
     c->N = n;
     c->cfg.n_particles = n;
-    stencil_free(c);               // sized by N
+    c->st_valid = false;
     int rc = alloc_cloud(c);
     auto gather = [&](auto *from, auto *to, int stride) {
         const size_t tot = (size_t)n * stride;
@@ -446,7 +460,7 @@ int relayout_cloud(ab_ctx *c, const int *src, int n)
         if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
         { c->err = "cloud re-layout: gather failed"; rc = AB_ERR_HIP; }
     }
-    void *old[] = {og, ogt, olim, oovr, opm, opn, opr, opc, oalpha, ores, opass, omls, omood, omf,
+    void *old[] = {og, ogt, olim, oovr, opm, oalpha, ores, opass, omls, omood, omf,
                    onb, onn, oil, obl, obnd, obid, c->vox, c->vlist, c->dm_rec};
     for (void *p : old) if (p) (void)hipFree(p);
     for (int k = 0; k < nc; ++k) if (od[k]) (void)hipFree(od[k]);

@@ -114,6 +114,7 @@ struct ab_ctx
     double *pnew = nullptr;        // committed mass per particle of the fused commit and collision
     double *prho = nullptr;        // its wall densities (3-D)
     double *pcol = nullptr;        // its collided masses
+    size_t pnew_cap = 0;           // particles that pnew, prho and pcol (one allocation) hold
     double *scal = nullptr;        // ab::ScalarSlot
     bool mass_valid = false;       // pmass holds the current g's masses
     // Bumped whenever the device arrays are freed, re-allocated or refilled
@@ -140,6 +141,7 @@ struct ab_ctx
     unsigned char *st_follow = nullptr;
     double *st_coef = nullptr;
     int st_maxslot = 0;
+    int st_cap = 0;                // particles the arrays hold
     bool st_valid = false;         // false once positions, lists or wall state change
 
     // table pipelines (AB_PREC_MIXED / AB_PREC_FP64_TABLE)

@@ -836,7 +836,7 @@ __global__ __launch_bounds__(kBlock, DIAG ? 2 : 3) void k_apply_runs(DevCloud c,
 }
 
 template <typename T>
-bool dev(T **p, size_t n) { return *p || hipMalloc((void **)p, n * sizeof(T)) == hipSuccess; }
+bool dev(T **p, size_t n) { return hipMalloc((void **)p, n * sizeof(T)) == hipSuccess; }
 
 }  // namespace
 
@@ -849,6 +849,7 @@ void stencil_free(ab_ctx *c)
     c->st_run = c->st_int = c->st_bnd = c->st_bin = nullptr;
     c->st_follow = nullptr;
     c->st_coef = nullptr;
+    c->st_cap = 0;
     c->st_valid = false;
 }
 
@@ -871,11 +872,6 @@ int stencil_prepare(ab_ctx *c)
 {
     const size_t N = (size_t)c->N;
     const int nchunk = (c->nodes + kWave - 1) / kWave;
-    // coefficient slots: the 125 classes of a box lattice and some more, but
-    // never more memory than g itself takes
-    const size_t one = (size_t)nchunk * kCoefRows * kWave;
-    c->st_maxslot = (int)std::min<size_t>(160, N * c->gstride / one);
-    const int ms = std::max(c->st_maxslot, 1);
     const ab_config &f = c->cfg;
     // the lattice spacing, a guess that the checks do not rely on: voxels are
     // three spacings wide; without a voxel grid the radius is 2.5 of them
@@ -886,11 +882,24 @@ int stencil_prepare(ab_ctx *c)
     const int nbin = bins.ny * bins.nz;
     if (N >= (size_t)INT_MAX / kItem)
     { c->err = "FP64 transport: too many particles"; return AB_ERR_UNSUPPORTED; }
-    if (!dev(&c->st_key, N) || !dev(&c->st_rb, N * kRowPad) || !dev(&c->st_rep, kKeys) ||
-        !dev(&c->st_cnt, kKeys) || !dev(&c->st_slot, kKeys) || !dev(&c->st_skey, ms) ||
-        !dev(&c->st_n, N_COUNT) || !dev(&c->st_run, N * kItem) || !dev(&c->st_int, N) ||
-        !dev(&c->st_bnd, N) || !dev(&c->st_bin, (size_t)nbin) || !dev(&c->st_follow, 2 * N) || !dev(&c->st_coef, one * ms))
-    { c->err = "FP64 transport: device allocation failed"; return AB_ERR_NOMEM; }
+    // coefficient slots: the 125 classes of a box lattice and some more, but
+    // never more memory than g itself takes
+    const size_t one = (size_t)nchunk * kCoefRows * kWave;
+    auto slots = [&](size_t n) { return (int)std::min<size_t>(160, n * c->gstride / one); };
+    if (c->N > c->st_cap)
+    {
+        // some room for the particles that cloud management adds
+        stencil_free(c);
+        const size_t cap = N + N / 16, ms = std::max(slots(cap), 1);
+        if (!dev(&c->st_key, cap) || !dev(&c->st_rb, cap * kRowPad) || !dev(&c->st_rep, kKeys) ||
+            !dev(&c->st_cnt, kKeys) || !dev(&c->st_slot, kKeys) || !dev(&c->st_skey, ms) ||
+            !dev(&c->st_n, N_COUNT) || !dev(&c->st_run, cap * kItem) || !dev(&c->st_int, cap) ||
+            !dev(&c->st_bnd, cap) || !dev(&c->st_bin, (size_t)nbin) ||
+            !dev(&c->st_follow, 2 * cap) || !dev(&c->st_coef, one * ms))
+        { c->err = "FP64 transport: device allocation failed"; return AB_ERR_NOMEM; }
+        c->st_cap = (int)cap;
+    }
+    c->st_maxslot = slots(N);          // of this N, whatever the arrays hold
     DevCloud v = c->view();
     hipStream_t s = c->stream;
     const int nw = (c->N + kBlock / kWave - 1) / (kBlock / kWave), nt = (c->N + 255) / 256;

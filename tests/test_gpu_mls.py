@@ -305,3 +305,47 @@ def test_shared_stencils_off_the_voxel_origin(n, nv, order, y0, frac, eps):
     cl.cfg.vbox *= 1.0 + eps
     cl.neigh, cl.nneigh = _ball_lists(n, 2.5)
     _against_oracle(cl, _oracle_cloud(cl, cl.neigh, cl.nneigh), 0.5 * dx / 1303.0, order)
+
+
+def test_shared_stencils_follow_a_relayout():
+    """A hole that fills (more particles than the class arrays had room for),
+    then one that opens (fewer): each step is, bit for bit, that of a fresh
+    upload of the cloud it starts from."""
+    nx, nv = 16, 7
+    case, cl, *_ = setup("cavity3d", nx, nv)
+    dx = 1e-6 / (nx - 1)
+    c0 = np.array([0.51e-6, 0.49e-6, 0.5e-6])
+    pos = np.stack([cl.x, cl.y, cl.z], 1)
+    keep = (cl.boundary == 1) | (((pos - c0) ** 2).sum(1) > (4.6 * dx) ** 2)
+    k = np.arange(12) + 0.5
+    zk, ph = 1.0 - 2.0 * k / 12, k * np.pi * (3.0 - np.sqrt(5.0))
+    nrm = np.stack([np.sqrt(1 - zk * zk) * np.cos(ph), np.sqrt(1 - zk * zk) * np.sin(ph), zk], 1)
+    surf = c0 + 0.7 * dx * nrm
+    wall = np.zeros((12, 7))
+    wall[:, :3], wall[:, 6] = nrm, case.Tw
+    p = int(np.argmax(cl.boundary == 0))
+    cat = lambda a, b: np.ascontiguousarray(np.concatenate([a[keep], b]))
+    cloud = A.Cloud(cl.cfg, cat(cl.x, surf[:, 0]), cat(cl.y, surf[:, 1]), cat(cl.z, surf[:, 2]),
+                    cat(cl.boundary, np.ones(12, np.uint8)), cat(cl.wall, wall),
+                    cat(cl.mom, np.tile(cl.mom[p], (12, 1))), cat(cl.g, np.tile(cl.g[p], (12, 1))))
+    dt = 0.3 * dx / 1303.0
+    dom = (0.0, 1e-6) * 3
+    sol = A.Solver(cloud, precision=A.PREC_FP64)
+    ids = np.concatenate([np.full(int(keep.sum()), -1, np.int32), np.zeros(12, np.int32)])
+    n0 = sol.N
+    sizes = []
+    for size in (None, 0.7, 3.1, 2.5):
+        if size is not None:
+            _, counts = sol.cloud_manage([A.body(A.BODY_SPHERE, c0, size * dx)], ids, dx, 0.3 * dx, dom)
+            ids = sol.body_ids()
+            sizes.append((sol.N, tuple(counts)))
+        q, mom = sol.particles(), sol.moments()
+        now = A.Cloud(cl.cfg, q["x"], q["y"], q["z"], q["boundary"], q["wall"], mom, sol.g())
+        now.neigh, now.nneigh = sol.neighbours()
+        sol.step(dt)
+        other = A.Solver(now, precision=A.PREC_FP64)
+        other.step(dt)
+        assert np.array_equal(sol.g(), other.g())
+        assert np.array_equal(sol.moments(), other.moments())
+    print(f"[mls] relayout {n0} -> {sizes}", flush=True)
+    assert sizes[0][0] > n0 + n0 // 16 and sizes[1][0] < sizes[0][0]
