@@ -2188,12 +2188,15 @@ struct ApplyShape { int K, W, TX, TY, S; };
 constexpr ApplyShape kShapes32[] = {{12, 3, 1, 1, 0}, {9, 3, 1, 1, 0}, {12, 2, 2, 2, 0},
                                     {12, 2, 2, 2, 1}, {8, 2, 2, 3, 1}, {6, 2, 2, 4, 1},
                                     {6, 2, 2, 4, 2}};
-constexpr ApplyShape kShapes64[] = {{9, 2, 1, 1, 0}, {7, 2, 1, 1, 0}, {0, 2, 2, 2, 1},
-                                    {0, 2, 2, 2, 2}};
+constexpr ApplyShape kShapes64[] = {{9, 2, 1, 1, 0}, {8, 2, 1, 1, 0}, {7, 2, 1, 1, 0},
+                                    {6, 2, 1, 1, 0}, {0, 2, 2, 2, 1}, {0, 2, 2, 2, 2}};
 constexpr int kMaxBlockPlanes = kMaxZBlockPlanes;
 
 template <typename T>
-constexpr int nshapes() { return sizeof(T) == 4 ? 7 : 4; }
+constexpr int nshapes()
+{
+    return (int)((sizeof(T) == 4 ? sizeof kShapes32 : sizeof kShapes64) / sizeof(ApplyShape));
+}
 
 template <typename T>
 ApplyShape shape_at(int i) { return sizeof(T) == 4 ? kShapes32[i] : kShapes64[i]; }
@@ -2236,8 +2239,14 @@ void launch_shape(int i, Lat L, const T *g, T *gt, const T *cf, const double *sc
             const MarchItems m = march_items<T, 2, 2>(L, sh.S);
             k_apply_march<T, 2, 2><<<waves(m.per_chunk(L.nx, L.ny)), 256, 0, s>>>(L, g, gt, cf, m);
         }
-        else if (i == 1) k_apply<T, 7, 2><<<waves(all), 256, 0, s>>>(L, g, gt, cf, scal);
-        else k_apply<T, 9, 2><<<waves(all), 256, 0, s>>>(L, g, gt, cf, scal);
+        else
+            switch (i)
+            {
+            case 0: k_apply<T, 9, 2><<<waves(all), 256, 0, s>>>(L, g, gt, cf, scal); break;
+            case 1: k_apply<T, 8, 2><<<waves(all), 256, 0, s>>>(L, g, gt, cf, scal); break;
+            case 2: k_apply<T, 7, 2><<<waves(all), 256, 0, s>>>(L, g, gt, cf, scal); break;
+            default: k_apply<T, 6, 2><<<waves(all), 256, 0, s>>>(L, g, gt, cf, scal); break;
+            }
     }
 }
 
@@ -2263,7 +2272,7 @@ int default_shape(const Lat &L)
 {
     if (sizeof(T) == 4)
         return L.nx * L.ny * L.nchunk < 1024 || !shape_fits<T>(5, L.nx, L.ny) ? 1 : 5;
-    return shape_fits<T>(2, L.nx, L.ny) && L.nx * L.ny * L.nchunk >= 1024 ? 2 : 0;
+    return shape_fits<T>(4, L.nx, L.ny) && L.nx * L.ny * L.nchunk >= 1024 ? 4 : 0;
 }
 
 template <typename T>
