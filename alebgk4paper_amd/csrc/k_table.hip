@@ -2179,11 +2179,13 @@ bool is_fp32(const ab_ctx *ctx) { return ctx->cfg.precision == AB_PREC_MIXED; }
 
 // Launch shapes of the transport contraction the autotuner chooses from:
 // K outputs per z block (values reused across K + 4 planes), W the waves per
-// SIMD the register allocation targets. Every shape does the same products
-// in the same order per output, so the results do not depend on the choice.
+// SIMD the register allocation targets. Every shape does the same 81 products
+// per output. Single columns sum them in one order, whatever K, and a block
+// shape in one order of its own, in whole columns or slabs: between those the
+// results differ by rounding.
 // TX x TY > 1: interior blocks + edge columns. FP32, S > 0: the slab order, items
-// of S z blocks. FP64: marched through z, S items per block (these sum an output's
-// terms plane by plane).
+// of S z blocks. FP64: marched through z, S items per block (an output's terms
+// plane by plane).
 struct ApplyShape { int K, W, TX, TY, S; };
 constexpr ApplyShape kShapes32[] = {{12, 3, 1, 1, 0}, {9, 3, 1, 1, 0}, {12, 2, 2, 2, 0},
                                     {12, 2, 2, 2, 1}, {8, 2, 2, 3, 1}, {6, 2, 2, 4, 1},
@@ -2258,21 +2260,49 @@ bool shape_fits(int i, int nx, int ny)
     return sh.TX == 1 || (nx - 4 >= sh.TX && ny - 4 >= sh.TY);
 }
 
-// Default shape before tuning. FP32: the 2 x 4 column blocks with K = 6 in the
-// slab order, the fastest shape from 10^3 to 60^3 particles whether or not
-// they tile the interior (us against single columns: 264 / 580 at 40^3 / Nv 10,
-// 986 / 2423 at 31^3 / Nv 20, 66 / 125 at 21^3 / Nv 10, 21 / 31 at 10^3 / Nv 10).
-// Single columns in z blocks of 9 where the launch has fewer of them than the
-// chip has SIMDs: every wave then runs alone and the shorter one ends first
-// (18.2 / 22.2 us at 13^3 / Nv 7, 16.4 / 19.4 at 11^3 / Nv 6), and where no block
-// fits. FP64: the marched 2 x 2 blocks by the same rule (29 / 37 us at 13^3 / Nv 7,
-// 51 / 46 at 10^3 / Nv 10).
+// Default shape before tuning. The launches are bound by issue, so a SIMD takes
+// its waves one after another and a launch lasts a whole number of rounds of
+// 1,024 waves, one per SIMD; every figure here is us per transport.
+//
+// FP32: the 2 x 4 column blocks with K = 6 in the slab order, the fastest shape
+// from 10^3 to 60^3 particles whether or not they tile the interior (against
+// single columns: 264 / 580 at 40^3 / Nv 10, 986 / 2423 at 31^3 / Nv 20, 21 / 28
+// at 10^3 / Nv 10). Single columns where they are one round (18.2 / 21.5 at 13^3 /
+// Nv 7, 16.2 / 19.2 at 12^3 / Nv 6), and where no block fits: in z blocks of 12
+// where that saves a block, else of 9 (K12 / K9 18.0 / 20.4 at 14^3 / Nv 6, 17.2 /
+// 16.2 at 12^3 / Nv 6).
+//
+// FP64: the marched 2 x 2 blocks as one item each (M1) or two (M2). Where single
+// columns are one round, M2 if that is one round too (19 / 31 at 16^3 / Nv 5, 50 /
+// 65 at 9 x 9 x 60 / Nv 6), else single columns (28 against 33 at 8^3 / Nv 10 and
+// 10^3 / Nv 8, 28 against 31 at 13^3 / Nv 7). Beyond that M1 (against single
+// columns 35 / 48 at 12^3 / Nv 8, 71 / 116 at 20^3 / Nv 8, 785 / 1213 at 40^3 / Nv
+// 10), unless it is a round more than they are: with few rounds that is dear (M1 /
+// M2 / single 101 / 67 / 78 at 31^3 / Nv 5, 76 / 68 / 82 at 16^3 / Nv 9), with many
+// it is not (M1 / M2 128 / 134 at 26^3 / Nv 8, 7 rounds). (Where one z block of 9
+// is the whole run, single columns would stay ahead in two rounds: 50 / 56 at
+// 13^3 / Nv 9.)
 template <typename T>
 int default_shape(const Lat &L)
 {
-    if (sizeof(T) == 4)
-        return L.nx * L.ny * L.nchunk < 1024 || !shape_fits<T>(5, L.nx, L.ny) ? 1 : 5;
-    return shape_fits<T>(4, L.nx, L.ny) && L.nx * L.ny * L.nchunk >= 1024 ? 4 : 0;
+    auto rounds = [](long long waves) { return (int)((waves + 1023) / 1024); };
+    const int run = L.nz - 4, singles = rounds((long long)L.nx * L.ny * L.nchunk);
+    if constexpr (sizeof(T) == 4)
+    {
+        if (singles > 1 && shape_fits<T>(5, L.nx, L.ny)) return 5;
+        return (run + 11) / 12 < (run + 8) / 9 ? 0 : 1;
+    }
+    else
+    {
+        // the single columns' z block that divides the run
+        const int one = run % 9 == 0 ? 0 : (run % 7 == 0 ? 2 : 1);
+        if (!shape_fits<T>(4, L.nx, L.ny)) return one;
+        auto marched = [&](int nslab) {
+            return rounds((long long)march_items<T, 2, 2>(L, nslab).per_chunk(L.nx, L.ny) * L.nchunk);
+        };
+        if (singles == 1) return marched(2) == 1 ? 5 : one;
+        return marched(1) > singles && marched(1) <= 4 ? 5 : 4;
+    }
 }
 
 template <typename T>

@@ -19,7 +19,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("prec,tol", [(A.PREC_MIXED, 1e-6), (A.PREC_FP64_TABLE, 1e-13)])
 @pytest.mark.parametrize("n,nv", [((13, 13, 13), 5), ((11, 9, 13), 4), ((10, 8, 7), 6),
                                   ((7, 12, 9), 5), ((8, 15, 6), 4), ((23, 10, 5), 4),
-                                  ((6, 6, 12), 4), ((9, 8, 11), 9)])
+                                  ((6, 6, 12), 4), ((9, 8, 11), 9), ((14, 14, 14), 8),
+                                  ((8, 9, 40), 5)])
 def test_block_shapes_on_ragged_lattices(n, nv, prec, tol):
     print(f"[shapes] lattice {n} Nv {nv} precision {prec}", flush=True)
     case = A.configure("cavity3d", nx=n[0], nv=nv, mls_order=2)
