@@ -214,6 +214,9 @@ int fp64_step(ab_ctx *c, double dt, bool diag)
     // collision keeps its separate passes
     const bool fused = c->cfg.collision == AB_COLLISION_CONTINUOUS;
     double *rho_wall = c->dim == 3 ? c->prho : c->rho;
+    const double coeff = 1.0 / (1.0 + dt / c->cfg.tau);
+    // (the 2-D table formulation takes the one rescale for every particle)
+    const bool kept = fused && !table2d(c);
     tm.tic();
     if (!c->mass_valid) launch_mass_partials(v, c->g, c->pmass, s);
     if (!fused) launch_reduce_mass(c->N, c->pmass, c->scal, R_MASS_OLD, 0, s, c->seg, c->nbatch);
@@ -234,7 +237,7 @@ int fp64_step(ab_ctx *c, double dt, bool diag)
         tm.toc(ST_WALL_COLLIDE);
         tm.tic();
         launch_reduce_mass(c->N, c->pcol, c->scal, R_MASS_FUSED, c->cfg.no_mass_fix, s, c->seg,
-                           c->nbatch, c->pnew, c->pmass);
+                           c->nbatch, c->pnew, c->pmass, kept ? c->bnd : nullptr, coeff);
         tm.toc(ST_REDUCE);
     }
     else
@@ -257,7 +260,9 @@ int fp64_step(ab_ctx *c, double dt, bool diag)
     }
     tm.tic();
     launch_final(v, c->g, c->scal, c->cfg.R, c->rho, c->ux, c->uy, c->uz, c->T, c->pmass, s,
-                 nullptr, fused ? rho_wall : nullptr);
+                 nullptr,
+                 fused ? FusedFinal{rho_wall, kept ? c->pnew : nullptr, c->gt, c->limflag, coeff}
+                       : FusedFinal{});
     tm.toc(ST_FINAL);
     c->mass_valid = true;
     return hipGetLastError() == hipSuccess ? AB_OK : AB_ERR_HIP;

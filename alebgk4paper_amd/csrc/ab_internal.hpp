@@ -67,6 +67,10 @@ enum ScalarSlot
 // commit and collision, giving all scales at once.
 enum ReduceMode { R_MASS_OLD = 0, R_MASS_NEW = 1, R_MASS_COLL = 2, R_MASS_FUSED = 3 };
 
+// A wall that emits nothing, in the limiter flags between the fused commit and
+// collision and k_final.
+constexpr double kNoEmission = 8.0;
+
 // Stages timed by ab_profile, in report order.
 enum Stage
 {
@@ -293,10 +297,13 @@ void launch_pad_check(const DevCloud &c, const double *g, const double *rho, con
                       double *limflag, int *fail, hipStream_t s);
 void launch_mass_partials(const DevCloud &c, const double *g, double *pmass, hipStream_t s);
 // One sum per instance when seg is given (nseg instances, first particles
-// seg[0..nseg], scalars S_COUNT apart); else one over all N.
+// seg[0..nseg], scalars S_COUNT apart); else one over all N. R_MASS_FUSED also
+// takes the boundary flags and the collision's 1 / (1 + dt / tau), for the
+// particles without mass (bnd null: these are taken like the others).
 void launch_reduce_mass(int N, const double *pmass, double *scal, int mode, int nofix,
                         hipStream_t s, const int *seg = nullptr, int nseg = 1,
-                        const double *pnew = nullptr, const double *pold = nullptr);
+                        const double *pnew = nullptr, const double *pold = nullptr,
+                        const unsigned char *bnd = nullptr, double coeff = 0.0);
 void launch_limit_commit(const DevCloud &c, double *g, const double *gt, const double *rho,
                          double *limflag, double *pmass, hipStream_t s);
 // guard (may be null): when given, the launch acts only if *guard is set,
@@ -306,21 +313,30 @@ void launch_wall_collide(const DevCloud &c, const DmArgs &dm, double *g, const d
                          double tau, double R, double *rho, double *ux, double *uy,
                          double *uz, double *T, double *pmass, hipStream_t s,
                          const int *guard = nullptr);
-// rho_wall: after launch_commit_collide2/3, whose wall densities still lack
-// the first rescale, the boundary particles' rho is rho_wall times it.
+// What the fused commit and collision leaves to k_final: the boundary particles'
+// rho is rho_wall times the first rescale, and 1 where limflag says kNoEmission;
+// the rows of particles without mass (pnew) still lack a share of their
+// Maxwellian, which is what they hold beyond coeff = 1 / (1 + dt / tau) times gt.
+struct FusedFinal
+{
+    const double *rho_wall = nullptr, *pnew = nullptr, *gt = nullptr;
+    double *limflag = nullptr;
+    double coeff = 0.0;
+};
 void launch_final(const DevCloud &c, double *g, const double *scal, double R, double *rho,
                   double *ux, double *uy, double *uz, double *T, double *pmass,
-                  hipStream_t s, const int *guard = nullptr, const double *rho_wall = nullptr);
+                  hipStream_t s, const int *guard = nullptr, const FusedFinal &fused = {});
 // The 2-D step's positivity, commit, wall and collision in one pass (the
 // first rescale folded into the end-of-step one): g from gt, the committed
-// masses into pnew, the collided masses into pmass.
-void launch_commit_collide2(const DevCloud &c, double *g, const double *gt, double dt,
+// masses into pnew, the collided masses into pmass. gt is written only where a
+// particle without mass was repaired.
+void launch_commit_collide2(const DevCloud &c, double *g, double *gt, double dt,
                             double tau, double R, double *rho, double *ux, double *uy,
                             double *T, double *limflag, double *pnew, double *pmass,
                             hipStream_t s);
 // The same of the 3-D step (continuous collision); the wall densities into
 // rho_wall, rho itself only read (NAD).
-void launch_commit_collide3(const DevCloud &c, double *g, const double *gt, double dt,
+void launch_commit_collide3(const DevCloud &c, double *g, double *gt, double dt,
                             double tau, double R, const double *rho, double *rho_wall, double *ux,
                             double *uy, double *uz, double *T, double *limflag, double *pnew,
                             double *pmass, hipStream_t s);

@@ -33,6 +33,12 @@ __global__ __launch_bounds__(kBlock) void k_mass_partials(DevCloud c, const doub
     if (threadIdx.x == 0) pmass[i] = m[0];
 }
 
+// A particle without mass keeps its moments; its Maxwellian then does not scale
+// with the rows, and the end-of-step factor, which holds s1, rescales it by that
+// too much: the share it lacks until then.
+__device__ __forceinline__ double kept_share(double s1) { return s1 != 0.0 ? 1.0 / s1 - 1.0 : 0.0; }
+__device__ __forceinline__ bool no_mass(double m) { return !(m > 1e-30); }
+
 // Fixed-order sum of the per-particle partials and the rescale factor
 // (sumMassHost + the scalar logic of cudaStep :1627, :1706-1710, :1773-1780),
 // kept on the device so no host synchronisation is needed.
@@ -42,9 +48,11 @@ __global__ __launch_bounds__(1024) void k_reduce_mass(int N, const double *__res
                                                       double *scal, int mode, int nofix,
                                                       const int *__restrict__ seg,
                                                       const double *__restrict__ pnew,
-                                                      const double *__restrict__ pold)
+                                                      const double *__restrict__ pold,
+                                                      const unsigned char *__restrict__ bnd,
+                                                      double coeff)
 {
-    __shared__ double sh[1024 / kWave], shn[1024 / kWave], sho[1024 / kWave];
+    __shared__ double sh[1024 / kWave], shn[1024 / kWave], sho[1024 / kWave], shk[1024 / kWave];
     int lo = 0, hi = N;
     if (seg)
     {
@@ -54,7 +62,11 @@ __global__ __launch_bounds__(1024) void k_reduce_mass(int N, const double *__res
     }
     // eight loads in flight per thread while eight are left: the one workgroup
     // is bound by their latency (64,000 particles: 29 -> 21 us)
-    auto total = [&](const double *__restrict__ p) {
+    double sk = 0.0;               // mass of the Maxwellians that do not scale
+    auto add_kept = [&](double v, int i) {
+        if (no_mass(v) && !bnd[i]) sk += pmass[i] - coeff * v;
+    };
+    auto total = [&](const double *__restrict__ p, bool kept) {
         constexpr int U = 8;
         double t = 0.0;
         int i = lo + (int)threadIdx.x;
@@ -65,16 +77,30 @@ __global__ __launch_bounds__(1024) void k_reduce_mass(int N, const double *__res
             for (int u = 0; u < U; ++u) v[u] = p[i + u * 1024];
 #pragma unroll
             for (int u = 0; u < U; ++u) t += v[u];
+            if (!kept) continue;
+            bool any = false;
+#pragma unroll
+            for (int u = 0; u < U; ++u) any = any || no_mass(v[u]);
+            if (any)
+                for (int u = 0; u < U; ++u) add_kept(p[i + u * 1024], i + u * 1024);
         }
-        for (; i < hi; i += 1024) t += p[i];
+        for (; i < hi; i += 1024)
+        {
+            const double v = p[i];
+            t += v;
+            if (kept) add_kept(v, i);
+        }
         return t;
     };
-    double s = total(pmass), sn = pnew ? total(pnew) : 0.0, so = pold ? total(pold) : 0.0;
+    double s = total(pmass, false), sn = pnew ? total(pnew, bnd != nullptr) : 0.0,
+           so = pold ? total(pold, false) : 0.0;
     s = wave_sum(s);
     sn = wave_sum(sn);
     so = wave_sum(so);
+    if (__any(sk != 0.0)) sk = wave_sum(sk);
     if ((threadIdx.x & (kWave - 1)) == 0)
     {
+        shk[threadIdx.x / kWave] = sk;
         sh[threadIdx.x / kWave] = s;
         shn[threadIdx.x / kWave] = sn;
         sho[threadIdx.x / kWave] = so;
@@ -82,14 +108,15 @@ __global__ __launch_bounds__(1024) void k_reduce_mass(int N, const double *__res
     __syncthreads();
     if (threadIdx.x == 0)
     {
-        double t = 0.0, tn = 0.0, to = 0.0;
-        for (int q = 0; q < 1024 / kWave; ++q) { t += sh[q]; tn += shn[q]; to += sho[q]; }
+        double t = 0.0, tn = 0.0, to = 0.0, tk = 0.0;
+        for (int q = 0; q < 1024 / kWave; ++q) { t += sh[q]; tn += shn[q]; to += sho[q]; tk += shk[q]; }
         if (mode == R_MASS_FUSED)
         {
             // massOld / massNew, the collided mass after that rescale, and the
             // one end-of-step factor that the unscaled collided rows need:
             // massOld / massColl * massOld / massNew = massOld / t
             const double s1 = (tn > 1e-30) ? to / tn : 1.0;
+            if (tk != 0.0) t += tk * kept_share(s1);
             scal[S_MASS_OLD] = to;
             scal[S_MASS_NEW] = tn;
             scal[S_SCALE1] = s1;
@@ -434,14 +461,16 @@ __global__ __launch_bounds__(kBlock) void k_wall_collide(DevCloud c, DmArgs dm, 
 // of the rescaled one divided by massOld / massNew. The reduction then takes
 // the committed masses (pnew) and the collided masses (pmass) and gives
 // k_final the one factor that the rows need; the wall densities get the
-// first factor there. Results agree with the separate kernels to rounding.
+// first factor there. A particle without mass keeps its moments and a wall that
+// emits nothing has density 1, whatever the rescale: the reduction and k_final
+// make up for it (FusedFinal). Results agree with the separate kernels to rounding.
 // U > 0: rows of at most U * 64 nodes (Nv <= 16 for U = 4), which each lane
 // loads into registers once (U values of each layer); U == 0: any row, read
 // again from memory in every pass. Both sum in the same order, so they give
 // identical results.
 template <int U>
 __global__ __launch_bounds__(kBlock) void k_commit_collide2(DevCloud c, double *__restrict__ g,
-                                                            const double *__restrict__ gt,
+                                                            double *__restrict__ gt,
                                                             double dt, double tau, double R,
                                                             double *rho, double *ux, double *uy,
                                                             double *T, double *__restrict__ limflag,
@@ -452,8 +481,7 @@ __global__ __launch_bounds__(kBlock) void k_commit_collide2(DevCloud c, double *
     if (i >= c.N) return;                              // whole wave: one particle
     const int lane = threadIdx.x & (kWave - 1);
     const size_t gs = (size_t)c.gstride;
-    double *gp = g + (size_t)i * gs;
-    const double *tp = gt + (size_t)i * gs;
+    double *gp = g + (size_t)i * gs, *tp = gt + (size_t)i * gs;
     const int nodes = c.nodes, Nv = c.Nv;
     const double dvd = c.dv * c.dv;
     const int nu = U > 0 ? U : (nodes + kWave - 1) / kWave;   // passes of a wave over the row
@@ -494,7 +522,7 @@ __global__ __launch_bounds__(kBlock) void k_commit_collide2(DevCloud c, double *
         }
     };
     double m[1] = {0.0};
-    double mnew = 0.0;
+    double mnew = 0.0, flag = fires ? 1.0 : 0.0;
 
     if (c.bnd[i])
     {
@@ -525,6 +553,7 @@ __global__ __launch_bounds__(kBlock) void k_commit_collide2(DevCloud c, double *
         }
         wave_sums<3>(r);
         const double rho_w = (r[1] > 1e-30) ? (-r[0] / r[1]) : 1.0;
+        if (!(r[1] > 1e-30)) flag += kNoEmission;
         mnew = r[2];
 #pragma unroll
         for (int u = 0; u < nu; ++u)
@@ -568,7 +597,8 @@ __global__ __launch_bounds__(kBlock) void k_commit_collide2(DevCloud c, double *
         wave_sums<5>(r);
         mnew = r[0];
         double mrho = rho[i], mux = ux[i], muy = uy[i], mT = T[i];
-        if (r[0] > 1e-30)
+        const bool kept = no_mass(r[0]);
+        if (!kept)
         {
             mrho = r[0];
             mux = r[1] / r[0];
@@ -586,6 +616,7 @@ __global__ __launch_bounds__(kBlock) void k_commit_collide2(DevCloud c, double *
             const double vy = vnode(c.vlo, c.dv, (k / Nv) % Nv);
             double f, f2;
             committed(u, k, f, f2);
+            if (kept && fires) { tp[k] = f; tp[k + nodes] = f2; }      // for k_final
             const double Mg1 = maxwellian_g1(vx, vy, mux, muy, mT, mrho, R);
             f = coeff * (f + lam * Mg1);
             f2 = coeff * (f2 + lam * 0.5 * R * mT * Mg1);
@@ -600,7 +631,7 @@ __global__ __launch_bounds__(kBlock) void k_commit_collide2(DevCloud c, double *
     {
         pmass[i] = m[0];
         pnew[i] = mnew;
-        limflag[i] = fires ? 1.0 : 0.0;
+        limflag[i] = flag;
     }
 }
 
@@ -624,7 +655,7 @@ __global__ __launch_bounds__(kBlock) void k_commit_collide2(DevCloud c, double *
 // mg1, mg2: ceil(2^32 / Nv), ceil(2^32 / Nv^2), exact quotients for k < Nv^3.
 template <int U>
 __global__ __launch_bounds__(kBlock) void k_commit_collide3(
-    DevCloud c, double *__restrict__ g, const double *__restrict__ gt, unsigned mg1, unsigned mg2,
+    DevCloud c, double *__restrict__ g, double *__restrict__ gt, unsigned mg1, unsigned mg2,
     double dt, double tau, double R, const double *__restrict__ rho, double *__restrict__ rho_wall,
     double *ux, double *uy, double *uz, double *T, double *__restrict__ limflag,
     double *__restrict__ pnew, double *__restrict__ pmass)
@@ -634,8 +665,7 @@ __global__ __launch_bounds__(kBlock) void k_commit_collide3(
     const int i = xcd_remap(blockIdx.x, gridDim.x) * (kBlock / kWave) + w;
     if (i >= c.N) return;                              // whole wave: one particle
     const size_t gs = (size_t)c.gstride;
-    double *gp = g + (size_t)i * gs;
-    const double *tp = gt + (size_t)i * gs;
+    double *gp = g + (size_t)i * gs, *tp = gt + (size_t)i * gs;
     const int nodes = c.nodes, Nv = c.Nv;
     const double dv3 = c.dv * c.dv * c.dv;
     const int nu = U > 0 ? U : (nodes + kWave - 1) / kWave;
@@ -772,6 +802,7 @@ __global__ __launch_bounds__(kBlock) void k_commit_collide3(
         wave_sums<3>(q);
         const double intM = q[0] * dv3, intP = q[1] * in * dv3;
         const double rho_w = (intP > 1e-30) ? (-intM / intP) : 1.0, am = rho_w * in;
+        if (!(intP > 1e-30)) flag += kNoEmission;
         mnew = q[2] * dv3;
 #pragma unroll
         for (int u = 0; u < nu; ++u)
@@ -811,7 +842,8 @@ __global__ __launch_bounds__(kBlock) void k_commit_collide3(
         for (int a = 0; a < 5; ++a) q[a] *= dv3;
         mnew = q[0];
         double mrho = rho[i], mux = ux[i], muy = uy[i], muz = uz[i], mT = T[i];
-        if (q[0] > 1e-30)
+        const bool kept = no_mass(q[0]), repaired = kept && (fires || sc2 != 1.0);
+        if (!kept)
         {
             mrho = q[0];
             mux = q[1] / q[0];
@@ -830,7 +862,9 @@ __global__ __launch_bounds__(kBlock) void k_commit_collide3(
             if (k >= nodes) continue;
             int iv, jv, kv;
             node(k, iv, jv, kv);
-            const double f = coeff * (value(u, k) + am * (tab[w][0][iv] * tab[w][1][jv] * tab[w][2][kv]));
+            const double v = value(u, k);
+            if (repaired) tp[k] = v;                                   // for k_final
+            const double f = coeff * (v + am * (tab[w][0][iv] * tab[w][1][jv] * tab[w][2][kv]));
             gp[k] = f;
             m += f;
         }
@@ -855,8 +889,7 @@ __global__ __launch_bounds__(kBlock) void k_final(DevCloud c, double *__restrict
                                                   double *rho, double *ux, double *uy,
                                                   double *uz, double *T,
                                                   double *__restrict__ pmass,
-                                                  const int *__restrict__ guard,
-                                                  const double *rho_wall)
+                                                  const int *__restrict__ guard, FusedFinal fu)
 {
     constexpr int kPer = kBlock / kWave;
     const int i = xcd_remap(blockIdx.x, gridDim.x) * kPer + (int)(threadIdx.x / kWave);
@@ -872,13 +905,10 @@ __global__ __launch_bounds__(kBlock) void k_final(DevCloud c, double *__restrict
     const int nodes = c.nodes, Nv = c.Nv;
     const double dvd = (DIM == 3) ? c.dv * c.dv * c.dv : c.dv * c.dv;
     const bool inner = !c.bnd[i];
+    // (loaded beside the row, looked at once that is there)
+    const double mnew = fu.pnew ? fu.pnew[i] : 1.0;
     double r[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};   // rho, rux, ruy, ruz, E, mass
-    auto node = [&](int k, double f, double f2) {
-        if (doScale)
-        {
-            f *= s2; gp[k] = f;
-            if constexpr (DIM == 2) { f2 *= s2; gp[k + nodes] = f2; }
-        }
+    auto sums = [&](int k, double f, double f2) {
         r[5] += f * dvd;
         if (inner)
         {
@@ -897,17 +927,52 @@ __global__ __launch_bounds__(kBlock) void k_final(DevCloud c, double *__restrict
                 r[4] += (vx * vx + vy * vy) * f * dvd + 2.0 * f2 * dvd;
         }
     };
+    auto node = [&](int k, double f, double f2) {
+        if (doScale)
+        {
+            f *= s2; gp[k] = f;
+            if constexpr (DIM == 2) { f2 *= s2; gp[k + nodes] = f2; }
+        }
+        sums(k, f, f2);
+    };
     constexpr int U = 4;
-    int k0 = 0;
-    for (; k0 + U * kWave <= nodes; k0 += U * kWave)
-    {
-        double f[U], f2[U];
+    auto load = [&](int k0, double (&f)[U], double (&f2)[U]) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
         {
             f[u] = gp[k0 + u * kWave + lane];
             f2[u] = (DIM == 2) ? gp[k0 + u * kWave + lane + nodes] : 0.0;
         }
+    };
+    int k0 = 0;
+    double f[U], f2[U];
+    if (U * kWave <= nodes) load(0, f, f2);
+    if (__any(inner && no_mass(mnew)))                 // whole wave: one particle
+    {
+        // a particle without mass: the share that its Maxwellian lacks
+        const double *tp = fu.gt + (size_t)i * gs;
+        const double b = kept_share(s1);
+#pragma unroll 1
+        for (int k = lane; k < nodes; k += kWave)
+        {
+            double v = gp[k], v2 = 0.0;
+            v += b * (v - fu.coeff * tp[k]);
+            if constexpr (DIM == 2)
+            {
+                v2 = gp[k + nodes];
+                v2 += b * (v2 - fu.coeff * tp[k + nodes]);
+            }
+            v *= s2;
+            v2 *= s2;
+            gp[k] = v;
+            if constexpr (DIM == 2) gp[k + nodes] = v2;
+            sums(k, v, v2);
+        }
+        k0 = nodes;
+    }
+    for (; k0 + U * kWave <= nodes; k0 += U * kWave)
+    {
+        if (k0) load(k0, f, f2);
 #pragma unroll
         for (int u = 0; u < U; ++u) node(k0 + u * kWave + lane, f[u], f2[u]);
     }
@@ -918,7 +983,13 @@ __global__ __launch_bounds__(kBlock) void k_final(DevCloud c, double *__restrict
     if (lane == 0)
     {
         pmass[i] = r[5];
-        if (!inner && rho_wall) rho[i] = rho_wall[i] * s1;
+        if (!inner && fu.rho_wall)
+        {
+            const double lim = fu.limflag[i];
+            const bool none = lim >= kNoEmission;
+            rho[i] = none ? 1.0 : fu.rho_wall[i] * s1;
+            if (none) fu.limflag[i] = lim - kNoEmission;
+        }
         if (inner && r[0] > 1e-30)
         {
             double mux = r[1] / r[0], muy = r[2] / r[0], muz = 0.0, u2;
@@ -1078,9 +1149,10 @@ void launch_mass_partials(const DevCloud &c, const double *g, double *pmass, hip
 
 void launch_reduce_mass(int N, const double *pmass, double *scal, int mode, int nofix,
                         hipStream_t s, const int *seg, int nseg, const double *pnew,
-                        const double *pold)
+                        const double *pold, const unsigned char *bnd, double coeff)
 {
-    k_reduce_mass<<<seg ? nseg : 1, 1024, 0, s>>>(N, pmass, scal, mode, nofix, seg, pnew, pold);
+    k_reduce_mass<<<seg ? nseg : 1, 1024, 0, s>>>(N, pmass, scal, mode, nofix, seg, pnew, pold, bnd,
+                                                  coeff);
 }
 
 void launch_limit_commit(const DevCloud &c, double *g, const double *gt, const double *rho,
@@ -1105,18 +1177,18 @@ void launch_wall_collide(const DevCloud &c, const DmArgs &dm, double *g, const d
 
 void launch_final(const DevCloud &c, double *g, const double *scal, double R, double *rho,
                   double *ux, double *uy, double *uz, double *T, double *pmass, hipStream_t s,
-                  const int *guard, const double *rho_wall)
+                  const int *guard, const FusedFinal &fused)
 {
     const int nb = (c.N + kBlock / kWave - 1) / (kBlock / kWave);
     if (c.dim == 3)
         k_final<3><<<nb, kBlock, 0, s>>>(c, g, scal, R, rho, ux, uy, uz, T, pmass, guard,
-                                         rho_wall);
+                                         fused);
     else
         k_final<2><<<nb, kBlock, 0, s>>>(c, g, scal, R, rho, ux, uy, uz, T, pmass, guard,
-                                         rho_wall);
+                                         fused);
 }
 
-void launch_commit_collide2(const DevCloud &c, double *g, const double *gt, double dt,
+void launch_commit_collide2(const DevCloud &c, double *g, double *gt, double dt,
                             double tau, double R, double *rho, double *ux, double *uy,
                             double *T, double *limflag, double *pnew, double *pmass,
                             hipStream_t s)
@@ -1138,7 +1210,7 @@ void launch_commit_collide2(const DevCloud &c, double *g, const double *gt, doub
                                                    pnew, pmass);
 }
 
-void launch_commit_collide3(const DevCloud &c, double *g, const double *gt, double dt,
+void launch_commit_collide3(const DevCloud &c, double *g, double *gt, double dt,
                             double tau, double R, const double *rho, double *rho_wall, double *ux,
                             double *uy, double *uz, double *T, double *limflag, double *pnew,
                             double *pmass, hipStream_t s)

@@ -51,7 +51,8 @@ extern "C" {
                                  tables, and positivity, commit, wall and
                                  collision in one pass with the two mass
                                  rescales applied as one (equal to the
-                                 FP64 step to rounding; lattice clouds;
+                                 FP64 step to rounding where every
+                                 particle has mass; lattice clouds;
                                  MIXED is 3-D only) */
 
 typedef struct ab_ctx ab_ctx;
