@@ -618,20 +618,23 @@ struct Wave                                            // what the loads of an i
 };
 
 // Rows in flight: the loads of row U + D - 1 are issued before the products of
-// row U. Short pieces have registers for deeper rings, and are what a small
-// cloud's launch waits for.
-template <int YN, int R>
-constexpr int depth() { return R >= 8 && YN > 1 ? 2 : (R >= 4 ? 3 : 4); }
+// row U. A patch of full pieces has registers for two rows; the others take three
+// (a step of 20^3 / Nv 8, 13^3 / Nv 7, 40^3 / Nv 10: 263, 197, 1690 us with two rows
+// everywhere, 260, 194, 1671 with three; four are no faster), but not with the
+// neighbours' ranges, which the third row costs registers (40^3 / Nv 10 with
+// statistics: 3.90 ms with two, 4.33 with three).
+template <int YN, int R, bool DIAG>
+constexpr int depth() { return DIAG || (R >= 8 && YN > 1) ? 2 : 3; }
 
 // Where the coefficients of the stencil row at oy are kept until the last run of
 // the patch has met it: by oy (the same row of the next plane comes after
 // that), or in the ring of a single run.
-template <int YN, int R>
-constexpr int coef_at(int U, int oy) { return YN > 1 ? oy + 2 : U % depth<YN, R>(); }
+template <int YN, int R, bool DIAG>
+constexpr int coef_at(int U, int oy) { return YN > 1 ? oy + 2 : U % depth<YN, R, DIAG>(); }
 
 // Values of patch row U into v, and into cm the coefficients of the stencil row
 // that the first run meets there (the later runs meet it at later rows).
-template <int YN, int R, int U>
+template <int YN, int R, bool DIAG, int U>
 __device__ __forceinline__ void patch_load(const Wave &w, const int (&first)[YN], double (&v)[R + 4],
                                            double (&cm)[5][5])
 {
@@ -650,20 +653,20 @@ __device__ __forceinline__ void patch_load(const Wave &w, const int (&first)[YN]
         constexpr Row k = kRowTab.r[row_of(q.y, q.oz)];
 #pragma clang loop unroll(full)
         for (int j = 0; j <= 2 * k.d; ++j)
-            cm[coef_at<YN, R>(U, q.y)][j] = (w.cf + (size_t)(k.o0 + j) * kWave)[w.lane];
+            cm[coef_at<YN, R, DIAG>(U, q.y)][j] = (w.cf + (size_t)(k.o0 + j) * kWave)[w.lane];
     }
 }
 
 template <int YN, int R, bool DIAG, int U>
 __device__ __forceinline__ void patch_step(const Wave &w, const int (&first)[YN],
-                                           double (&v)[depth<YN, R>()][R + 4],
+                                           double (&v)[depth<YN, R, DIAG>()][R + 4],
                                            double (&cm)[5][5], double (&acc)[YN][R], double (&gmin)[DIAG ? R : 1],
                                            double (&gmax)[DIAG ? R : 1])
 {
     constexpr auto q = Patch<YN>::tab.r[U];
-    constexpr int D = depth<YN, R>(), B = U % D;
+    constexpr int D = depth<YN, R, DIAG>(), B = U % D;
     if constexpr (U + D - 1 < Patch<YN>::tab.n)
-        patch_load<YN, R, U + D - 1>(w, first, v[(U + D - 1) % D], cm);
+        patch_load<YN, R, DIAG, U + D - 1>(w, first, v[(U + D - 1) % D], cm);
 #pragma clang loop unroll(full)
     for (int k = 0; k < YN; ++k)
     {
@@ -674,7 +677,7 @@ __device__ __forceinline__ void patch_step(const Wave &w, const int (&first)[YN]
         for (int j = 0; j <= 4; ++j)
         {
             if (j > 2 * d) continue;
-            const double cj = cm[coef_at<YN, R>(U, q.y - k)][j];
+            const double cj = cm[coef_at<YN, R, DIAG>(U, q.y - k)][j];
 #pragma clang loop unroll(full)
             for (int r = 0; r < R; ++r) acc[k][r] += cj * v[B][r + j + q.d - d];
             if constexpr (DIAG)
@@ -706,11 +709,10 @@ __device__ __forceinline__ void patch_rows(const Wave &w, const int (&first)[YN]
                                            double (&gmax)[DIAG ? R : 1],
                                            std::integer_sequence<int, U...>)
 {
-    constexpr int D = depth<YN, R>();
+    constexpr int D = depth<YN, R, DIAG>();
     double v[D][R + 4], cm[5][5];
-    patch_load<YN, R, 0>(w, first, v[0], cm);
-    if constexpr (D > 2) patch_load<YN, R, 1>(w, first, v[1], cm);
-    if constexpr (D > 3) patch_load<YN, R, 2>(w, first, v[2], cm);
+    patch_load<YN, R, DIAG, 0>(w, first, v[0], cm);
+    if constexpr (D > 2) patch_load<YN, R, DIAG, 1>(w, first, v[1], cm);
     (patch_step<YN, R, DIAG, U>(w, first, v, cm, acc, gmin, gmax), ...);
 }
 
