@@ -82,6 +82,7 @@ __global__ __launch_bounds__(1024) void k_reduce_mass(int N, const double *__res
 #pragma unroll
             for (int u = 0; u < U; ++u) any = any || no_mass(v[u]);
             if (any)
+#pragma unroll 1
                 for (int u = 0; u < U; ++u) add_kept(p[i + u * 1024], i + u * 1024);
         }
         for (; i < hi; i += 1024)
@@ -936,48 +937,43 @@ __global__ __launch_bounds__(kBlock) void k_final(DevCloud c, double *__restrict
         sums(k, f, f2);
     };
     constexpr int U = 4;
-    auto load = [&](int k0, double (&f)[U], double (&f2)[U]) {
+    int k0 = 0;
+    for (; k0 + U * kWave <= nodes; k0 += U * kWave)
+    {
+        double f[U], f2[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
         {
             f[u] = gp[k0 + u * kWave + lane];
             f2[u] = (DIM == 2) ? gp[k0 + u * kWave + lane + nodes] : 0.0;
         }
-    };
-    int k0 = 0;
-    double f[U], f2[U];
-    if (U * kWave <= nodes) load(0, f, f2);
-    if (__any(inner && no_mass(mnew)))                 // whole wave: one particle
-    {
-        // a particle without mass: the share that its Maxwellian lacks
-        const double *tp = fu.gt + (size_t)i * gs;
-        const double b = kept_share(s1);
-#pragma unroll 1
-        for (int k = lane; k < nodes; k += kWave)
-        {
-            double v = gp[k], v2 = 0.0;
-            v += b * (v - fu.coeff * tp[k]);
-            if constexpr (DIM == 2)
-            {
-                v2 = gp[k + nodes];
-                v2 += b * (v2 - fu.coeff * tp[k + nodes]);
-            }
-            v *= s2;
-            v2 *= s2;
-            gp[k] = v;
-            if constexpr (DIM == 2) gp[k + nodes] = v2;
-            sums(k, v, v2);
-        }
-        k0 = nodes;
-    }
-    for (; k0 + U * kWave <= nodes; k0 += U * kWave)
-    {
-        if (k0) load(k0, f, f2);
 #pragma unroll
         for (int u = 0; u < U; ++u) node(k0 + u * kWave + lane, f[u], f2[u]);
     }
     for (int k = k0 + lane; k < nodes; k += kWave)
         node(k, gp[k], (DIM == 2) ? gp[k + nodes] : 0.0);
+    if (__any(inner && no_mass(mnew)))                 // whole wave: one particle
+    {
+        // a particle without mass: the share that its Maxwellian lacks, and the
+        // sums again (after the loop: in it the test would wait before the row's
+        // loads, or its registers cost a wave)
+        const double *tp = fu.gt + (size_t)i * gs;
+        const double b = kept_share(s1), sc = s2 * fu.coeff;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) r[q] = 0.0;
+#pragma unroll 1
+        for (int k = lane; k < nodes; k += kWave)
+        {
+            double f = gp[k], f2 = 0.0;
+            gp[k] = f += b * (f - sc * tp[k]);
+            if constexpr (DIM == 2)
+            {
+                f2 = gp[k + nodes];
+                gp[k + nodes] = f2 += b * (f2 - sc * tp[k + nodes]);
+            }
+            sums(k, f, f2);
+        }
+    }
 #pragma unroll
     for (int q = 0; q < 6; ++q) r[q] = wave_sum(r[q]);
     if (lane == 0)
