@@ -1,7 +1,8 @@
 """The 3-D FP64 step's fused positivity, NAD, commit, wall and collision at the
 row lengths where its variants change (rows of 4, 8 and 16 values a lane in
-registers, longer rows read again), with both limiters firing, and the mass
-sums around the lengths of their unrolled loop.
+registers, longer rows read again), with both limiters firing, the mass sums
+around the lengths of their unrolled loop, and particles and walls whose
+collision does not scale with g.
 
 Tolerances: 1e-10 relative on g and the moments (the FP64 step's); limiter
 flags identical.
@@ -13,7 +14,7 @@ import pytest
 
 import alebgk4paper_amd as A
 import oracle_ctypes as O
-from helpers import rel_err, setup
+from helpers import local_maxwellian, rel_err, setup
 
 pytestmark = pytest.mark.gpu
 
@@ -42,15 +43,31 @@ def test_step_with_limiters_matches_oracle(nv, order):
     assert fired == 3
 
 
-@pytest.mark.parametrize("nx", [6, 20, 21, 24])
-def test_mass_over_many_particles(nx):
-    """N below, at and above multiples of the sum's 8 x 1024 particles."""
-    case, cl, *_ = setup("cavity3d", nx, 3, order=1)
+@pytest.mark.parametrize("n,extra", [((6, 6, 6), 0), ((16, 16, 32), -1), ((16, 16, 32), 0),
+                                     ((16, 16, 32), 1), ((16, 32, 32), -1), ((16, 32, 32), 0),
+                                     ((16, 32, 32), 1), ((24, 24, 24), 0)])
+def test_mass_over_many_particles(n, extra):
+    """N below, at and above multiples of the sum's 8 x 1024 particles (extra: an
+    interior particle less, or one more)."""
+    case = A.configure("cavity3d", nx=n[0], nv=3, mls_order=1)
+    dx = 1e-6 / (n[0] - 1)
+    case.raw.ny, case.raw.nz = n[1], n[2]
+    case.raw.dom[2], case.raw.dom[4] = dx * (n[1] - 1), dx * (n[2] - 1)
+    cl = A.build_lattice(case, precision=A.PREC_FP64, mls_order=1)
+    cl.g, cl.mom = local_maxwellian(cl, case)
+    p = np.nonzero(cl.boundary == 0)[0][7]
+    q = np.arange(cl.N)
+    q = np.delete(q, p) if extra < 0 else np.concatenate([q, np.full(extra, p)])
+    for k in ("x", "y", "z", "boundary", "wall", "mom", "g"):
+        setattr(cl, k, np.ascontiguousarray(getattr(cl, k)[q]))
+    if extra > 0:
+        cl.x[-1] += 0.4 * dx
+    assert cl.N == n[0] * n[1] * n[2] + extra
     sol = A.Solver(cl, precision=A.PREC_FP64)
     dv = (cl.cfg.vmax - cl.cfg.vmin) / 2
     want = cl.g.sum() * dv ** 3
     assert abs(sol.total_mass() - want) <= 1e-13 * want
-    st = sol.step(0.5 * (1e-6 / (nx - 1)) / 1303.0, stats=True)
+    st = sol.step(0.5 * dx / 1303.0, stats=True)
     assert abs(st["mass_old"] - want) <= 1e-13 * want
     assert abs(sol.total_mass() - want) <= 1e-13 * want
 
