@@ -995,6 +995,9 @@ __global__ __launch_bounds__(kBlock) void k_final(DevCloud c, double *__restrict
             rho[i] = r[0]; ux[i] = mux; uy[i] = muy; T[i] = t1 > 1e-6 ? t1 : 1e-6;
             if (DIM == 3) uz[i] = muz;
         }
+        // no mass at the step's end (or none that is a number), and some before
+        // the collision: the density is the collision's
+        else if (inner && fu.pnew && !no_mass(mnew)) rho[i] = mnew * s1;
     }
 }
 
