@@ -60,12 +60,12 @@ __global__ __launch_bounds__(1024) void k_reduce_mass(int N, const double *__res
         hi = seg[blockIdx.x + 1];
         scal += (size_t)blockIdx.x * S_COUNT;
     }
+    double sk = 0.0;               // mass of the Maxwellians that do not scale
+    auto add_kept = [&](double v, double m, bool wall) {
+        if (no_mass(v) && !wall) sk += m - coeff * v;
+    };
     // eight loads in flight per thread while eight are left: the one workgroup
     // is bound by their latency (64,000 particles: 29 -> 21 us)
-    double sk = 0.0;               // mass of the Maxwellians that do not scale
-    auto add_kept = [&](double v, int i) {
-        if (no_mass(v) && !bnd[i]) sk += pmass[i] - coeff * v;
-    };
     auto total = [&](const double *__restrict__ p, bool kept) {
         constexpr int U = 8;
         double t = 0.0;
@@ -83,13 +83,15 @@ __global__ __launch_bounds__(1024) void k_reduce_mass(int N, const double *__res
             for (int u = 0; u < U; ++u) any = any || no_mass(v[u]);
             if (any)
 #pragma unroll 1
-                for (int u = 0; u < U; ++u) add_kept(p[i + u * 1024], i + u * 1024);
+                for (int k = i; k <= i + (U - 1) * 1024; k += 1024) add_kept(p[k], pmass[k], bnd[k]);
         }
         for (; i < hi; i += 1024)
         {
-            const double v = p[i];
+            // (all three loaded at once: a small cloud's sum is one round trip)
+            const double v = p[i], m = kept ? pmass[i] : 0.0;
+            const bool wall = kept && bnd[i];
             t += v;
-            if (kept) add_kept(v, i);
+            if (kept) add_kept(v, m, wall);
         }
         return t;
     };
