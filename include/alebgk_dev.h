@@ -360,11 +360,12 @@ int ab_body_step_many(int n, ab_ctx *const *ctxs, const ab_body_task *tasks);
  * following steps. Shapes: one lattice column per wave with z blocks of K
  * outputs ("K9/W3": bit-identical results for every K), or TX x TY blocks of
  * interior columns per wave ("B2x4/K6/S": the same sum in another order,
- * equal to FP32 rounding; "/S": items of one z block, "/S2" of two, edge
- * columns first).
+ * equal to rounding; "/S": items of one z block, "/S2" of two, edge columns
+ * first; FP64: "B2x2/M1" and "/M2", marched through z, one or two items a
+ * block). FP64 indices 0 to 3 are single columns with K = 9, 8, 7, 6.
  * names/ms (cap entries each, may be NULL) receive every
  * candidate's name and best time in ms, "n/a" and -1 for a shape that does
- * not tile the lattice; *n the number of candidates, *chosen the index kept.
+ * not fit the lattice; *n the number of candidates, *chosen the index kept.
  * ab_set_transport_shape forces an index (-1: the default for the lattice).
  * On a 2-D table context the candidates are the apply's run lengths ("R4",
  * "R8", "R12": outputs per work item along a lattice line, bit-identical
