@@ -37,6 +37,12 @@ __global__ __launch_bounds__(kBlock) void k_mass_partials(DevCloud c, const doub
 // with the rows, and the end-of-step factor, which holds s1, rescales it by that
 // too much: the share it lacks until then.
 __device__ __forceinline__ double kept_share(double s1) { return s1 != 0.0 ? 1.0 / s1 - 1.0 : 0.0; }
+// The Maxwellian's part of a collided value (or mass) f whose relaxed part is r;
+// where f is not finite it stays as it is.
+__device__ __forceinline__ double kept_part(double f, double r)
+{
+    return isfinite(f - r) ? f - r : 0.0;
+}
 __device__ __forceinline__ bool no_mass(double m) { return !(m > 1e-30); }
 
 // Fixed-order sum of the per-particle partials and the rescale factor
@@ -62,7 +68,7 @@ __global__ __launch_bounds__(1024) void k_reduce_mass(int N, const double *__res
     }
     double sk = 0.0;               // mass of the Maxwellians that do not scale
     auto add_kept = [&](double v, double m, bool wall) {
-        if (no_mass(v) && !wall) sk += m - coeff * v;
+        if (no_mass(v) && !wall) sk += kept_part(m, coeff * v);
     };
     // eight loads in flight per thread while eight are left: the one workgroup
     // is bound by their latency (64,000 particles: 29 -> 21 us)
@@ -967,11 +973,11 @@ __global__ __launch_bounds__(kBlock) void k_final(DevCloud c, double *__restrict
         for (int k = lane; k < nodes; k += kWave)
         {
             double f = gp[k], f2 = 0.0;
-            gp[k] = f += b * (f - sc * tp[k]);
+            gp[k] = f += b * kept_part(f, sc * tp[k]);
             if constexpr (DIM == 2)
             {
                 f2 = gp[k + nodes];
-                gp[k + nodes] = f2 += b * (f2 - sc * tp[k + nodes]);
+                gp[k + nodes] = f2 += b * kept_part(f2, sc * tp[k + nodes]);
             }
             sums(k, f, f2);
         }
